@@ -68,9 +68,10 @@ __device__ __forceinline__ bool pair_readable(int n, uint8_t ty, bool ghost_zero
 // neither (every tile of the launch reads its neighbours' old values while
 // the others write theirs).
 template <class V, bool DOT>
-__global__ __launch_bounds__(64) void k_gs_pair(Ctx c, const TileRec* __restrict__ list, int n, const V* __restrict__ XI,
-                                                const V* __restrict__ XG, V* __restrict__ XO, int c1, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_pair(const TileRec* __restrict__ list, int n, int flags,
+                                                const V* __restrict__ XI, const V* __restrict__ XG,
+                                                V* __restrict__ XO, int c1, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   __shared__ PairLDS L;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const int c2 = c1 ^ 1;

@@ -290,11 +290,12 @@ __device__ __forceinline__ double wave_sum(double v) {
 // Block -> worklist position.  Consecutive workgroups go round-robin to the 8
 // XCDs; giving each XCD a contiguous (Morton-ordered) run of tiles keeps the
 // face halos of a tile in the L2 of the XCD that reads them.
-__device__ __forceinline__ int work_index(int xcd_swizzle) {
-  int b = blockIdx.x;
-  if (!xcd_swizzle) return b;
-  int per = (int(gridDim.x) + 7) >> 3;
-  return (b & 7) * per + (b >> 3);
+// n: the launch's work items (its grid, rounded up to a multiple of 8 with the
+// swizzle).
+__device__ __forceinline__ int work_index(int xcd_swizzle, int n) {
+  const int b = blockIdx.x;
+  const int per = (n + 7) >> 3;
+  return xcd_swizzle ? (b & 7) * per + (b >> 3) : b;
 }
 
 // Each tile is worked by exactly one wavefront with its own LDS region, so
@@ -1335,9 +1336,60 @@ __device__ __forceinline__ void tile_gs_prolong(const Ctx& c, const TileRec& T, 
 // ---------------------------------------------------------------------------
 // One-tile-per-workgroup kernels over a worklist
 // ---------------------------------------------------------------------------
-#define TILE_KERNEL_PROLOGUE                     \
-  int w = work_index(flags & F_SWIZZLE);         \
-  if (w >= n) return;                            \
+// The first 128 bytes of a tile's record (everything but the ghost children's
+// slots), fetched by two scalar loads that nothing else waits behind: the held
+// words keep the compiler from splitting the fetch into pieces that it would
+// load, wait for and test one after another.  A wavefront's cost on a small
+// level is its chain of memory round trips: with the launch's n and flags
+// preloaded (the kernels' first arguments) the record's fetch is the first, the
+// tile's loads the second.  k_gs_color on 64 tiles 2.90 -> 2.57 us a launch, on
+// the 360,472-tile level of the 256-problem pool in bfloat16 187 -> 178 us; the
+// adaptive 256^3 solve 5.18 -> 4.87 ms, the pool 242 -> 231 ms.
+typedef int32_t RecWords __attribute__((ext_vector_type(16), aligned(16)));
+__device__ __forceinline__ TileRec unpack_rec(RecWords a, RecWords b) {
+  TileRec T;
+  for (int f = 0; f < 6; f++) T.nbr[f] = a[f];
+  T.parent = a[6];
+  T.prob = a[7];
+  T.leaf_slot = a[8];
+  T.gslot = a[9];
+  T.self = a[10];
+  T.h = __int_as_float(a[11]);
+  T.meta = uint32_t(a[12]);
+  T.ntypes = uint32_t(a[13]);
+  T.bc[0] = __int_as_float(a[14]);
+  T.bc[1] = __int_as_float(a[15]);
+  for (int f = 2; f < 7; f++) T.bc[f] = __int_as_float(b[f - 2]);
+  for (int f = 0; f < 6; f++) T.nbr_parent[f] = b[5 + f];
+  return T;
+}
+__device__ __forceinline__ TileRec load_rec(const TileRec* __restrict__ list, int w) {
+  const RecWords* r = reinterpret_cast<const RecWords*>(list + w);
+  RecWords a = r[0], b = r[1];
+  __asm__ volatile("" : "+s"(a), "+s"(b));
+  return unpack_rec(a, b);
+}
+// The same with one pointer of each 64 bytes of the kernel's Ctx argument
+// fetched alongside, so that the pointers the loads need are in the scalar
+// cache when the record arrives.
+__device__ __forceinline__ TileRec load_rec(const TileRec* __restrict__ list, int w, const Ctx& c) {
+  const RecWords* r = reinterpret_cast<const RecWords*>(list + w);
+  RecWords a = r[0], b = r[1];
+  __asm__ volatile("" : "+s"(a), "+s"(b) : "s"(c.fmask), "s"(c.zh), "s"(c.ps));
+  return unpack_rec(a, b);
+}
+#define TILE_KERNEL_PROLOGUE                                                           \
+  const int w = work_index(flags & F_SWIZZLE, n);                                      \
+  if (w >= n) return;                                                                  \
+  const TileRec T = load_rec(list, w);
+#define TILE_KERNEL_PROLOGUE_C                                                         \
+  const int w = work_index(flags & F_SWIZZLE, n);                                      \
+  if (w >= n) return;                                                                  \
+  const TileRec T = load_rec(list, w, c);
+// The whole record, the ghost children's slots among it.
+#define TILE_KERNEL_PROLOGUE_ALL                                                       \
+  const int w = work_index(flags & F_SWIZZLE, n);                                      \
+  if (w >= n) return;                                                                  \
   const TileRec T = list[w];
 // In a CG iteration's launch, a tile that k_cg_init found inert exits: the
 // launch would write the values its arrays already hold.
@@ -1345,9 +1397,9 @@ __device__ __forceinline__ void tile_gs_prolong(const Ctx& c, const TileRec& T, 
   if ((flags & F_INERT) && tr_inert_cand(T) && c.inert[T.self]) return;
 
 template <class V, bool DOT = false>
-__global__ __launch_bounds__(64) void k_gs_color(Ctx c, const TileRec* __restrict__ list, int n, int level, V* X,
-                                                 const V* F, int color, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_color(const TileRec* __restrict__ list, int n, int flags, int level, V* X,
+                                                 const V* F, int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ GsLDS L;
   tile_gs<V, DOT>(c, T, level, X, F, color, flags, L);
@@ -1356,9 +1408,9 @@ __global__ __launch_bounds__(64) void k_gs_color(Ctx c, const TileRec* __restric
 // the other colour as read) to Y and leaves X as it was, so that the next
 // launch may read Y while it writes X.
 template <class V>
-__global__ __launch_bounds__(64) void k_gs_color_to(Ctx c, const TileRec* __restrict__ list, int n, const V* X, V* Y,
-                                                    int color, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_color_to(const TileRec* __restrict__ list, int n, int flags, const V* X,
+                                                    V* Y, int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   __shared__ GsLDS L;
   const GsIn g = gs_load<V, false>(c, T, X, static_cast<const V*>(nullptr), color, flags);
   gs_stage(g, L);
@@ -1377,10 +1429,10 @@ __global__ __launch_bounds__(64) void k_gs_color_to(Ctx c, const TileRec* __rest
 // (tiles 4b .. 4b+3 of the list in workgroup b): a quarter of the workgroups
 // to dispatch for the same tiles.
 template <class V, bool DOT = false>
-__global__ __launch_bounds__(256) void k_gs_color4(Ctx c, const TileRec* __restrict__ list, int n, int level, V* X,
-                                                   const V* F, int color, int flags) {
+__global__ __launch_bounds__(256) void k_gs_color4(const TileRec* __restrict__ list, int n, int flags, int level,
+                                                   V* X, const V* F, int color, Ctx c) {
   const int wave = threadIdx.x >> 6;
-  const int w = work_index(flags & F_SWIZZLE) * 4 + wave;
+  const int w = work_index(flags & F_SWIZZLE, (n + 3) / 4) * 4 + wave;
   __shared__ GsLDS L[4];
   if (w >= n) return;  // whole wavefronts leave; the others synchronise within their wavefront only
   const TileRec T = list[w];
@@ -1390,9 +1442,9 @@ __global__ __launch_bounds__(256) void k_gs_color4(Ctx c, const TileRec* __restr
 // and 2w+1 of the list, loads of both in flight together.  Every tile's
 // update is the one above (tiles of a colour pass are independent).
 template <class V, bool DOT = false>
-__global__ __launch_bounds__(64) void k_gs_color2(Ctx c, const TileRec* __restrict__ list, int n, int level, V* X,
-                                                  const V* F, int color, int flags) {
-  const int w = work_index(flags & F_SWIZZLE);
+__global__ __launch_bounds__(64) void k_gs_color2(const TileRec* __restrict__ list, int n, int flags, int level, V* X,
+                                                  const V* F, int color, Ctx c) {
+  const int w = work_index(flags & F_SWIZZLE, (n + 1) / 2);
   const int t0 = 2 * w;
   if (t0 >= n) return;
   const bool two = t0 + 1 < n;
@@ -1419,8 +1471,8 @@ __global__ __launch_bounds__(64) void k_gs_color2(Ctx c, const TileRec* __restri
 // grid is sized to the wavefronts the device holds at once.  Every tile's
 // update is the one above.
 template <class V, bool DOT = false>
-__global__ __launch_bounds__(64) void k_gs_color_loop(Ctx c, const TileRec* __restrict__ list, int n, int level, V* X,
-                                                      const V* F, int color, int flags) {
+__global__ __launch_bounds__(64) void k_gs_color_loop(const TileRec* __restrict__ list, int n, int flags, int level,
+                                                      V* X, const V* F, int color, Ctx c) {
   __shared__ GsLDS L;
   const int b = blockIdx.x, nb = gridDim.x;
   int t, end, stride;
@@ -1501,8 +1553,8 @@ __device__ __forceinline__ float first_red(float b, float d) {
 // halo are formed from the neighbours' rhs and stored diagonals and the second
 // pass needs no grid-wide wait.  Every value is the one the two passes give.
 template <class V>
-__global__ __launch_bounds__(64) void k_gs_first(Ctx c, const TileRec* __restrict__ list, int n, V* X, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ list, int n, int flags, V* X, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ GsLDS L;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
@@ -1727,42 +1779,42 @@ __device__ __forceinline__ void tile_gs_prolong_eager(const Ctx& c, const TileRe
   store_pencil_split(XO + size_t(T.self) * 512, lane, out0, out1);
 }
 template <class V>
-__global__ __launch_bounds__(64) void k_gs_prolong_eager(Ctx c, const TileRec* __restrict__ list, int n, const V* XD,
-                                                         V* XO, float pcoef, int color, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_prolong_eager(const TileRec* __restrict__ list, int n, int flags,
+                                                         const V* XD, V* XO, float pcoef, int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   tile_gs_prolong_eager(c, T, XD, XO, pcoef, color, flags, L);
 }
 template <class V>
-__global__ __launch_bounds__(64) void k_gs_prolong(Ctx c, const TileRec* __restrict__ list, int n, const V* XD,
-                                                   V* XO, float pcoef, int color, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_gs_prolong(const TileRec* __restrict__ list, int n, int flags, const V* XD,
+                                                   V* XO, float pcoef, int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   tile_gs_prolong(c, T, XD, XO, pcoef, color, flags, L);
 }
 template <class V>
-__global__ __launch_bounds__(64) void k_jacobi(Ctx c, const TileRec* __restrict__ list, int n, int level, const V* X,
-                                               const V* XG, V* Y, const V* F, float omega, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_jacobi(const TileRec* __restrict__ list, int n, int flags, int level,
+                                               const V* X, const V* XG, V* Y, const V* F, float omega, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   tile_jacobi(c, T, level, X, XG, Y, F, omega, flags, L);
 }
 template <class V, bool EAGER = false>
-__global__ __launch_bounds__(64) void k_restrict(Ctx c, const TileRec* __restrict__ list, int n, int level, const V* X,
-                                                 const V* F, V* CO, float one_over_alpha, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_restrict(const TileRec* __restrict__ list, int n, int flags, int level,
+                                                 const V* X, const V* F, V* CO, float one_over_alpha, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   __shared__ float res[512];
   tile_restrict<V, EAGER>(c, T, level, X, F, CO, one_over_alpha, flags, L, res);
 }
 template <class V>
-__global__ __launch_bounds__(64) void k_prolong(Ctx c, const TileRec* __restrict__ list, int n, int level,
-                                                const V* XC, const V* XF, V* XO, V* XG, float pcoef, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_prolong(const TileRec* __restrict__ list, int n, int flags, int level,
+                                                const V* XC, const V* XF, V* XO, V* XG, float pcoef, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   tile_prolong(c, T, level, XC, XF, XO, XG, pcoef, flags);
 }
@@ -2040,8 +2092,8 @@ __device__ __forceinline__ void mark_inert(const Ctx& c, const TileRec& T, int l
 // Init: x = 0, p = 0 on LEAF tiles, V-cycle rhs = b; partials of |b|^2
 // (GMGSolver.cu:537-555).
 template <class V>
-__global__ __launch_bounds__(64) void k_cg_init(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_init(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -2061,9 +2113,9 @@ __global__ __launch_bounds__(64) void k_cg_init(Ctx c, const TileRec* __restrict
 // operator kernels), p = 0, V-cycle rhs = r; partials of |b|^2, against which
 // the tolerance is measured.
 template <class V>
-__global__ __launch_bounds__(64) void k_cg_init_warm(Ctx c, const TileRec* __restrict__ list, int n, const float* __restrict__ B,
-                                                     int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_init_warm(const TileRec* __restrict__ list, int n, int flags,
+                                                     const float* __restrict__ B, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float bv[8], av[8], rv[8];
@@ -2218,8 +2270,8 @@ __global__ __launch_bounds__(256) void k_gather_recs(const TileRec* const* __res
 
 // partials of gamma = r.z over LEAF tiles (GMGSolver.cu:634)
 template <class V>
-__global__ __launch_bounds__(64) void k_cg_dot_rz(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_dot_rz(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
@@ -2240,8 +2292,8 @@ __global__ __launch_bounds__(64) void k_cg_dot_rz(Ctx c, const TileRec* __restri
 // children's p (the parent's INTERIOR values, PoissonGrid.cu:585-605) is not
 // stored: the operator reads it from here (k_apply<true>).
 template <class V>
-__global__ __launch_bounds__(64) void k_cg_update_p(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_update_p(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
@@ -2272,9 +2324,10 @@ __global__ __launch_bounds__(64) void k_cg_update_p(Ctx c, const TileRec* __rest
 // PG (the CG iteration's operator on p): GHOST values from their parents
 // (stage_issue_pg), as p is not copied into ghost tiles.
 template <bool PG = false>
-__global__ __launch_bounds__(64) void k_apply(Ctx c, const TileRec* __restrict__ list, int n, const float* __restrict__ X,
-                                              float* __restrict__ AX, int sl, int diag, int dot, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_apply(const TileRec* __restrict__ list, int n, int flags,
+                                              const float* __restrict__ X, float* __restrict__ AX, int sl, int diag,
+                                              int dot, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   __shared__ float gl[512];
@@ -2311,8 +2364,8 @@ __global__ __launch_bounds__(64) void k_apply(Ctx c, const TileRec* __restrict__
 
 // LEAF tiles with ghost children: A p += ghost row sums (the += of
 // AccumulateToParents128), then the p.Ap partial (GMGSolver.cu:580).
-__global__ __launch_bounds__(64) void k_ghost_gather(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_ghost_gather(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float av[8], pv[8];
@@ -2343,8 +2396,8 @@ __global__ __launch_bounds__(64) void k_ghost_gather(Ctx c, const TileRec* __res
 // also the next V-cycle's rhs; partials of |r|^2.  The iteration's x += alpha p
 // is left to the next k_cg_update_p (or k_cg_finish_x).
 template <class V>
-__global__ __launch_bounds__(64) void k_cg_update_xr(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_update_xr(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
@@ -2367,8 +2420,8 @@ __global__ __launch_bounds__(64) void k_cg_update_xr(Ctx c, const TileRec* __res
 // The last iteration's pending x += alpha p on INTERIOR cells of LEAF tiles,
 // once after a problem's iterations end (every problem of the list, done or
 // not; none when no iteration ran).
-__global__ __launch_bounds__(64) void k_cg_finish_x(Ctx c, const TileRec* __restrict__ list, int n, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_cg_finish_x(const TileRec* __restrict__ list, int n, int flags, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
@@ -2508,8 +2561,9 @@ __global__ __launch_bounds__(FIN_THREADS) void k_finalize(Ctx c, int mode, int f
 // Pure-Neumann re-centring (MeanAsync + ReCenterLeafVoxels,
 // PoissonGrid.cu:231-325, PoissonSolver.cu:356-368): mean of r over all cells
 // of LEAF tiles divided by the INTERIOR count, subtracted on INTERIOR cells.
-__global__ __launch_bounds__(64) void k_mean(Ctx c, const TileRec* __restrict__ list, int n, const float* __restrict__ X, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_mean(const TileRec* __restrict__ list, int n, int flags,
+                                             const float* __restrict__ X, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   if (prob_done(c, T, flags)) return;
   ProbState* ps = c.ps + T.prob;
   if (!ps->pure_neumann) return;
@@ -2525,9 +2579,9 @@ __global__ __launch_bounds__(64) void k_mean(Ctx c, const TileRec* __restrict__ 
   if (lane == 0) { c.part[T.leaf_slot] = a; c.part2[T.leaf_slot] = q; }
 }
 template <class V>
-__global__ __launch_bounds__(64) void k_subtract_mean(Ctx c, const TileRec* __restrict__ list, int n, float* __restrict__ X,
-                                                      int write_rhsv, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_subtract_mean(const TileRec* __restrict__ list, int n, int flags,
+                                                      float* __restrict__ X, int write_rhsv, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   if (prob_done(c, T, flags)) return;
   ProbState* ps = c.ps + T.prob;
   if (!ps->pure_neumann) return;
@@ -2867,9 +2921,10 @@ __device__ __forceinline__ void amg_rows(const TileRec& T, const float* __restri
 
 // One colour of GaussSeidelAMG (AMGSolver.cu:540-578) on LEAF|NONLEAF tiles
 // (D = 0 leaves the cell unchanged, as in the GMG smoother).
-__global__ __launch_bounds__(64) void k_amg_gs(Ctx c, const TileRec* __restrict__ list, int n, float* __restrict__ X,
-                                               const float* __restrict__ RHS, AmgC A, int color, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_amg_gs(const TileRec* __restrict__ list, int n, int flags,
+                                               float* __restrict__ X, const float* __restrict__ RHS, AmgC A,
+                                               int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   float x0[8], ax[8];
   amg_rows(T, X, A, x0, ax);
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
@@ -2892,10 +2947,10 @@ __global__ __launch_bounds__(64) void k_amg_gs(Ctx c, const TileRec* __restrict_
 
 // The residual of VCycleAMG (AMGSolver.cu:638-642): tmp = rhs - A x on
 // INTERIOR cells, 0 elsewhere, on every tile of a level.
-__global__ __launch_bounds__(64) void k_amg_residual(Ctx c, const TileRec* __restrict__ list, int n,
+__global__ __launch_bounds__(64) void k_amg_residual(const TileRec* __restrict__ list, int n, int flags,
                                                      const float* __restrict__ X, const float* __restrict__ RHS,
-                                                     float* __restrict__ TMP, AmgC A, int flags) {
-  TILE_KERNEL_PROLOGUE
+                                                     float* __restrict__ TMP, AmgC A, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   float x0[8], ax[8], rhs[8];
   amg_rows(T, X, A, x0, ax);
   const size_t b = size_t(T.self) * 512 + lane_id() * 8;
@@ -2910,10 +2965,10 @@ __global__ __launch_bounds__(64) void k_amg_residual(Ctx c, const TileRec* __res
 // Restrict (PoissonSolver.cu:292-316) from the child side: the LEAF|NONLEAF
 // tiles of a level fill their NONLEAF parent's octant, rhs = sum over the 8
 // children (x fastest) of their INTERIOR residuals, times one_over_alpha.
-__global__ __launch_bounds__(64) void k_amg_restrict(Ctx c, const TileRec* __restrict__ list, int n,
+__global__ __launch_bounds__(64) void k_amg_restrict(const TileRec* __restrict__ list, int n, int flags,
                                                      const float* __restrict__ TMP, float* __restrict__ RHS, AmgC A,
-                                                     float alpha, int flags) {
-  TILE_KERNEL_PROLOGUE
+                                                     float alpha, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   if (prob_done(c, T, flags)) return;
   const int lane = lane_id();
   const int qi = lane >> 4, qj = (lane >> 2) & 3, qk = lane & 3;
@@ -2931,10 +2986,10 @@ __global__ __launch_bounds__(64) void k_amg_restrict(Ctx c, const TileRec* __res
 // VCycleAMG's rhs on the LEAF and GHOST tiles of the coarser level
 // (AMGSolver.cu:652-656): LEAF rhs = f plus the 8-cell sums of the GHOST
 // children's residuals (AccumulateToParents, PoissonGrid.cu:721-755), GHOST rhs = 0.
-__global__ __launch_bounds__(64) void k_amg_leaf_rhs(Ctx c, const TileRec* __restrict__ list, int n,
+__global__ __launch_bounds__(64) void k_amg_leaf_rhs(const TileRec* __restrict__ list, int n, int flags,
                                                      const float* __restrict__ TMP, const float* __restrict__ F,
-                                                     float* __restrict__ RHS, int flags) {
-  TILE_KERNEL_PROLOGUE
+                                                     float* __restrict__ RHS, Ctx c) {
+  TILE_KERNEL_PROLOGUE_ALL
   const uint8_t ty = tr_type(T);
   if (ty == T_NONLEAF || prob_done(c, T, flags)) return;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
@@ -2964,9 +3019,9 @@ __global__ __launch_bounds__(64) void k_amg_leaf_rhs(Ctx c, const TileRec* __res
 // ProlongateAndUpdate128 (GMGSolver.cu:345-380) on the AMG hierarchy, natural
 // order: GHOST x = parent x on INTERIOR cells, others x += pcoef parent x on
 // INTERIOR cells, 0 elsewhere.
-__global__ __launch_bounds__(64) void k_amg_prolong(Ctx c, const TileRec* __restrict__ list, int n, float* __restrict__ X,
-                                                    AmgC A, float pcoef, int flags) {
-  TILE_KERNEL_PROLOGUE
+__global__ __launch_bounds__(64) void k_amg_prolong(const TileRec* __restrict__ list, int n, int flags,
+                                                    float* __restrict__ X, AmgC A, float pcoef, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t b = size_t(T.self) * 512 + lane * 8;
   float x[8];
@@ -3440,7 +3495,7 @@ __device__ __forceinline__ void tile_accumulate_children(const Ctx& c, const Til
 __global__ __launch_bounds__(64) void k_accumulate_children(Ctx c, const TileRec* __restrict__ list, int n,
                                                             float* __restrict__ X, uint8_t mask, float coeff) {
   const int flags = 0;
-  TILE_KERNEL_PROLOGUE
+  TILE_KERNEL_PROLOGUE_ALL
   tile_accumulate_children(c, T, X, mask, coeff);
 }
 // The same for the three face-velocity channels in one launch (one after the
@@ -3448,7 +3503,7 @@ __global__ __launch_bounds__(64) void k_accumulate_children(Ctx c, const TileRec
 __global__ __launch_bounds__(64) void k_accumulate_children_vel(Ctx c, const TileRec* __restrict__ list, int n, Vel U,
                                                                 uint8_t mask, float coeff) {
   const int flags = 0;
-  TILE_KERNEL_PROLOGUE
+  TILE_KERNEL_PROLOGUE_ALL
   for (int a = 0; a < 3; a++) tile_accumulate_children(c, T, U.u[a], mask, coeff);
 }
 

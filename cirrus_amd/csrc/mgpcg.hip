@@ -803,13 +803,13 @@ template <class V, bool DOT>
 void launch_gs_as(cg_problem& P, const DList& a, const Ctx& c, int l, V* Z, const V* R, int color, int flags) {
   const int lw = P.gs_block == 8 ? loop_waves<V, DOT>() : 0;
   if (lw > 0 && a.n > lw) {
-    k_gs_color_loop<V, DOT><<<unsigned(lw), 64, 0, P.stream>>>(c, P.L(a), a.n, l, Z, R, color, flags);
+    k_gs_color_loop<V, DOT><<<unsigned(lw), 64, 0, P.stream>>>(P.L(a), a.n, flags, l, Z, R, color, c);
   } else if (P.gs_block == 2 && a.n > 1)
-    k_gs_color2<V, DOT><<<grid_for((a.n + 1) / 2, flags), 64, 0, P.stream>>>(c, P.L(a), a.n, l, Z, R, color, flags);
+    k_gs_color2<V, DOT><<<grid_for((a.n + 1) / 2, flags), 64, 0, P.stream>>>(P.L(a), a.n, flags, l, Z, R, color, c);
   else if (P.gs_block == 4 && a.n > 1)
-    k_gs_color4<V, DOT><<<grid_for((a.n + 3) / 4, flags), 256, 0, P.stream>>>(c, P.L(a), a.n, l, Z, R, color, flags);
+    k_gs_color4<V, DOT><<<grid_for((a.n + 3) / 4, flags), 256, 0, P.stream>>>(P.L(a), a.n, flags, l, Z, R, color, c);
   else
-    k_gs_color<V, DOT><<<grid_for(a.n, flags), 64, 0, P.stream>>>(c, P.L(a), a.n, l, Z, R, color, flags);
+    k_gs_color<V, DOT><<<grid_for(a.n, flags), 64, 0, P.stream>>>(P.L(a), a.n, flags, l, Z, R, color, c);
 }
 template <class V>
 void launch_gs(cg_problem& P, const DList& a, const Ctx& c, int l, V* Z, const V* R, int color, int flags) {
@@ -826,8 +826,9 @@ void launch_gs(cg_problem& P, const DList& a, const Ctx& c, int l, V* Z, const V
 template <class V>
 void launch_gs_pair(cg_problem& P, const DList& a, const Ctx& c, const V* XI, const V* XG, V* XO, int c1, int flags) {
   if (a.n == 0) return;
-  if (flags & F_DOT_RZ) k_gs_pair<V, true><<<grid_for(a.n, flags), 64, 0, P.stream>>>(c, P.L(a), a.n, XI, XG, XO, c1, flags);
-  else k_gs_pair<V, false><<<grid_for(a.n, flags), 64, 0, P.stream>>>(c, P.L(a), a.n, XI, XG, XO, c1, flags);
+  if (flags & F_DOT_RZ) k_gs_pair<V, true><<<grid_for(a.n, flags), 64, 0, P.stream>>>(P.L(a), a.n, flags, XI, XG, XO, c1,
+      c);
+  else k_gs_pair<V, false><<<grid_for(a.n, flags), 64, 0, P.stream>>>(P.L(a), a.n, flags, XI, XG, XO, c1, c);
 }
 // The pool's V-cycle vectors of storage type V.
 template <class V> V* pool_z(cg_problem& P);
@@ -902,7 +903,7 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
       for (int s = 0; s < v.nu; s++) {
         if (s == 0 && P.d_diag && (std::is_same<V, float>::value || a.n <= P.fused16_max)) {
           // both colours of the first iteration from the zero guess in one launch
-          if (a.n) k_gs_first<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(c, P.L(a), a.n, cur, base | F_GHOST_ZERO);
+          if (a.n) k_gs_first<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(P.L(a), a.n, base | F_GHOST_ZERO, cur, c);
           continue;
         }
         if (s == 0 || !pairs) {  // two colour passes in place (s == 0: from the zero guess)
@@ -919,16 +920,16 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
       for (int s = 0; s < v.nu; s++) {
         V* dst = ((v.nu - 1 - s) % 2 == 0) ? Z : ZB;
         int fl = base | F_GHOST_ZERO | (s == 0 ? F_ZERO_X : 0);
-        if (a.n) k_jacobi<V><<<grid_for(a.n, fl), 64, 0, P.stream>>>(c, P.L(a), a.n, l, src, Z, dst, R, v.omega, fl);
+        if (a.n) k_jacobi<V><<<grid_for(a.n, fl), 64, 0, P.stream>>>(P.L(a), a.n, fl, l, src, Z, dst, R, v.omega, c);
         src = dst;
       }
     }
     const DList& al = P.lvlg[l];
     int fl = base | F_GHOST_ZERO | (v.nu == 0 ? F_ZERO_X : 0);
     if (al.n > P.eager_max)
-      k_restrict<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(c, P.L(al), al.n, l, Z, R, nullptr, v.ooa, fl);
+      k_restrict<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
     else if (al.n)
-      k_restrict<V, true><<<grid_for(al.n, fl), 64, 0, P.stream>>>(c, P.L(al), al.n, l, Z, R, nullptr, v.ooa, fl);
+      k_restrict<V, true><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
   }
   if (!P.plans.empty()) {
     VCycleArgs va{v.nu, v.coarsest, v.smoother, v.omega, v.ooa, v.pcoef};
@@ -955,9 +956,9 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
     if (!jac && v.nu > 0) {
       // prolongation fused into the first (black) pass; the level's result goes to ZO
       if (al.n > P.eager_max)
-        k_gs_prolong<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(c, P.L(al), al.n, Z, ZO, v.pcoef, 1, base);
+        k_gs_prolong<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, Z, ZO, v.pcoef, 1, c);
       else if (al.n)
-        k_gs_prolong_eager<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(c, P.L(al), al.n, Z, ZO, v.pcoef, 1, base);
+        k_gs_prolong_eager<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, Z, ZO, v.pcoef, 1, c);
       if (c.tiles == nullptr || v.nu < 2) {
         launch_gs(P, a, c, l, ZO, R, 0, base | (v.nu == 1 ? last_flags : 0));
         for (int s = 1; s < v.nu; s++) {
@@ -972,7 +973,7 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
       // their prolongated values in ZO throughout
       V* cur = ZO;
       if ((v.nu - 1) % 2 == 1) {
-        if (a.n) k_gs_color_to<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(c, P.L(a), a.n, ZO, Z, 0, base);
+        if (a.n) k_gs_color_to<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(P.L(a), a.n, base, ZO, Z, 0, c);
         cur = Z;
       } else {
         launch_gs(P, a, c, l, ZO, R, 0, base);
@@ -986,13 +987,13 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
     }
     V* XO = (jac && (v.nu % 2 == 1)) ? ZB : ZO;
     int fl = base | (v.nu == 0 ? F_ZERO_X : 0);
-    if (al.n) k_prolong<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(c, P.L(al), al.n, l, ZO, Z, XO, ZO, v.pcoef, fl);
+    if (al.n) k_prolong<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, ZO, Z, XO, ZO, v.pcoef, c);
     if (!jac) continue;
     {
       const V* src = XO;
       for (int s = 0; s < v.nu; s++) {
         V* dst = ((v.nu - 1 - s) % 2 == 0) ? Z : ZB;
-        if (a.n) k_jacobi<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(c, P.L(a), a.n, l, src, Z, dst, R, v.omega, base);
+        if (a.n) k_jacobi<V><<<grid_for(a.n, base), 64, 0, P.stream>>>(P.L(a), a.n, base, l, src, Z, dst, R, v.omega, c);
         src = dst;
       }
     }
@@ -1045,22 +1046,25 @@ void enqueue_amg_vcycle(cg_problem& P, const VParams& v) {
   const float* F = c.r;
   k_amg_init<<<grid_for(P.all.n, fl), 64, 0, P.stream>>>(P.L(P.all), P.all.n, X, F, RHS, fl);
   auto gs = [&](int l, int color) {
-    if (P.act[l].n) k_amg_gs<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(c, P.L(P.act[l]), P.act[l].n, X, RHS, A, color, fl);
+    if (P.act[l].n) k_amg_gs<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(P.L(P.act[l]), P.act[l].n, fl, X, RHS, A,
+        color, c);
   };
   const int L = P.max_level;
   for (int l = L; l >= 1; l--) {
     for (int it = 0; it < v.nu; it++) { gs(l, 0); gs(l, 1); }
     if (P.lvl[l].n)
-      k_amg_residual<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(c, P.L(P.lvl[l]), P.lvl[l].n, X, RHS, TMP, A, fl);
+      k_amg_residual<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l]), P.lvl[l].n, fl, X, RHS, TMP, A, c);
     if (P.act[l].n)
-      k_amg_restrict<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(c, P.L(P.act[l]), P.act[l].n, TMP, RHS, A, v.ooa, fl);
+      k_amg_restrict<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(P.L(P.act[l]), P.act[l].n, fl, TMP, RHS, A, v.ooa, c);
     if (P.lvl[l - 1].n)
-      k_amg_leaf_rhs<<<grid_for(P.lvl[l - 1].n, fl), 64, 0, P.stream>>>(c, P.L(P.lvl[l - 1]), P.lvl[l - 1].n, TMP, F, RHS, fl);
+      k_amg_leaf_rhs<<<grid_for(P.lvl[l - 1].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l - 1]), P.lvl[l - 1].n, fl, TMP, F,
+          RHS, c);
   }
   for (int it = 0; it < v.coarsest / 2; it++) { gs(0, 0); gs(0, 1); }
   for (int it = 0; it < v.coarsest / 2; it++) { gs(0, 1); gs(0, 0); }
   for (int l = 1; l <= L; l++) {
-    if (P.lvl[l].n) k_amg_prolong<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(c, P.L(P.lvl[l]), P.lvl[l].n, X, A, v.pcoef, fl);
+    if (P.lvl[l].n) k_amg_prolong<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l]), P.lvl[l].n, fl, X, A,
+        v.pcoef, c);
     for (int it = 0; it < v.nu; it++) { gs(l, 1); gs(l, 0); }
   }
   k_to_split<<<unsigned(P.leaf.n), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, X, c.z);
@@ -1081,9 +1085,9 @@ void enqueue_cg_iteration(cg_problem& P, const VParams& vp, int pure_neumann) {
   const bool one = P.nprob == 1 && !c.pmap && P.leaf_count.size() == 1 && P.leaf_begin.size() == 1;
   const int rb = one ? P.leaf_begin[0] : 0, rc = one ? P.leaf_count[0] : -1;
   if (pure_neumann) {
-    k_mean<<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, fl & ~F_INERT);
+    k_mean<<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl & ~F_INERT, c.r, c);
     k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_MEAN, fl);
-    k_subtract_mean<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, 1, fl & ~F_INERT);
+    k_subtract_mean<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl & ~F_INERT, c.r, 1, c);
   }
   // RB-GS: down-sweep in the scratch buffer, z assembled in z by the up-sweep
   V* Z = pool_z<V>(P);
@@ -1092,13 +1096,13 @@ void enqueue_cg_iteration(cg_problem& P, const VParams& vp, int pure_neumann) {
   const bool rz_fused = !v.amg && v.smoother == CG_SMOOTH_RBGS && v.nu > 0 && P.rz_in_vcycle;
   if (v.amg) enqueue_amg_vcycle(P, v);
   else enqueue_vcycle<V>(P, v.smoother == CG_SMOOTH_RBGS ? pool_zb<V>(P) : Z, Z, nullptr, v, rz_fused ? F_DOT_RZ : 0);
-  if (!rz_fused) k_cg_dot_rz<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, fl);
+  if (!rz_fused) k_cg_dot_rz<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
   k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_RZ, fl, rb, rc);
-  k_cg_update_p<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, fl);
-  k_apply<true><<<grid_for(P.applyl.n, fl), 64, 0, P.stream>>>(c, P.L(P.applyl), P.applyl.n, c.p, c.ap, -1, 0, 1, fl);
-  if (P.gather.n) k_ghost_gather<<<grid_for(P.gather.n, fl), 64, 0, P.stream>>>(c, P.L(P.gather), P.gather.n, fl);
+  k_cg_update_p<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
+  k_apply<true><<<grid_for(P.applyl.n, fl), 64, 0, P.stream>>>(P.L(P.applyl), P.applyl.n, fl, c.p, c.ap, -1, 0, 1, c);
+  if (P.gather.n) k_ghost_gather<<<grid_for(P.gather.n, fl), 64, 0, P.stream>>>(P.L(P.gather), P.gather.n, fl, c);
   k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_PAP, fl, rb, rc);
-  k_cg_update_xr<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, fl);
+  k_cg_update_xr<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
   k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_RR, fl, rb, rc);
 }
 void enqueue_cg_iteration(cg_problem& P, const VParams& v, int pure_neumann, int storage) {
@@ -1141,7 +1145,7 @@ double dot_types(cg_problem& P, const float* A, const float* B, int types) {
 void full_negative_laplacian(cg_problem& P, float* X, float* AX, int diag) {
   const Ctx c = P.ctx();
   if (P.ghosts.n) k_propagate_ghosts<<<P.ghosts.n, 64, 0, P.stream>>>(c, P.L(P.ghosts), P.ghosts.n, X, X);
-  k_apply<<<P.applyl.n, 64, 0, P.stream>>>(c, P.L(P.applyl), P.applyl.n, X, AX, -1, diag, 0, 0);
+  k_apply<<<P.applyl.n, 64, 0, P.stream>>>(P.L(P.applyl), P.applyl.n, 0, X, AX, -1, diag, 0, c);
   if (P.ghosts.n) k_accumulate_ghosts<<<P.ghosts.n, 64, 0, P.stream>>>(c, P.L(P.ghosts), P.ghosts.n, AX);
 }
 
@@ -1241,11 +1245,11 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
     k_scale_leaf<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, 1);
   }
   if (prm.storage == CG_STORE_BF16)
-    k_cg_init<bf16><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, P.swz);
+    k_cg_init<bf16><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz, c);
   else if (f16s)
-    k_cg_init<f16><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, P.swz);
+    k_cg_init<f16><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz, c);
   else
-    k_cg_init<float><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, P.swz);
+    k_cg_init<float><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz, c);
   k_finalize<<<unsigned(P.nprob), FIN_THREADS, 0, P.stream>>>(c, FIN_BB, 0);
   HIPC(hipGetLastError());
 
@@ -1301,8 +1305,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
     slot = 1 - slot;
   }
   // the last iteration's x update (k_cg_update_p applies each earlier one)
-  k_cg_finish_x<<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n,
-                                                                 P.swz | (c.inert ? F_INERT : 0));
+  k_cg_finish_x<<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz | (c.inert ? F_INERT : 0), c);
   if (f16s) {  // back to the caller's scale: x and the residual r
     k_scale_leaf<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.x, -1);
     k_scale_leaf<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, -1);
@@ -2147,8 +2150,8 @@ cg_status cg_negative_laplacian_same_level(cg_problem* p, int32_t level, int32_t
     if (l.empty()) return;
     const TileRec* dl = tmp_list(*p, l);
     const Ctx c = p->ctx();
-    k_apply<<<unsigned(l.size()), 64, 0, p->stream>>>(c, dl, int(l.size()), p->d_ch[x_channel], p->d_ch[ax_channel],
-                                                       subtree_level, calc_diag, 0, 0);
+    k_apply<<<unsigned(l.size()), 64, 0, p->stream>>>(dl, int(l.size()), 0, p->d_ch[x_channel], p->d_ch[ax_channel],
+        subtree_level, calc_diag, 0, c);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));
   });
@@ -2180,7 +2183,7 @@ cg_status cg_jacobi_sweep(cg_problem* p, int32_t level, int32_t x_channel, int32
     const float* X = api_split(*p, 0, p->d_ch[x_channel]);
     const float* F = api_split(*p, 1, p->d_ch[rhs_channel]);
     float* Y = api_split(*p, 2, nullptr);
-    k_jacobi<float><<<a.n, 64, 0, p->stream>>>(p->ctx(), p->L(a), a.n, level, X, X, Y, F, omega, 0);
+    k_jacobi<float><<<a.n, 64, 0, p->stream>>>(p->L(a), a.n, 0, level, X, X, Y, F, omega, p->ctx());
     api_unsplit(*p, a, Y, p->d_ch[x_channel]);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));
@@ -2200,7 +2203,7 @@ cg_status cg_residual_restrict(cg_problem* p, int32_t level, int32_t x_channel, 
     const float* X = api_split(*p, 0, p->d_ch[x_channel]);
     const float* F = api_split(*p, 1, p->d_ch[rhs_channel]);
     float* CO = api_split(*p, 2, p->d_ch[coarse_channel]);
-    k_restrict<float><<<al.n, 64, 0, p->stream>>>(p->ctx(), p->L(al), al.n, level, X, F, CO, one_over_alpha, 0);
+    k_restrict<float><<<al.n, 64, 0, p->stream>>>(p->L(al), al.n, 0, level, X, F, CO, one_over_alpha, p->ctx());
     api_unsplit(*p, p->all, CO, p->d_ch[coarse_channel]);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));
@@ -2217,7 +2220,7 @@ cg_status cg_prolongate(cg_problem* p, int32_t level, int32_t coarse_channel, in
     if (!al.n) return;
     const float* XC = api_split(*p, 0, p->d_ch[coarse_channel]);
     float* F = api_split(*p, 1, p->d_ch[fine_channel]);
-    k_prolong<float><<<al.n, 64, 0, p->stream>>>(p->ctx(), p->L(al), al.n, level, XC, F, F, F, prolong_coeff, 0);
+    k_prolong<float><<<al.n, 64, 0, p->stream>>>(p->L(al), al.n, 0, level, XC, F, F, F, prolong_coeff, p->ctx());
     api_unsplit(*p, al, F, p->d_ch[fine_channel]);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));
@@ -2270,9 +2273,9 @@ cg_status cg_recenter_leaf_voxels(cg_problem* p, int32_t channel) {
     check_channel(channel);
     set_prob_state(*p, 0.0, 0, 1);
     const Ctx c = p->ctx();
-    k_mean<<<p->leaf.n, 64, 0, p->stream>>>(c, p->L(p->leaf), p->leaf.n, p->d_ch[channel], 0);
+    k_mean<<<p->leaf.n, 64, 0, p->stream>>>(p->L(p->leaf), p->leaf.n, 0, p->d_ch[channel], c);
     k_finalize<<<1, FIN_THREADS, 0, p->stream>>>(c, FIN_MEAN, 0);
-    k_subtract_mean<float><<<p->leaf.n, 64, 0, p->stream>>>(c, p->L(p->leaf), p->leaf.n, p->d_ch[channel], 0, 0);
+    k_subtract_mean<float><<<p->leaf.n, 64, 0, p->stream>>>(p->L(p->leaf), p->leaf.n, 0, p->d_ch[channel], 0, c);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));
   });
@@ -2331,8 +2334,8 @@ cg_status cg_benchmark_kernel(cg_problem* p, int32_t kernel, int32_t level, int3
           const DList& a = P.act[level];
           nt = a.n;
           if (a.n)
-            k_amg_gs<<<grid_for(a.n, base), 64, 0, P.stream>>>(c, P.L(a), a.n, P.d_zb, P.d_ch[CG_CH_TMP], amg_arrays(P), 0,
-                                                               base);
+            k_amg_gs<<<grid_for(a.n, base), 64, 0, P.stream>>>(P.L(a), a.n, base, P.d_zb, P.d_ch[CG_CH_TMP],
+                amg_arrays(P), 0, c);
           break;
         }
         case CG_KERNEL_GS_SWEEP_F16: {
@@ -2344,42 +2347,44 @@ cg_status cg_benchmark_kernel(cg_problem* p, int32_t kernel, int32_t level, int3
         case CG_KERNEL_GS_PROLONG_BF16: {
           const DList& al = P.lvl[level];
           nt = al.n;
-          k_gs_prolong<bf16><<<grid_for(al.n, base), 64, 0, P.stream>>>(c, P.L(al), al.n, c.zbh, c.zh, 1.f, 1, base);
+          k_gs_prolong<bf16><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, c.zbh, c.zh, 1.f, 1, c);
           break;
         }
         case CG_KERNEL_JACOBI: {
           const DList& a = P.act[level];
           nt = a.n;
-          if (a.n) k_jacobi<float><<<grid_for(a.n, base), 64, 0, P.stream>>>(c, P.L(a), a.n, level, c.z, c.z, c.zb, c.r, 0.5f, base);
+          if (a.n) k_jacobi<float><<<grid_for(a.n, base), 64, 0, P.stream>>>(P.L(a), a.n, base, level, c.z, c.z, c.zb,
+              c.r, 0.5f, c);
           break;
         }
         case CG_KERNEL_APPLY:
           nt = P.applyl.n;
-          k_apply<true><<<grid_for(P.applyl.n, base), 64, 0, P.stream>>>(c, P.L(P.applyl), P.applyl.n, c.p, c.ap, -1, 0, 1,
-                                                                        base);
+          k_apply<true><<<grid_for(P.applyl.n, base), 64, 0, P.stream>>>(P.L(P.applyl), P.applyl.n, base, c.p, c.ap, -1,
+              0, 1, c);
           break;
         case CG_KERNEL_RESTRICT: {
           const DList& al = P.lvl[level];
           nt = al.n;
           int fl = base | F_GHOST_ZERO;
-          k_restrict<float><<<grid_for(al.n, fl), 64, 0, P.stream>>>(c, P.L(al), al.n, level, c.z, c.r, nullptr, 1.f, fl);
+          k_restrict<float><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, level, c.z, c.r, nullptr, 1.f, c);
           break;
         }
         case CG_KERNEL_PROLONG: {
           const DList& al = P.lvl[level];
           nt = al.n;
-          k_prolong<float><<<grid_for(al.n, base), 64, 0, P.stream>>>(c, P.L(al), al.n, level, c.z, c.z, c.zb, c.zb, 1.f, base);
+          k_prolong<float><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, level, c.z, c.z, c.zb, c.zb,
+              1.f, c);
           break;
         }
         case CG_KERNEL_GS_PROLONG: {
           const DList& al = P.lvl[level];
           nt = al.n;
-          k_gs_prolong<float><<<grid_for(al.n, base), 64, 0, P.stream>>>(c, P.L(al), al.n, c.zb, c.z, 1.f, 1, base);
+          k_gs_prolong<float><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, c.zb, c.z, 1.f, 1, c);
           break;
         }
         case CG_KERNEL_UPDATE_XR:
           nt = P.leaf.n;
-          k_cg_update_xr<float><<<grid_for(P.leaf.n, base), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, base);
+          k_cg_update_xr<float><<<grid_for(P.leaf.n, base), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, base, c);
           break;
         case CG_KERNEL_COARSE: {
           nt = int64_t(P.coarse_slots.size());

@@ -771,15 +771,16 @@ void server_start_queued(cg_server& S, int k) {
       k_finalize<<<unsigned(G.nfull), FIN_THREADS, 0, st>>>(group_ctx(S), FIN_IRBB, 0);
     }
     // the step solves A d = float(r) from d = 0
-    if (S.prm.storage == CG_STORE_BF16) k_cg_init<bf16><<<G.leaf.n, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, 0);
-    else k_cg_init<float><<<G.leaf.n, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, 0);
+    if (S.prm.storage == CG_STORE_BF16) k_cg_init<bf16><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, c);
+    else k_cg_init<float><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, c);
   } else {
     float* X = S.d_ch[CG_CH_X];
     if (G.ghosts.n) k_propagate_ghosts<<<G.ghosts.n, 64, 0, st>>>(c, GL(S, G.ghosts), G.ghosts.n, X, X);
-    k_apply<<<G.applyl.n, 64, 0, st>>>(c, GL(S, G.applyl), G.applyl.n, X, c.ap, -1, 0, 0, 0);
+    k_apply<<<G.applyl.n, 64, 0, st>>>(GL(S, G.applyl), G.applyl.n, 0, X, c.ap, -1, 0, 0, c);
     if (G.ghosts.n) k_accumulate_ghosts<<<G.ghosts.n, 64, 0, st>>>(c, GL(S, G.ghosts), G.ghosts.n, c.ap);
-    if (S.prm.storage == CG_STORE_BF16) k_cg_init_warm<bf16><<<G.leaf.n, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, S.d_b, 0);
-    else k_cg_init_warm<float><<<G.leaf.n, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, S.d_b, 0);
+    if (S.prm.storage == CG_STORE_BF16) k_cg_init_warm<bf16><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, S.d_b,
+        c);
+    else k_cg_init_warm<float><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, S.d_b, c);
   }
   Ctx ci = group_ctx(S);
   ci.dflag = S.d_dflag_init;
@@ -927,11 +928,11 @@ void server_collect(cg_server& S, int k) {
   // the last iteration's x update (k_cg_update_p applies each earlier one)
   for (int q : rest) {
     const Instance& I = *S.inst[q];
-    k_cg_finish_x<<<grid_for(I.leaf.n, kSwizzle), 64, 0, stm>>>(c, I.L(I.leaf), I.leaf.n, kSwizzle | F_INERT);
+    k_cg_finish_x<<<grid_for(I.leaf.n, kSwizzle), 64, 0, stm>>>(I.L(I.leaf), I.leaf.n, kSwizzle | F_INERT, c);
   }
   if (!check.empty()) {
     const Group G = group_lists(S, k, GRP_FINISH, check, int(check.size()), nullptr);
-    k_cg_finish_x<<<grid_for(G.leaf.n, kSwizzle), 64, 0, stm>>>(c, GL(S, G.leaf), G.leaf.n, kSwizzle | F_INERT);
+    k_cg_finish_x<<<grid_for(G.leaf.n, kSwizzle), 64, 0, stm>>>(GL(S, G.leaf), G.leaf.n, kSwizzle | F_INERT, c);
     enqueue_verify(S, G, check);
   }
   for (int q : rest) {
