@@ -1820,240 +1820,295 @@ __global__ __launch_bounds__(64) void k_prolong(const TileRec* __restrict__ list
 }
 
 // ---------------------------------------------------------------------------
-// Coarse levels 0..C of the V-cycle (smoothing, restriction, the bottom solve
-// on level 0, prolongation) for one problem in one workgroup, with every tile
-// of those levels (active and ghost, at most CL_MAX_TILES) resident in LDS and
-// one thread per cell.  The host picks C so that these levels are tiny; one
-// launch then replaces the ~10 launches per level a grid-wide phase each would
-// need.  The per-cell arithmetic is the same as the tile kernels', so results
-// are identical; the bottom is GMGSolver.cu:432-433.
+// Coarse levels 0..C (C <= 1) of the V-cycle (smoothing, restriction, the bottom
+// solve on level 0, prolongation) for one problem in one workgroup, every tile
+// of those levels resident in LDS.  The host takes level 0 in when it has at most
+// CL_ROOTS tiles, level 1 when it is the eight children of one of them and holds
+// no GHOST tile (a third level would have 64 tiles); one launch then replaces the
+// ~10 launches per level a grid-wide phase each would need.  The per-cell
+// arithmetic is the tile kernels' (GMGSolver.cu:216-376, bottom :432-433).
 // ---------------------------------------------------------------------------
-constexpr int CL_MAX_TILES = 12;     // tiles on levels 0..C together
-constexpr int CL_MAX_PER_LEVEL = 8;  // tiles on any one of those levels
-constexpr int CL_MAX_LEVELS = 8;
+constexpr int CL_MAX_LEVELS = 2;
+constexpr int CL_ROOTS = 8;                        // tiles on level 0 at most (slots 0 ..)
+constexpr int CL_CHILDREN = 8;                     // tiles on level 1 (slots CL_ROOTS ..)
+constexpr int CL_SLOTS = CL_ROOTS + CL_CHILDREN;
 constexpr int CL_THREADS = 1024;
-constexpr int CL_CPT = CL_MAX_PER_LEVEL * 256 / CL_THREADS;  // cells of one colour per thread
-constexpr int CL_ZERO = CL_MAX_TILES * 512;                 // LDS index of a cell that stays 0
+constexpr int CL_CPT = 8 * 256 / CL_THREADS;       // cells of one colour of a level per thread
+constexpr int CL_ZERO = CL_SLOTS * 512;            // LDS index of a cell that stays 0
 struct alignas(16) CoarseSlot {
   int32_t tile;      // tile index
   int32_t nbr[6];    // slot of the same-level face neighbour (x-,y-,z-,x+,y+,z+), -1: none
   int32_t parent;    // slot of the parent, -1 on level 0
-  int32_t level;
+  int32_t octant;
   float h;
-  uint8_t type, octant, pad[2];
-  float bc[7];       // base coefficients at the slot's own level: faces x-,y-,z-,x+,y+,z+ and inside
+  float bc;          // face coefficient of the slot's level (every face: no GHOST tile, GMGSolver.cu:26-39)
+  int32_t pad;
 };
-static_assert(sizeof(CoarseSlot) == 72 || sizeof(CoarseSlot) == 80, "CoarseSlot layout");
-struct CoarsePlan {
-  int prob;                           // problem index in the pool
-  int C;                              // deepest level held in LDS
-  int nslots;
-  int lvl_begin[CL_MAX_LEVELS + 1];   // slots sorted by level
-  const CoarseSlot* slots;
+static_assert(sizeof(CoarseSlot) == 48, "CoarseSlot is 48 bytes");
+struct alignas(16) CoarsePlan {
+  int32_t prob;      // problem index in the pool
+  int32_t n0, n1;    // tiles on level 0, tiles on level 1 (0: not taken in; CL_CHILDREN)
+  int32_t pad;
+  CoarseSlot slots[CL_SLOTS];  // level 0 from 0, level 1 from CL_ROOTS
 };
 struct VCycleArgs {
   int nu, coarsest, smoother;
   float omega, ooa, pcoef;
 };
+// Colour-split like the V-cycle arrays (slot * 512 + colour * 256 + pencil * 4 +
+// k / 2): consecutive threads work consecutive words, and so do their six
+// neighbour reads.
 struct CoarseLDS {
-  float z[CL_MAX_TILES * 512 + 4];  // V-cycle x of every slot (slot * 512 + cell), then CL_ZERO = 0
-  float b[CL_MAX_TILES][512];       // V-cycle rhs
-  float t[CL_MAX_TILES][512];       // residuals (restriction) or new values (damped Jacobi)
-  alignas(16) uint8_t ct[CL_MAX_TILES][512];
-  CoarseSlot S[CL_MAX_TILES];
+  float z[CL_ZERO + 4];         // V-cycle x of every slot, then CL_ZERO = 0
+  float t[CL_CHILDREN * 512];   // level 1: residuals (restriction) or new values (damped Jacobi)
+  float b0[CL_ROOTS * 512];     // V-cycle rhs of level 0
 };
 
-// The static part of one cell's row, prepared once per level phase and kept in
-// registers: LDS indices of the cell and its six neighbours (faces x-, x+, y-,
-// y+, z-, z+; CL_ZERO outside the grid), the face coefficients after the
-// NEUMANN cut, the diagonal and the rhs.  A pass then costs seven independent
-// LDS reads and the fma chain of cell_row_m, with the same operations in the same
-// order (GMGSolver.cu:56-76).
-struct CellPrep {
-  int own;      // slot * 512 + cell, -1: no cell
-  int nb[6];
-  float cf[6];
-  float dg, h, b;
-  bool in;
-};
-
-__device__ __forceinline__ void cl_prep(const CoarseLDS& M, int s, int cc, CellPrep& P) {
-  const CoarseSlot& S = M.S[s];
-  const int i = cc >> 6, j = (cc >> 3) & 7, k = cc & 7;
-  const uint8_t c0 = M.ct[s][cc];
-  const bool inside[6] = {i > 0, i < 7, j > 0, j < 7, k > 0, k < 7};
-  const int step[6] = {-64, 64, -8, 8, -1, 1};
-  const int face[6] = {0, 3, 1, 4, 2, 5};
-  P.own = s * 512 + cc;
-  float d = 0.f;
-#pragma unroll
-  for (int e = 0; e < 6; e++) {
-    const int q = inside[e] ? s : S.nbr[face[e]];
-    const int nc = inside[e] ? cc + step[e] : cc - 7 * step[e];
-    const uint8_t cn = q < 0 ? uint8_t(C_DIR) : M.ct[q < 0 ? 0 : q][nc];
-    const float bc = inside[e] ? S.bc[6] : S.bc[face[e]];
-    P.nb[e] = q < 0 ? CL_ZERO : q * 512 + nc;
-    P.cf[e] = ((c0 | cn) & C_NEU) ? 0.f : bc;
-    d = d + P.cf[e];
-  }
-  P.in = c0 & C_INT;
-  P.h = S.h;
-  P.dg = P.in ? ((d * P.h) * P.h) * P.h : 0.f;
-  P.b = M.b[s][cc];
+// The quotient a / d, correctly rounded, from rd = 1/d in FP64 (within 2^-51
+// of it): the product's relative error is below 2^-50, and a quotient of two
+// 24-bit significands lies at least 2^-49 (relative) from every rounding
+// boundary of FP32, so the conversion rounds to the same value (results below
+// 2^-126, where FP32 has fewer bits, within one unit of their last place).
+// 4 issue slots against 15.5 for the FP32 division on gfx950.
+__device__ __forceinline__ float div_by(float a, double rd) { return float(double(a) * rd); }
+// 1/d in FP64 for d > 0: the FP32 reciprocal and two Newton steps.
+__device__ __forceinline__ double recip64(float d) {
+  const double dd = double(d);
+  double y = double(__builtin_amdgcn_rcpf(d));
+  y = __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
 }
 
-// A x of a prepared cell (cell_row_m's arithmetic); x0 returns the cell's value.
-__device__ __forceinline__ float cl_ax(const CoarseLDS& M, const CellPrep& P, float& x0) {
-  x0 = M.z[P.own];
+// One cell of a level: LDS byte addresses of its six neighbours (faces x-, x+,
+// y-, y+, z-, z+; CL_ZERO outside the grid, the cell itself across a face cut by
+// a NEUMANN cell, so that its term is c * 0), the reciprocal of its diagonal (0:
+// the cell is not updated) and its rhs.  Prepared once per launch and kept in
+// registers.
+struct CoarseCell {
+  uint32_t nb[3];   // two 16-bit addresses each
+  double rd;
+  float b;
+};
+__device__ __forceinline__ float& cl_at(CoarseLDS& M, uint32_t byte) {
+  return *reinterpret_cast<float*>(reinterpret_cast<char*>(M.z) + byte);
+}
+// cell r (pencil * 4 + k / 2) of colour col of slot s, with face mask m and diagonal d
+__device__ __forceinline__ void cl_prep(const CoarseSlot& S, int s, int col, int r, uint32_t m, float d, CoarseCell& P) {
+  const int i = r >> 5, j = (r >> 2) & 7, e = r & 3;
+  const bool p = ((col + i + j) & 1) != 0;  // the cell is k = 2 e + p
+  const int oth = ((col ^ 1) << 8) + r;     // the other colour's cell of the same pencil and e
+  const int own = s * 512 + (col << 8) + r, base = s * 512 + oth;
+  auto at = [&](int q, int cell) { return q < 0 ? CL_ZERO : q * 512 + cell; };
+  int nb[6];
+  nb[0] = i > 0 ? base - 32 : at(S.nbr[0], oth + 224);
+  nb[1] = i < 7 ? base + 32 : at(S.nbr[3], oth - 224);
+  nb[2] = j > 0 ? base - 4 : at(S.nbr[1], oth + 28);
+  nb[3] = j < 7 ? base + 4 : at(S.nbr[4], oth - 28);
+  nb[4] = p ? base : (e > 0 ? base - 1 : at(S.nbr[2], oth + 3));
+  nb[5] = p ? (e < 3 ? base + 1 : at(S.nbr[5], oth - 3)) : base;
+#pragma unroll
+  for (int f = 0; f < 6; f++) nb[f] = 4 * (((m >> f) & 1) ? nb[f] : own);
+#pragma unroll
+  for (int f = 0; f < 3; f++) P.nb[f] = uint32_t(nb[2 * f]) | (uint32_t(nb[2 * f + 1]) << 16);
+  P.rd = d > 0.f ? recip64(d) : 0.0;  // D is 0 off INTERIOR cells
+}
+// b - A x of a prepared cell with value x0 (cell_row_m's operations; a cut face
+// adds c * 0).
+__device__ __forceinline__ float cl_residual(CoarseLDS& M, const CoarseCell& P, float x0, bool in, float cf, float h) {
   float xn[6];
 #pragma unroll
-  for (int e = 0; e < 6; e++) xn[e] = M.z[P.nb[e]];
+  for (int f = 0; f < 3; f++) {
+    xn[2 * f] = cl_at(M, P.nb[f] & 0xffffu);
+    xn[2 * f + 1] = cl_at(M, P.nb[f] >> 16);
+  }
   float sum = 0.f;
 #pragma unroll
-  for (int e = 0; e < 6; e++) sum = __builtin_fmaf(P.cf[e], x0 - xn[e], sum);
-  return P.in ? ((sum * P.h) * P.h) * P.h : 0.f;
+  for (int f = 0; f < 6; f++) sum = __builtin_fmaf(cf, x0 - xn[f], sum);
+  return P.b - (in ? ((sum * h) * h) * h : 0.f);
+}
+// The cells of one level that a thread works: cell (tid & 255) of each colour of
+// its slots (tid >> 8) + 4 m (one slot per wavefront and m).
+struct CoarseCells {
+  CoarseCell P[2][CL_CPT];  // [colour][m]
+  uint32_t in;              // bit 2 * m + colour: INTERIOR
+  uint32_t own;             // LDS byte address of colour 0, m = 0 (+ CL_COL for colour 1, + CL_M per m)
+  int n;                    // m < n exist (level 1: all)
+  float h, cf;
+};
+constexpr uint32_t CL_COL = 1024, CL_M = 8192;
+// The loads of a level's cells (a slot that does not exist reads slot 0's tile)
+struct CoarseRaw {
+  uint32_t mask[2][CL_CPT];
+  float d[2][CL_CPT], b[2][CL_CPT];
+};
+template <class V>
+__device__ __forceinline__ void cl_issue(const Ctx& c, const CoarsePlan& cp, int first, int n, CoarseRaw& R) {
+  const int q0 = uni(int(threadIdx.x) >> 8), r = threadIdx.x & 255;
+#pragma unroll
+  for (int m = 0; m < CL_CPT; m++) {
+    const size_t tile = size_t(cp.slots[q0 + 4 * m < n ? first + q0 + 4 * m : 0].tile) * 512;
+#pragma unroll
+    for (int col = 0; col < 2; col++) {
+      R.mask[col][m] = reinterpret_cast<const uint8_t*>(c.fsplit)[tile + col * 256 + r];
+      R.d[col][m] = c.diag[tile + col * 256 + r];
+      R.b[col][m] = to_f(vc_rhs<V>(c)[tile + col * 256 + r]);
+    }
+  }
+}
+__device__ __forceinline__ void cl_commit(const CoarsePlan& cp, int first, int n, const CoarseRaw& R, CoarseLDS& M,
+                                          CoarseCells& L) {
+  const int q0 = uni(int(threadIdx.x) >> 8), r = threadIdx.x & 255;
+  L.own = uint32_t(4 * ((first + q0) * 512 + r));
+  L.n = n > q0 ? (n - q0 + 3) >> 2 : 0;
+  L.h = cp.slots[n ? first : 0].h;
+  L.cf = cp.slots[n ? first : 0].bc;
+  L.in = 0;
+#pragma unroll
+  for (int m = 0; m < CL_CPT; m++)
+    if (m < L.n) {
+      const int s = first + q0 + 4 * m;
+#pragma unroll
+      for (int col = 0; col < 2; col++) {
+        L.P[col][m].b = R.b[col][m];
+        L.in |= uint32_t((R.mask[col][m] & M_INT) != 0) << (2 * m + col);
+        cl_prep(cp.slots[s], s, col, r, R.mask[col][m], R.d[col][m], L.P[col][m]);
+        cl_at(M, L.own + m * CL_M + col * CL_COL) = 0.f;
+      }
+    }
+}
+// f(m, byte address) for each of the thread's cells of colour col; FULL: every
+// m exists (level 1), so the cells' latencies overlap
+template <bool FULL, class F>
+__device__ __forceinline__ void cl_each(const CoarseCells& L, int col, F f) {
+#pragma unroll
+  for (int m = 0; m < CL_CPT; m++)
+    if (FULL || m < L.n) f(m, L.own + m * CL_M + col * CL_COL);
+}
+// one red-black colour pass
+template <class V, bool FULL>
+__device__ __forceinline__ void cl_gs(CoarseLDS& M, const CoarseCells& L, int col) {
+  float nv[CL_CPT];
+  cl_each<FULL>(L, col, [&](int m, uint32_t at) {
+    const CoarseCell& Q = L.P[col][m];
+    const float x0 = cl_at(M, at);
+    const float res = cl_residual(M, Q, x0, true, L.cf, L.h);  // used on INTERIOR cells only
+    nv[m] = vround<V>(x0 + (Q.rd != 0.0 ? div_by(res, Q.rd) : 0.f));
+  });
+  cl_each<FULL>(L, col, [&](int m, uint32_t at) { cl_at(M, at) = nv[m]; });
+  __syncthreads();
 }
 
-// The coarse levels 0..C of one V-cycle in one 1024-thread workgroup with every
-// tile of those levels in LDS (the host keeps levels with GHOST tiles out of C
-// and at most CL_MAX_PER_LEVEL tiles on a level): smoothing, restriction and
-// prolongation per level and the bottom sweeps on level 0.  Each thread owns up
-// to CL_CPT cells of each colour of the level being worked and keeps their
-// prepared rows in registers.  One launch replaces ~10 launches per coarse
-// level; the per-cell arithmetic is that of the tile kernels
-// (GMGSolver.cu:216-376, bottom :432-433).
+// Latency bound on one CU (a scalar round trip for the plan, one for the cells,
+// then about 30 passes with a barrier each), so what counts is the length of a
+// pass: the rows are prepared once and kept for the down- and the up-sweep,
+// neighbours are read without bank conflicts, and the division is a product with
+// the prepared reciprocal.  Nine tiles, two sweeps per level, ten bottom
+// iterations: 21.4 -> 13.5 us; six roots alone: 14.2 -> 10.2 us.  (Sixteen tiles
+// on level 1 were measured too: 27 us, no better than that level's grid-wide
+// launches.)
 template <class V>
-__global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(Ctx c, const CoarsePlan* __restrict__ plans, VCycleArgs v,
-                                                           V* Z, int flags) {
+__global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __restrict__ plans, int flags, V* Z,
+                                                           VCycleArgs v, Ctx c) {
   __shared__ CoarseLDS M;
-  __shared__ CoarsePlan cp;  // one workgroup per problem; in LDS, as its level table is indexed per level
   const int tid = threadIdx.x;
-  if (tid == 0) cp = plans[blockIdx.x];
-  __syncthreads();
-  if ((flags & F_CHECK_DONE) && c.ps[cp.prob].done) return;
-  if (tid < cp.nslots) M.S[tid] = cp.slots[tid];
-  if (tid < 4) M.z[CL_ZERO + tid] = 0.f;
-  __syncthreads();
-  // cell types and rhs; z = 0
-  for (int q = tid; q < cp.nslots * 128; q += CL_THREADS) {
-    const int s = q >> 7, o = (q & 127) * 4;
-    const size_t g = size_t(M.S[s].tile) * 512 + o;
-    *reinterpret_cast<float4*>(&M.b[s][o]) = load_quad_split(vc_rhs<V>(c) + size_t(M.S[s].tile) * 512, o >> 3, o & 7);
-    *reinterpret_cast<float4*>(&M.z[s * 512 + o]) = make_float4(0.f, 0.f, 0.f, 0.f);
-    *reinterpret_cast<uint32_t*>(&M.ct[s][o]) = *reinterpret_cast<const uint32_t*>(c.ctype + g);
+  const CoarsePlan& cp = plans[blockIdx.x];
+  const int n0 = cp.n0, n1 = cp.n1;
+  CoarseCells L0, L1;
+  {
+    const int32_t done = (flags & F_CHECK_DONE) ? c.ps[cp.prob].done : 0;
+    CoarseRaw R0, R1;
+    cl_issue<V>(c, cp, CL_ROOTS, n1, R1);
+    cl_issue<V>(c, cp, 0, n0, R0);
+    if (done) return;
+    if (tid < 4) M.z[CL_ZERO + tid] = 0.f;
+    cl_commit(cp, CL_ROOTS, n1, R1, M, L1);
+    cl_commit(cp, 0, n0, R0, M, L0);
   }
+#pragma unroll
+  for (int col = 0; col < 2; col++) cl_each<false>(L0, col, [&](int m, uint32_t at) { M.b0[at >> 2] = L0.P[col][m].b; });
   __syncthreads();
-  CellPrep P[2][CL_CPT];  // [colour][m]
-  // rows of this thread's cells of level l (cell m of colour col: q = tid + m * CL_THREADS)
-  auto prep = [&](int l) {
-    const int s0 = cp.lvl_begin[l], n = (cp.lvl_begin[l + 1] - s0) * 256;
+  constexpr uint32_t T0 = CL_ROOTS * 512;  // M.t starts at level 1's first cell
+  // one damped-Jacobi sweep of level 1
+  auto jacobi1 = [&]() {
 #pragma unroll
     for (int col = 0; col < 2; col++)
-#pragma unroll
-      for (int m = 0; m < CL_CPT; m++) {
-        const int q = tid + m * CL_THREADS;
-        P[col][m].own = -1;
-        if (q < n) {
-          const int s = s0 + (q >> 8), r = q & 255;
-          const int i = r >> 5, j = (r >> 2) & 7;
-          cl_prep(M, s, (i << 6) | (j << 3) | (2 * (r & 3) + ((col + i + j) & 1)), P[col][m]);
-        }
-      }
-  };
-  // one red-black colour pass of the prepared level
-  auto gs = [&](int col) {
-#pragma unroll
-    for (int m = 0; m < CL_CPT; m++) {
-      const CellPrep& Q = P[col][m];
-      if (Q.own >= 0) {
-        float x0;
-        const float ax = cl_ax(M, Q, x0);
-        float delta = 0.f;
-        if (Q.in && Q.dg != 0.f) delta = (Q.b - ax) / Q.dg;
-        M.z[Q.own] = vround<V>(x0 + delta);
-      }
-    }
-    __syncthreads();
-  };
-  // one damped-Jacobi sweep of the prepared level
-  auto jacobi = [&]() {
-    float out[2][CL_CPT];
-#pragma unroll
-    for (int col = 0; col < 2; col++)
-#pragma unroll
-      for (int m = 0; m < CL_CPT; m++) {
-        const CellPrep& Q = P[col][m];
-        out[col][m] = 0.f;
-        if (Q.own >= 0) {
-          float x0;
-          const float ax = cl_ax(M, Q, x0);
-          out[col][m] = x0;
-          if (Q.in) out[col][m] = (Q.dg == 0.f) ? 0.f : x0 + (v.omega * (Q.b - ax)) / Q.dg;
-        }
-      }
+      cl_each<true>(L1, col, [&](int m, uint32_t at) {
+        const CoarseCell& Q = L1.P[col][m];
+        const bool in = (L1.in >> (2 * m + col)) & 1;
+        const float x0 = cl_at(M, at);
+        const float res = cl_residual(M, Q, x0, in, L1.cf, L1.h);
+        M.t[(at >> 2) - T0] = in ? (Q.rd != 0.0 ? x0 + div_by(v.omega * res, Q.rd) : 0.f) : x0;
+      });
     __syncthreads();
 #pragma unroll
     for (int col = 0; col < 2; col++)
-#pragma unroll
-      for (int m = 0; m < CL_CPT; m++)
-        if (P[col][m].own >= 0) M.z[P[col][m].own] = vround<V>(out[col][m]);
+      cl_each<true>(L1, col, [&](int, uint32_t at) { cl_at(M, at) = vround<V>(M.t[(at >> 2) - T0]); });
     __syncthreads();
   };
-  auto smooth = [&](int order) {
-    for (int it = 0; it < v.nu; it++) {
-      if (v.smoother != 0) jacobi();
-      else { gs(order); gs(1 - order); }
-    }
-  };
-  for (int l = cp.C; l >= 1; l--) {
-    prep(l);
-    smooth(0);
-    // residuals of level l, then their 2x2x2 sums into the rhs of level l-1
-#pragma unroll
-    for (int col = 0; col < 2; col++)
-#pragma unroll
-      for (int m = 0; m < CL_CPT; m++) {
-        const CellPrep& Q = P[col][m];
-        if (Q.own >= 0) {
-          float x0;
-          const float ax = cl_ax(M, Q, x0);
-          (&M.t[0][0])[Q.own] = Q.b - ax;
-        }
-      }
-    __syncthreads();
-    const int s0 = cp.lvl_begin[l], ns = cp.lvl_begin[l + 1] - s0;
-    for (int q = tid; q < ns * 64; q += CL_THREADS) {
-      const int s = s0 + (q >> 6), lq = q & 63;
-      const float sum = octet_sum(M.t[s], lq);
-      const CoarseSlot& S = M.S[s];
-      const int a = lq >> 4, bq = (lq >> 2) & 3, cq = lq & 3;
-      const int ox = S.octant & 1, oy = (S.octant >> 1) & 1, oz = (S.octant >> 2) & 1;
-      M.b[S.parent][((ox * 4 + a) << 6) | ((oy * 4 + bq) << 3) | (oz * 4 + cq)] = vround<V>(sum * v.ooa);
-    }
-    __syncthreads();
-  }
-  prep(0);
   const int it0 = v.coarsest / 2;
-  for (int it = 0; it < it0; it++) { gs(0); gs(1); }
-  for (int it = 0; it < it0; it++) { gs(1); gs(0); }
-  for (int l = 1; l <= cp.C; l++) {
-    const int s0 = cp.lvl_begin[l], ns = cp.lvl_begin[l + 1] - s0;
-    for (int q = tid; q < ns * 512; q += CL_THREADS) {
-      const int s = s0 + (q >> 9), cc = q & 511;
-      const CoarseSlot& S = M.S[s];
-      const int i = cc >> 6, j = (cc >> 3) & 7, k = cc & 7;
+  if (n1) {
+    for (int it = 0; it < v.nu; it++) {
+      if (v.smoother != 0) jacobi1();
+      else { cl_gs<V, true>(M, L1, 0); cl_gs<V, true>(M, L1, 1); }
+    }
+    // residuals of level 1, then their 2x2x2 sums into the rhs of level 0, in the
+    // reference's (ii, jj, kk) order (GMGSolver.cu:319-328)
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<true>(L1, col, [&](int m, uint32_t at) {
+        M.t[(at >> 2) - T0] =
+            cl_residual(M, L1.P[col][m], cl_at(M, at), (L1.in >> (2 * m + col)) & 1, L1.cf, L1.h);
+      });
+    __syncthreads();
+    if (tid < CL_CHILDREN * 64) {
+      const int q = uni(tid >> 6), lq = tid & 63;
+      const CoarseSlot& S = cp.slots[CL_ROOTS + q];
+      const int a = lq >> 4, bq = (lq >> 2) & 3, cq = lq & 3;
+      float sum = 0.f;
+#pragma unroll
+      for (int o = 0; o < 8; o++)
+        sum += M.t[q * 512 + split_cell(2 * a + (o >> 2), 2 * bq + ((o >> 1) & 1), 2 * cq + (o & 1))];
       const int ox = S.octant & 1, oy = (S.octant >> 1) & 1, oz = (S.octant >> 2) & 1;
-      const float cz = M.z[S.parent * 512 + (((ox * 4 + (i >> 1)) << 6) | ((oy * 4 + (j >> 1)) << 3) | (oz * 4 + (k >> 1)))];
-      M.z[s * 512 + cc] = (M.ct[s][cc] & C_INT) ? vround<V>(__builtin_fmaf(v.pcoef, cz, M.z[s * 512 + cc])) : 0.f;
+      M.b0[S.parent * 512 + split_cell(ox * 4 + a, oy * 4 + bq, oz * 4 + cq)] = vround<V>(sum * v.ooa);
     }
     __syncthreads();
-    prep(l);
-    smooth(1);
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<false>(L0, col, [&](int m, uint32_t at) { L0.P[col][m].b = M.b0[at >> 2]; });
   }
-  for (int q = tid; q < cp.nslots * 128; q += CL_THREADS) {
-    const int s = q >> 7, o = (q & 127) * 4;
-    store_quad_split(Z + size_t(M.S[s].tile) * 512, o >> 3, o & 7, *reinterpret_cast<const float4*>(&M.z[s * 512 + o]));
+  for (int it = 0; it < it0; it++) { cl_gs<V, false>(M, L0, 0); cl_gs<V, false>(M, L0, 1); }
+  for (int it = 0; it < it0; it++) { cl_gs<V, false>(M, L0, 1); cl_gs<V, false>(M, L0, 0); }
+  const int q0 = uni(tid >> 8), r = tid & 255;
+  if (n1) {
+    // prolongation: x += pcoef * parent on INTERIOR cells, 0 elsewhere (the two
+    // cells of a pair k = 2 e, 2 e + 1 have one parent cell)
+    const int i = r >> 5, j = (r >> 2) & 7, e = r & 3;
+    cl_each<true>(L1, 0, [&](int m, uint32_t at) {
+      const CoarseSlot& S = cp.slots[CL_ROOTS + q0 + 4 * m];
+      const int pi = (S.octant & 1) * 4 + (i >> 1), pj = ((S.octant >> 1) & 1) * 4 + (j >> 1);
+      const float cz = M.z[S.parent * 512 + split_cell(pi, pj, ((S.octant >> 2) & 1) * 4 + e)];
+#pragma unroll
+      for (int col = 0; col < 2; col++) {
+        float& z = cl_at(M, at + col * CL_COL);
+        z = ((L1.in >> (2 * m + col)) & 1) ? vround<V>(__builtin_fmaf(v.pcoef, cz, z)) : 0.f;
+      }
+    });
+    __syncthreads();
+    for (int it = 0; it < v.nu; it++) {
+      if (v.smoother != 0) jacobi1();
+      else { cl_gs<V, true>(M, L1, 1); cl_gs<V, true>(M, L1, 0); }
+    }
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<true>(L1, col, [&](int m, uint32_t at) {
+        Z[size_t(cp.slots[CL_ROOTS + q0 + 4 * m].tile) * 512 + col * 256 + r] = from_f<V>(cl_at(M, at));
+      });
   }
+#pragma unroll
+  for (int col = 0; col < 2; col++)
+    cl_each<false>(L0, col, [&](int m, uint32_t at) {
+      Z[size_t(cp.slots[q0 + 4 * m].tile) * 512 + col * 256 + r] = from_f<V>(cl_at(M, at));
+    });
 }
 
 // Empty kernel, for measuring the launch floor.

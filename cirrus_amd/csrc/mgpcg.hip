@@ -87,7 +87,6 @@ struct cg_problem {
   std::vector<DList> act, lvl;   // per level, all problems (operator API)
   std::vector<DList> actg, lvlg; // per level, tiles the V-cycle smooths with grid-wide launches
   std::vector<CoarsePlan> plans; // LDS-resident coarse levels, one per problem with C >= 0
-  std::vector<CoarseSlot> coarse_slots;
   // schedule (no effect on results): XCD-aware tile order, LDS-resident coarse
   // levels given up to grid-wide launches, tiles per wavefront of the colour sweeps
   int swz = F_SWIZZLE;
@@ -134,7 +133,6 @@ struct cg_problem {
   TileRec* d_tmp_list = nullptr;
   int tmp_list_cap = 0;
   int32_t* d_ext = nullptr;      // internal tile -> caller index (channel moves from and to device buffers)
-  CoarseSlot* d_coarse = nullptr;
   hipStream_t stream = nullptr;
   int* h_pin = nullptr;
   ProbState* h_ps = nullptr;     // pinned staging of the ProbState uploads
@@ -188,7 +186,7 @@ cg_problem::~cg_problem() {
   if (h_ps) (void)hipHostFree(h_ps);
   if (ev_ps) (void)hipEventDestroy(ev_ps);
   void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_zh, d_rhsvh, d_zbh, d_x64, d_r64, d_bsave, d_psum, d_gsum, d_ps,
-                  d_dflag, d_plans, d_part, d_part2, d_scalar, d_lists, d_tiles, d_tmp_list, d_coarse, d_amgc, d_amgct, d_ext};
+                  d_dflag, d_plans, d_part, d_part2, d_scalar, d_lists, d_tiles, d_tmp_list, d_amgc, d_amgct, d_ext};
   for (void* q : ptrs) if (q) (void)hipFree(q);
   for (auto q : d_ch) if (q) (void)hipFree(q);
   for (auto q : d_api) if (q) (void)hipFree(q);
@@ -365,13 +363,10 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
   }
 }
 
-// Deepest level C of a tree kept in LDS by the coarse kernel: levels 0..C hold
-// at most CL_MAX_TILES tiles in total, at most CL_MAX_PER_LEVEL on any level,
-// and no GHOST tile (-1 if level 0 alone is larger).  (A GHOST tile needs a LEAF
-// tile one level up beside a NONLEAF one, i.e. at least 14 tiles on two levels,
-// so the size bound alone already excludes them; the check keeps the kernel's
-// assumption explicit.)  CIRRUS_COARSE_LEVELS=k caps it at k levels, for
-// measurement.
+// Deepest level C of a tree kept in LDS by the coarse kernel: level 0 of at most
+// CL_ROOTS tiles, level 1 when it is one root's CL_CHILDREN children, and no
+// GHOST tile on either (-1 if level 0 alone is larger).  CIRRUS_COARSE_LEVELS=k
+// caps it at k levels, for measurement.
 int coarse_depth(const std::vector<int>& lev, const std::vector<uint8_t>& ty) {
   int L = 0;
   for (int l : lev) L = std::max(L, l);
@@ -380,56 +375,50 @@ int coarse_depth(const std::vector<int>& lev, const std::vector<uint8_t>& ty) {
     cnt[lev[i]]++;
     if (ty[i] != GHOST) cnt_act[lev[i]]++;
   }
-  int C = -1, total = 0;
-  while (C + 1 <= L && C + 1 < CL_MAX_LEVELS && total + cnt[C + 1] <= CL_MAX_TILES && cnt[C + 1] <= CL_MAX_PER_LEVEL &&
-         cnt[C + 1] == cnt_act[C + 1]) {
+  int C = -1;
+  while (C + 1 <= L && C + 1 < CL_MAX_LEVELS && cnt[C + 1] <= (C + 1 == 0 ? CL_ROOTS : CL_CHILDREN) &&
+         cnt[C + 1] == cnt_act[C + 1])
     C++;
-    total += cnt[C];
-  }
   if (const char* e = std::getenv("CIRRUS_COARSE_LEVELS")) C = std::max(-1, std::min(C, std::atoi(e) - 1));
   return C;
 }
 
-// Coarse plan of tiles [first, first + count) of `tiles` (global indices start at
-// base): slots of levels 0..C in level order; `slots` is filled in by the caller.
-void coarse_plan(const std::vector<TileRec>& tiles, int base, int C, int prob, CoarsePlan& cp, std::vector<CoarseSlot>& out) {
+// Coarse plan of levels 0..C of a tree's n tiles (in level order; their global
+// indices start at base).
+CoarsePlan coarse_plan(const TileRec* tiles, int n, int base, int C, int prob) {
+  CoarsePlan cp;
   std::memset(&cp, 0, sizeof(cp));
   cp.prob = prob;
-  cp.C = C;
-  const int n = int(tiles.size());
   std::unordered_map<int, int> slot_of;
-  const int first = int(out.size());
-  for (int l = 0; l <= C; l++) {
-    cp.lvl_begin[l] = int(out.size()) - first;
-    for (int i = 0; i < n; i++) {
-      if (tr_level(tiles[i]) != l) continue;
-      slot_of[base + i] = int(out.size()) - first;
-      CoarseSlot cs;
-      std::memset(&cs, 0, sizeof(cs));
-      cs.tile = base + i;
-      out.push_back(cs);
-    }
+  for (int i = 0; i < n; i++) {
+    const int l = tr_level(tiles[i]);
+    if (l > C) break;
+    int& k = l == 0 ? cp.n0 : cp.n1;
+    if (k >= (l == 0 ? CL_ROOTS : CL_CHILDREN)) fail(CG_ERR_INVALID, "coarse plan: too many slots");
+    const int s = (l == 0 ? 0 : CL_ROOTS) + k++;
+    slot_of[base + i] = s;
+    cp.slots[s].tile = base + i;
   }
-  cp.lvl_begin[C + 1] = int(out.size()) - first;
-  cp.nslots = cp.lvl_begin[C + 1];
-  for (int s = first; s < int(out.size()); s++) {
-    CoarseSlot& cs = out[s];
-    const TileRec& T = tiles[cs.tile - base];
+  // the kernel works level 1 as CL_CHILDREN tiles with one face coefficient per level
+  if (cp.n0 < 1 || (cp.n1 != 0 && cp.n1 != CL_CHILDREN)) fail(CG_ERR_INVALID, "coarse plan: incomplete level");
+  for (const auto& kv : slot_of) {
+    CoarseSlot& cs = cp.slots[kv.second];
+    const TileRec& T = tiles[kv.first - base];
     for (int f = 0; f < 6; f++) cs.nbr[f] = T.nbr[f] < 0 ? -1 : slot_of.at(T.nbr[f]);
     cs.parent = T.parent < 0 ? -1 : slot_of.at(T.parent);
-    cs.level = tr_level(T);
+    cs.octant = tr_octant(T);
     cs.h = T.h;
-    cs.type = tr_type(T);
-    cs.octant = uint8_t(tr_octant(T));
-    for (int f = 0; f < 7; f++) cs.bc[f] = T.bc[f];
+    cs.bc = T.bc[6];
+    for (int f = 0; f < 6; f++)
+      if (T.bc[f] != cs.bc) fail(CG_ERR_INVALID, "coarse plan: face coefficients differ");
   }
+  return cp;
 }
 
 // Worklists and coarse plans of a pool for its schedule (host side only):
 // each problem keeps its deepest LDS-resident coarse level coarse_auto -
 // coarse_shift (-1: none), the levels above it go to grid-wide launches.  The
-// lists' tile indices come back in `ids` (every list's DList indexes it); the
-// coarse plans hold slot offsets until upload_schedule patches them.
+// lists' tile indices come back in `ids` (every list's DList indexes it).
 void plan_schedule(cg_problem& P, std::vector<int32_t>& ids) {
   const int n = P.n, nprob = P.nprob;
   const std::vector<int>& lev = P.lev;
@@ -479,28 +468,10 @@ void plan_schedule(cg_problem& P, std::vector<int32_t>& ids) {
     ids.insert(ids.end(), s.second.begin(), s.second.end());
   }
 
-  // coarse plans and slots
   P.plans.clear();
-  P.coarse_slots.clear();
   for (int q = 0; q < nprob; q++) {
     if (P.coarse_C[q] < 0) continue;
-    CoarsePlan cp;
-    const int first = int(P.coarse_slots.size());
-    std::vector<TileRec> mine(P.tiles.begin() + tbase[q], P.tiles.begin() + tbase[q + 1]);
-    coarse_plan(mine, tbase[q], P.coarse_C[q], q, cp, P.coarse_slots);
-    cp.slots = reinterpret_cast<const CoarseSlot*>(size_t(first));  // offset, patched after upload
-    P.plans.push_back(cp);
-  }
-  for (const CoarsePlan& cp : P.plans) {  // every slot link stays inside its own plan (the kernel's LDS)
-    const size_t first = size_t(cp.slots);
-    if (cp.nslots > CL_MAX_TILES || first + size_t(cp.nslots) > P.coarse_slots.size())
-      fail(CG_ERR_INVALID, "coarse plan: too many slots");
-    for (int k = 0; k < cp.nslots; k++) {
-      const CoarseSlot& cs = P.coarse_slots[first + k];
-      for (int f = 0; f < 6; f++)
-        if (cs.nbr[f] >= cp.nslots) fail(CG_ERR_INVALID, "coarse plan: neighbour slot out of range");
-      if (cs.parent >= cp.nslots || cs.tile < 0 || cs.tile >= P.n) fail(CG_ERR_INVALID, "coarse plan: slot out of range");
-    }
+    P.plans.push_back(coarse_plan(&P.tiles[tbase[q]], tbase[q + 1] - tbase[q], tbase[q], P.coarse_C[q], q));
   }
   for (int32_t t : ids)
     if (t < 0 || t >= P.n) fail(CG_ERR_INVALID, "worklist: tile index out of range");
@@ -512,10 +483,8 @@ void upload_schedule(cg_problem& P, const std::vector<int32_t>& ids) {
   const size_t total = ids.size();
   HIPC(hipStreamSynchronize(P.stream));  // no kernel may still read the old lists
   if (P.d_lists) HIPC(hipFree(P.d_lists));
-  if (P.d_coarse) HIPC(hipFree(P.d_coarse));
   if (P.d_plans) HIPC(hipFree(P.d_plans));
   P.d_lists = nullptr;
-  P.d_coarse = nullptr;
   P.d_plans = nullptr;
   HIPC(hipMalloc(&P.d_lists, sizeof(TileRec) * std::max<size_t>(1, total)));
   if (total) {
@@ -528,10 +497,6 @@ void upload_schedule(cg_problem& P, const std::vector<int32_t>& ids) {
     HIPC(hipStreamSynchronize(P.stream));  // d_ids is freed at the end of this scope
   }
   if (!P.plans.empty()) {
-    HIPC(hipMalloc(&P.d_coarse, sizeof(CoarseSlot) * P.coarse_slots.size()));
-    HIPC(hipMemcpyAsync(P.d_coarse, P.coarse_slots.data(), sizeof(CoarseSlot) * P.coarse_slots.size(),
-                        hipMemcpyHostToDevice, P.stream));
-    for (auto& cp : P.plans) cp.slots = P.d_coarse + size_t(cp.slots);
     HIPC(hipMalloc(&P.d_plans, sizeof(CoarsePlan) * P.plans.size()));
     HIPC(hipMemcpyAsync(P.d_plans, P.plans.data(), sizeof(CoarsePlan) * P.plans.size(), hipMemcpyHostToDevice, P.stream));
   }
@@ -830,6 +795,11 @@ void launch_gs_pair(cg_problem& P, const DList& a, const Ctx& c, const V* XI, co
       c);
   else k_gs_pair<V, false><<<grid_for(a.n, flags), 64, 0, P.stream>>>(P.L(a), a.n, flags, XI, XG, XO, c1, c);
 }
+// The LDS-resident coarse levels of every problem that has some.
+template <class V>
+void launch_coarse(cg_problem& P, const Ctx& c, const VCycleArgs& va, V* Z, int flags) {
+  if (!P.plans.empty()) k_coarse_lds<V><<<unsigned(P.plans.size()), CL_THREADS, 0, P.stream>>>(P.d_plans, flags, Z, va, c);
+}
 // The pool's V-cycle vectors of storage type V.
 template <class V> V* pool_z(cg_problem& P);
 template <class V> V* pool_zb(cg_problem& P);
@@ -931,10 +901,7 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
     else if (al.n)
       k_restrict<V, true><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
   }
-  if (!P.plans.empty()) {
-    VCycleArgs va{v.nu, v.coarsest, v.smoother, v.omega, v.ooa, v.pcoef};
-    k_coarse_lds<V><<<unsigned(P.plans.size()), CL_THREADS, 0, P.stream>>>(c, P.d_plans, va, ZO, base & ~F_SWIZZLE);
-  }
+  launch_coarse<V>(P, c, VCycleArgs{v.nu, v.coarsest, v.smoother, v.omega, v.ooa, v.pcoef}, ZO, base & ~F_SWIZZLE);
   {
     // problems whose level 0 is too large for LDS: bottom sweeps as grid-wide launches
     const DList& a0 = P.actg[0];
@@ -1417,7 +1384,7 @@ void solve_refined(cg_problem& P, const cg_params& prm, const cg_refine_params& 
 // Autotuner: schedules timed on the pool's own right-hand sides
 // ---------------------------------------------------------------------------
 void set_schedule(cg_problem& P, int coarse_shift, int swizzle, int tile_block) {
-  if (coarse_shift < 0 || coarse_shift > CL_MAX_LEVELS) fail(CG_ERR_INVALID, "cg_set_schedule: coarse_shift out of range");
+  if (coarse_shift < 0 || coarse_shift > 8) fail(CG_ERR_INVALID, "cg_set_schedule: coarse_shift out of range");
   if (tile_block != 1 && tile_block != 2 && tile_block != 4 && tile_block != 8)
     fail(CG_ERR_INVALID, "cg_set_schedule: tile_block must be 1, 2, 4 or 8");
   if (!P.owner) fail(CG_ERR_INVALID, "cg_set_schedule: not an owning handle");
@@ -2387,10 +2354,10 @@ cg_status cg_benchmark_kernel(cg_problem* p, int32_t kernel, int32_t level, int3
           k_cg_update_xr<float><<<grid_for(P.leaf.n, base), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, base, c);
           break;
         case CG_KERNEL_COARSE: {
-          nt = int64_t(P.coarse_slots.size());
+          nt = 0;
+          for (const CoarsePlan& cp : P.plans) nt += cp.n0 + cp.n1;
           VCycleArgs va{2, level, 0, 2.f / 3.f, 1.f, 1.f};  // `level` = bottom iterations
-          if (!P.plans.empty())
-            k_coarse_lds<float><<<unsigned(P.plans.size()), CL_THREADS, 0, P.stream>>>(c, P.d_plans, va, c.z, base & ~F_SWIZZLE);
+          launch_coarse<float>(P, c, va, c.z, base & ~F_SWIZZLE);
           break;
         }
         case CG_KERNEL_COPY:

@@ -23,7 +23,7 @@
 // for all the requests that start, finish or pass in that step, over worklists
 // assembled like the active set's.  A release hands the instance's memory back
 // once the stream has passed it (an event), so it neither waits for the device
-// nor frees device memory: records and coarse slots live in server-wide arenas
+// nor frees device memory: records live in a server-wide arena
 // and pinned staging buffers are kept for later admissions.
 #pragma once
 
@@ -49,7 +49,6 @@ struct Instance {
   int rec_count = 0;
   DList leaf, gather, applyl, ghosts, all;
   std::vector<DList> actg, lvlg;
-  CoarseSlot* d_slots = nullptr;  // the slot's part of the server's coarse-slot arena
   CoarsePlan plan;
   float* h_buf = nullptr;  // pinned: rhs on the way in, pressure on the way out
   size_t h_bytes = 0;      // its capacity (a kept buffer may be larger than the instance needs)
@@ -103,7 +102,7 @@ struct cg_server {
   std::vector<Released> pending;  // releases the stream has not yet passed
   std::vector<hipEvent_t> ev_free;
   std::multimap<size_t, float*> hbuf_cache;  // pinned staging buffers of released instances, by size
-  // pinned ring for admission uploads (records, coarse slots, cell types),
+  // pinned ring for admission uploads (records, cell types),
   // copied on the stream; a segment is reused once its event has passed
   char* h_ring = nullptr;
   size_t ring_cap = 0, ring_head = 0;
@@ -151,7 +150,6 @@ struct cg_server {
   TileRec* d_asm = nullptr;
   int64_t asm_cap = 0;
   TileRec* d_recs = nullptr;  // arena of the instances' own records
-  CoarseSlot* d_cslots = nullptr;  // arena of the instances' coarse slots (CL_MAX_TILES per slot)
   TileRec* d_gasm = nullptr;  // group worklists
   int64_t gasm_cap = 0;
   // group tables (runs, map, staged problem states): pinned, per step parity and
@@ -198,7 +196,7 @@ cg_server::~cg_server() {
     for (auto e : row) if (e) (void)hipEventDestroy(e);
   if (h_ver) (void)hipHostFree(h_ver);
   void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_b, d_x64, d_r64, d_ver, d_zh, d_rhsvh, d_zbh, d_gsum, d_ps, d_dflag,
-                  d_dflag_init, d_pmap, d_part, d_part2, d_asm, d_recs, d_cslots, d_gasm, d_gtab, d_plans,
+                  d_dflag_init, d_pmap, d_part, d_part2, d_asm, d_recs, d_gasm, d_gtab, d_plans,
                   (void*)d_srcs, d_offs, d_counts};
   for (void* q : ptrs) if (q) (void)hipFree(q);
   for (auto q : d_ch) if (q) (void)hipFree(q);
@@ -292,7 +290,6 @@ void server_create(const cg_server_config* cfg, cg_server& S) {
   S.asm_cap = S.cap_tiles * kRecKindsPerTile;
   HIPC(hipMalloc(&S.d_asm, sizeof(TileRec) * S.asm_cap));
   HIPC(hipMalloc(&S.d_recs, sizeof(TileRec) * S.cap_tiles * kOwnRecsPerTile));
-  HIPC(hipMalloc(&S.d_cslots, sizeof(CoarseSlot) * CL_MAX_TILES * S.nslots));
   S.gasm_cap = S.cap_tiles * kGroupRecsPerTile;
   HIPC(hipMalloc(&S.d_gasm, sizeof(TileRec) * S.gasm_cap));
   {
@@ -384,7 +381,7 @@ int64_t alloc_range(cg_server& S, RangeAlloc& A, int64_t n) {
 }
 
 void admit_upload(cg_server& S, const cg_tree_desc* d, const TreeBuild& B, const std::vector<TileRec>& W,
-                  const std::vector<CoarseSlot>& cslots, Instance& inst, int slot, int64_t tb, int64_t rb);
+                  Instance& inst, int slot, int64_t tb, int64_t rb);
 
 void server_admit(cg_server& S, const cg_tree_desc* d, int32_t* out) {
   if (!d || !out) fail(CG_ERR_INVALID, "cg_server_admit: null argument");
@@ -455,9 +452,7 @@ void server_admit(cg_server& S, const cg_tree_desc* d, int32_t* out) {
     I->actg[l] = add_list([&](int i) { return B.lev[i] == l && B.ty[i] != GHOST && grid_level(i); });
     I->lvlg[l] = add_list([&](int i) { return B.lev[i] == l && grid_level(i); });
   }
-  std::vector<CoarseSlot> cslots;
-  if (I->C >= 0) coarse_plan(B.tiles, int(tb), I->C, slot, I->plan, cslots);
-  const bool fits = W.size() <= size_t(n) * kOwnRecsPerTile && cslots.size() <= size_t(CL_MAX_TILES);
+  const bool fits = W.size() <= size_t(n) * kOwnRecsPerTile;
   const int64_t rb = fits ? alloc_range(S, S.rec_alloc, int64_t(W.size())) : -2;
   auto undo = [&] {
     S.tiles_alloc.release(tb, n);
@@ -468,11 +463,12 @@ void server_admit(cg_server& S, const cg_tree_desc* d, int32_t* out) {
   };
   if (rb < 0) {
     undo();
-    if (rb == -2) fail(CG_ERR_INVALID, "cg_server_admit: more records or coarse slots than the tree allows");
+    if (rb == -2) fail(CG_ERR_INVALID, "cg_server_admit: more records than the tree allows");
     fail(CG_ERR_BUSY, "cg_server_admit: HBM budget exhausted");
   }
   try {
-    admit_upload(S, d, B, W, cslots, *I, slot, tb, rb);
+    if (I->C >= 0) I->plan = coarse_plan(B.tiles.data(), n, int(tb), I->C, slot);
+    admit_upload(S, d, B, W, *I, slot, tb, rb);
   } catch (...) {
     undo();
     if (I->h_buf) (void)hipHostFree(I->h_buf);
@@ -514,11 +510,11 @@ void ring_release_after_copies(cg_server& S, const char* p, size_t bytes) {
   S.ring_busy.push_back(g);
 }
 
-// The admitted instance's records, coarse slots and cell types to the device,
+// The admitted instance's records and cell types to the device,
 // its face masks, diagonal and zeroed vectors (on the server's stream), its
 // staging buffer and events.
 void admit_upload(cg_server& S, const cg_tree_desc* d, const TreeBuild& B, const std::vector<TileRec>& W,
-                  const std::vector<CoarseSlot>& cslots, Instance& inst, int slot, int64_t tb, int64_t rb) {
+                  Instance& inst, int slot, int64_t tb, int64_t rb) {
   Instance* I = &inst;
   const int n = d->num_tiles;
   // the instance's pinned staging buffer (right-hand sides in, pressures out)
@@ -535,30 +531,23 @@ void admit_upload(cg_server& S, const cg_tree_desc* d, const TreeBuild& B, const
   I->rec_begin = rb;
   I->rec_count = int(W.size());
   I->d_recs = S.d_recs + rb;
-  // records, coarse slots and cell types through the admission ring, copied on
+  // records and cell types through the admission ring, copied on
   // the stream (the host does not wait for a device that is busy with other
   // requests); a tree too large for the ring goes through its own staging
   // buffer with synchronous copies
   const size_t rec_bytes = sizeof(TileRec) * W.size(), ct_bytes = size_t(n) * 512;
-  const size_t slot_bytes = sizeof(CoarseSlot) * cslots.size();
-  const size_t o_ct = (rec_bytes + 255) & ~size_t(255), o_sl = o_ct + ((ct_bytes + 255) & ~size_t(255));
-  const size_t total = o_sl + slot_bytes;
+  const size_t o_ct = (rec_bytes + 255) & ~size_t(255);
+  const size_t total = o_ct + ct_bytes;
   char* ring = ring_take(S, total);
   char* stage = ring ? ring : reinterpret_cast<char*>(I->h_buf);
   if (!ring && total > I->h_bytes) fail(CG_ERR_INVALID, "cg_server_admit: staging buffer too small");
   std::memcpy(stage, W.data(), rec_bytes);
   for (int i = 0; i < n; i++) std::memcpy(stage + o_ct + size_t(i) * 512, d->cell_type + size_t(B.ext[i]) * 512, 512);
-  if (slot_bytes) std::memcpy(stage + o_sl, cslots.data(), slot_bytes);
   auto up = [&](void* dst, size_t off, size_t bytes) {
     if (ring) HIPC(hipMemcpyAsync(dst, stage + off, bytes, hipMemcpyHostToDevice, S.stream));
     else HIPC(hipMemcpy(dst, stage + off, bytes, hipMemcpyHostToDevice));
   };
   up(I->d_recs, 0, rec_bytes);
-  if (I->C >= 0) {
-    I->d_slots = S.d_cslots + size_t(slot) * CL_MAX_TILES;
-    up(I->d_slots, o_sl, slot_bytes);
-    I->plan.slots = I->d_slots;
-  }
   // cell types in internal order; x = 0 so that a first warm start is a cold one
   up(S.d_ctype + size_t(tb) * 512, o_ct, ct_bytes);
   if (ring) ring_release_after_copies(S, ring, total);
