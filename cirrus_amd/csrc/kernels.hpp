@@ -1871,9 +1871,12 @@ struct CoarseLDS {
 // 2^-126, where FP32 has fewer bits, within one unit of their last place).
 // 4 issue slots against 15.5 for the FP32 division on gfx950.
 __device__ __forceinline__ float div_by(float a, double rd) { return float(double(a) * rd); }
-// 1/d in FP64 for d > 0: the FP32 reciprocal and two Newton steps.
+// 1/d in FP64 for finite d != 0: the FP32 reciprocal and two Newton steps (a
+// divisor beyond the range where that reciprocal is a normal number: the division).
 __device__ __forceinline__ double recip64(float d) {
   const double dd = double(d);
+  const float a = __builtin_fabsf(d);
+  if (!(a >= 0x1p-100f && a <= 0x1p100f)) return 1.0 / dd;
   double y = double(__builtin_amdgcn_rcpf(d));
   y = __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
   return __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
@@ -1910,7 +1913,7 @@ __device__ __forceinline__ void cl_prep(const CoarseSlot& S, int s, int col, int
   for (int f = 0; f < 6; f++) nb[f] = 4 * (((m >> f) & 1) ? nb[f] : own);
 #pragma unroll
   for (int f = 0; f < 3; f++) P.nb[f] = uint32_t(nb[2 * f]) | (uint32_t(nb[2 * f + 1]) << 16);
-  P.rd = d > 0.f ? recip64(d) : 0.0;  // D is 0 off INTERIOR cells
+  P.rd = d != 0.f ? recip64(d) : 0.0;  // D is 0 off INTERIOR cells
 }
 // b - A x of a prepared cell with value x0 (cell_row_m's operations; a cut face
 // adds c * 0).
@@ -3095,6 +3098,178 @@ __global__ __launch_bounds__(64) void k_amg_prolong(const TileRec* __restrict__ 
     x[k] = in ? (ghost ? cx : __builtin_fmaf(pcoef, cx, x[k])) : 0.f;
   }
   store8(X + b, x);
+}
+
+// ---------------------------------------------------------------------------
+// The coarse levels 0..C (C <= 1) of VCycleAMG for one problem in one workgroup,
+// on the plan of k_coarse_lds and in its LDS layout: the sweeps, residual,
+// restriction and prolongation of the kernels above, cell by cell in their
+// order (AMGSolver.cu:540-715).  The rows are the stored coefficients: own entry
+// across a minus face, the plus neighbour's entry across a plus face (0 without
+// a neighbour), the diagonal.  With nine tiles, two sweeps and ten bottom
+// iterations it takes the place of 32 launches of 2-4 us, each bound by launch
+// and memory latency (the AMG solve on the 128^3 coarse/fine plane 8.2 -> 6.5 ms).
+// ---------------------------------------------------------------------------
+struct AmgCell {
+  uint32_t nb[3];  // LDS byte addresses of the six neighbours' x (CL_ZERO: none)
+  float cf[6];     // entries across x-, x+, y-, y+, z-, z+
+  float dg, b;
+  double rd;       // 1 / dg (0: not updated)
+};
+struct AmgCells {
+  AmgCell P[2][CL_CPT];  // as CoarseCells
+  uint32_t in, in1;      // bit 2 * m + colour: type has the INTERIOR bit; type is INTERIOR
+  uint32_t own;
+  int n;
+};
+// natural index of cell r (pencil * 4 + k / 2) of colour col
+__device__ __forceinline__ int cl_natural(int col, int r) {
+  return ((r >> 2) << 3) + 2 * (r & 3) + ((col + (r >> 5) + (r >> 2)) & 1);
+}
+__device__ __forceinline__ void amg_cells(const CoarsePlan& cp, int first, int n, const AmgC& A,
+                                          const float* __restrict__ RHS, AmgCells& L) {
+  const int q0 = uni(int(threadIdx.x) >> 8), r = threadIdx.x & 255;
+  const int i = r >> 5, j = (r >> 2) & 7;
+  L.own = uint32_t(4 * ((first + q0) * 512 + r));
+  L.n = n > q0 ? (n - q0 + 3) >> 2 : 0;
+  L.in = L.in1 = 0;
+#pragma unroll
+  for (int m = 0; m < CL_CPT; m++)
+    if (m < L.n) {
+      const int s = first + q0 + 4 * m;
+      const CoarseSlot& S = cp.slots[s];
+      const size_t tb = size_t(S.tile) * 512;
+#pragma unroll
+      for (int col = 0; col < 2; col++) {
+        AmgCell& P = L.P[col][m];
+        const int cc = cl_natural(col, r), k = cc & 7;
+        const bool inside[6] = {i > 0, i < 7, j > 0, j < 7, k > 0, k < 7};
+        const int step[6] = {-64, 64, -8, 8, -1, 1};
+        const int face[6] = {0, 3, 1, 4, 2, 5};
+        uint32_t at[6];
+#pragma unroll
+        for (int e = 0; e < 6; e++) {
+          const int q = inside[e] ? s : S.nbr[face[e]];
+          const int nc = inside[e] ? cc + step[e] : cc - 7 * step[e];
+          at[e] = 4u * uint32_t(q < 0 ? CL_ZERO : q * 512 + split_index(nc));
+          if ((e & 1) == 0) P.cf[e] = A.off[e >> 1][tb + cc];
+          else P.cf[e] = q < 0 ? 0.f : A.off[e >> 1][size_t(cp.slots[q].tile) * 512 + nc];
+        }
+#pragma unroll
+        for (int e = 0; e < 3; e++) P.nb[e] = at[2 * e] | (at[2 * e + 1] << 16);
+        P.dg = A.diag[tb + cc];
+        P.b = RHS[tb + cc];
+        const uint8_t ct = A.ct[tb + cc];
+        L.in |= uint32_t((ct & C_INT) != 0) << (2 * m + col);
+        L.in1 |= uint32_t(ct == C_INT) << (2 * m + col);
+        P.rd = ((ct & C_INT) && P.dg != 0.f) ? recip64(P.dg) : 0.0;
+      }
+    }
+}
+// rhs - A x of a cell with value x0 (amg_rows' order)
+__device__ __forceinline__ float amg_cell_residual(CoarseLDS& M, const AmgCell& P, float x0) {
+  float xn[6];
+#pragma unroll
+  for (int f = 0; f < 3; f++) {
+    xn[2 * f] = cl_at(M, P.nb[f] & 0xffffu);
+    xn[2 * f + 1] = cl_at(M, P.nb[f] >> 16);
+  }
+  float sum = x0 * P.dg;
+#pragma unroll
+  for (int f = 0; f < 6; f++) sum = __builtin_fmaf(P.cf[f], xn[f], sum);
+  return P.b - sum;
+}
+template <class F>
+__device__ __forceinline__ void amg_each(const AmgCells& L, int col, F f) {
+#pragma unroll
+  for (int m = 0; m < CL_CPT; m++)
+    if (m < L.n) f(m, L.own + m * CL_M + col * CL_COL);
+}
+__device__ __forceinline__ void amg_cl_gs(CoarseLDS& M, const AmgCells& L, int col) {
+  amg_each(L, col, [&](int m, uint32_t at) {
+    const AmgCell& Q = L.P[col][m];
+    const float x0 = cl_at(M, at);
+    const float res = amg_cell_residual(M, Q, x0);
+    cl_at(M, at) = x0 + (Q.rd != 0.0 ? div_by(res, Q.rd) : 0.f);
+  });
+  __syncthreads();
+}
+__global__ __launch_bounds__(CL_THREADS) void k_amg_coarse(const CoarsePlan* __restrict__ plans, int flags,
+                                                           float* __restrict__ X, const float* __restrict__ RHS, int nu,
+                                                           int coarsest, float alpha, float pcoef, AmgC A, Ctx c) {
+  __shared__ CoarseLDS M;
+  const int tid = threadIdx.x;
+  const CoarsePlan& cp = plans[blockIdx.x];
+  const int n0 = cp.n0, n1 = cp.n1;
+  if ((flags & F_CHECK_DONE) && c.ps[cp.prob].done) return;
+  for (int q = tid; q < CL_ZERO + 4; q += CL_THREADS) M.z[q] = 0.f;
+  AmgCells L;
+  const int q0 = uni(tid >> 8), r = tid & 255;
+  constexpr uint32_t T0 = CL_ROOTS * 512;
+  if (n1) {
+    amg_cells(cp, CL_ROOTS, n1, A, RHS, L);
+    __syncthreads();
+    for (int it = 0; it < nu; it++) { amg_cl_gs(M, L, 0); amg_cl_gs(M, L, 1); }
+    // residuals on INTERIOR cells (0 elsewhere), then their sums (x fastest)
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      amg_each(L, col, [&](int m, uint32_t at) {
+        const float res = amg_cell_residual(M, L.P[col][m], cl_at(M, at));
+        M.t[(at >> 2) - T0] = ((L.in1 >> (2 * m + col)) & 1) ? res : 0.f;
+      });
+    __syncthreads();
+    if (tid < CL_CHILDREN * 64) {
+      const int q = uni(tid >> 6), lq = tid & 63;
+      const CoarseSlot& S = cp.slots[CL_ROOTS + q];
+      const int a = lq >> 4, bq = (lq >> 2) & 3, cq = lq & 3;
+      float sum = 0.f;
+#pragma unroll
+      for (int o = 0; o < 8; o++)  // a cell that is not INTERIOR holds 0 in t
+        sum = sum + M.t[q * 512 + split_cell(2 * a + (o & 1), 2 * bq + ((o >> 1) & 1), 2 * cq + (o >> 2))];
+      M.b0[S.parent * 512 + split_cell((S.octant & 1) * 4 + a, ((S.octant >> 1) & 1) * 4 + bq,
+                                       ((S.octant >> 2) & 1) * 4 + cq)] = sum * alpha;
+    }
+    __syncthreads();
+  }
+  amg_cells(cp, 0, n0, A, RHS, L);
+  if (n1) {
+    // a root with children takes the restricted rhs (a LEAF root keeps its own)
+    const int refined = cp.slots[CL_ROOTS].parent;
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      amg_each(L, col, [&](int m, uint32_t at) {
+        if (q0 + 4 * m == refined) L.P[col][m].b = M.b0[at >> 2];
+      });
+  }
+  __syncthreads();
+  for (int it = 0; it < coarsest / 2; it++) { amg_cl_gs(M, L, 0); amg_cl_gs(M, L, 1); }
+  for (int it = 0; it < coarsest / 2; it++) { amg_cl_gs(M, L, 1); amg_cl_gs(M, L, 0); }
+  auto store = [&](int first) {
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      amg_each(L, col, [&](int m, uint32_t at) {
+        X[size_t(cp.slots[first + q0 + 4 * m].tile) * 512 + cl_natural(col, r)] = cl_at(M, at);
+      });
+  };
+  store(0);
+  if (n1) {
+    // the level's rows again (kept over the bottom solve they would not fit the registers)
+    amg_cells(cp, CL_ROOTS, n1, A, RHS, L);
+    const int i = r >> 5, j = (r >> 2) & 7, e = r & 3;
+    amg_each(L, 0, [&](int m, uint32_t at) {
+      const CoarseSlot& S = cp.slots[CL_ROOTS + q0 + 4 * m];
+      const int pi = (S.octant & 1) * 4 + (i >> 1), pj = ((S.octant >> 1) & 1) * 4 + (j >> 1);
+      const float cz = M.z[S.parent * 512 + split_cell(pi, pj, ((S.octant >> 2) & 1) * 4 + e)];
+#pragma unroll
+      for (int col = 0; col < 2; col++) {
+        float& z = cl_at(M, at + col * CL_COL);
+        z = ((L.in >> (2 * m + col)) & 1) ? __builtin_fmaf(pcoef, cz, z) : 0.f;
+      }
+    });
+    __syncthreads();
+    for (int it = 0; it < nu; it++) { amg_cl_gs(M, L, 1); amg_cl_gs(M, L, 0); }
+    store(CL_ROOTS);
+  }
 }
 
 // Fill whole tiles of a list with a value.

@@ -1012,26 +1012,30 @@ void enqueue_amg_vcycle(cg_problem& P, const VParams& v) {
   float* TMP = P.d_ch[CG_CH_AP];
   const float* F = c.r;
   k_amg_init<<<grid_for(P.all.n, fl), 64, 0, P.stream>>>(P.L(P.all), P.all.n, X, F, RHS, fl);
+  // levels above a problem's LDS-resident ones, grid-wide (actg / lvlg)
   auto gs = [&](int l, int color) {
-    if (P.act[l].n) k_amg_gs<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(P.L(P.act[l]), P.act[l].n, fl, X, RHS, A,
-        color, c);
+    const DList& a = P.actg[l];
+    if (a.n) k_amg_gs<<<grid_for(a.n, fl), 64, 0, P.stream>>>(P.L(a), a.n, fl, X, RHS, A, color, c);
   };
   const int L = P.max_level;
   for (int l = L; l >= 1; l--) {
+    const DList& a = P.actg[l];
+    const DList& al = P.lvlg[l];
+    if (!al.n) continue;
     for (int it = 0; it < v.nu; it++) { gs(l, 0); gs(l, 1); }
-    if (P.lvl[l].n)
-      k_amg_residual<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l]), P.lvl[l].n, fl, X, RHS, TMP, A, c);
-    if (P.act[l].n)
-      k_amg_restrict<<<grid_for(P.act[l].n, fl), 64, 0, P.stream>>>(P.L(P.act[l]), P.act[l].n, fl, TMP, RHS, A, v.ooa, c);
-    if (P.lvl[l - 1].n)
-      k_amg_leaf_rhs<<<grid_for(P.lvl[l - 1].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l - 1]), P.lvl[l - 1].n, fl, TMP, F,
-          RHS, c);
+    k_amg_residual<<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, X, RHS, TMP, A, c);
+    if (a.n) k_amg_restrict<<<grid_for(a.n, fl), 64, 0, P.stream>>>(P.L(a), a.n, fl, TMP, RHS, A, v.ooa, c);
+    const DList& below = P.lvl[l - 1];  // LDS-resident ones too: their LEAF tiles may have ghost children
+    if (below.n) k_amg_leaf_rhs<<<grid_for(below.n, fl), 64, 0, P.stream>>>(P.L(below), below.n, fl, TMP, F, RHS, c);
   }
+  if (!P.plans.empty())
+    k_amg_coarse<<<unsigned(P.plans.size()), CL_THREADS, 0, P.stream>>>(P.d_plans, fl, X, RHS, v.nu, v.coarsest, v.ooa,
+                                                                        v.pcoef, A, c);
   for (int it = 0; it < v.coarsest / 2; it++) { gs(0, 0); gs(0, 1); }
   for (int it = 0; it < v.coarsest / 2; it++) { gs(0, 1); gs(0, 0); }
   for (int l = 1; l <= L; l++) {
-    if (P.lvl[l].n) k_amg_prolong<<<grid_for(P.lvl[l].n, fl), 64, 0, P.stream>>>(P.L(P.lvl[l]), P.lvl[l].n, fl, X, A,
-        v.pcoef, c);
+    const DList& al = P.lvlg[l];
+    if (al.n) k_amg_prolong<<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, X, A, v.pcoef, c);
     for (int it = 0; it < v.nu; it++) { gs(l, 1); gs(l, 0); }
   }
   k_to_split<<<unsigned(P.leaf.n), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, X, c.z);

@@ -2,8 +2,8 @@
 they can go wrong: one to eight root tiles alone (level 0 in LDS), nine (too
 many: grid-wide launches), one root with its eight children (both levels in
 LDS), two roots (level 1 grid-wide), boxes of every axis order, both smoothers,
-every storage type -- each V-cycle solve equal to the oracle's bit for bit; and
-the arithmetic by which these kernels divide."""
+every storage type, the stored-coefficient preconditioner -- each solve equal to the
+oracle's bit for bit; and the arithmetic by which these kernels divide."""
 import numpy as np
 import pytest
 
@@ -32,6 +32,27 @@ def test_coarse_levels_give_the_oracle_solve(nroot, level, smoother, storage):
         # without bottom iterations a single level's z is 0 and both solves are NaN
         same = [S.last["iters"], S.last["rr"]], [ro["iters"], ro["rr"]]
         assert np.array_equal(*same, equal_nan=True), (coarsest, nu, same)
+        xo = o.get(po.CH_X).astype(np.float32)[typ == po.LEAF]
+        assert np.array_equal(P.get(ca.CH_X)[typ == po.LEAF], xo, equal_nan=True), (coarsest, nu)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nroot,level", BOXES)
+def test_amg_coarse_levels_give_the_oracle_solve(nroot, level):
+    o = po.Oracle(kind=po.SCENE_UNIFORM, nroot=list(nroot), uniform_level=level, seed=sum(nroot))
+    lev, crd, typ, nbr = o.topology()
+    P = ca.Problem(ca.Tree(o.params.h0, lev, crd, typ, o.celltypes()))
+    b = o.get(po.CH_B)
+    o.amg_prepare()
+    S = ca.AMGSolver()
+    S.prepareTypesAndCoeffs(P)
+    for coarsest, nu in ((10, 2), (3, 1), (0, 1)):
+        o.set(po.CH_B, b)
+        P.set(ca.CH_B, b.astype(np.float32))
+        ro = o.amg_solve(max_iters=12, tol=1e-6, level_iters=nu, coarsest_iters=coarsest)
+        S.solve(P, False, 12, 1e-6, nu, coarsest, 1, False)
+        r = S.last_batch[0]
+        assert np.array_equal([r["iters"], r["rr"]], [ro["iters"], ro["rr"]], equal_nan=True), (coarsest, nu, r, ro)
         xo = o.get(po.CH_X).astype(np.float32)[typ == po.LEAF]
         assert np.array_equal(P.get(ca.CH_X)[typ == po.LEAF], xo, equal_nan=True), (coarsest, nu)
 
