@@ -781,7 +781,7 @@ def main():
                     help="always replay one CG iteration's hipGraph (default: the library chooses per handle; "
                          "results identical)")
     ap.add_argument("--eager-max", type=int, default=-1,
-                    help="levels of at most this many tiles use the one-wait prolongation pass (-1: the library default)")
+                    help="accepted and without effect (one form of the prolongation pass serves every size)")
     ap.add_argument("--fused16-max", type=int, default=-1,
                     help="16-bit levels of at most this many tiles run the first down-sweep iteration in one launch "
                          "(-1: the library default)")

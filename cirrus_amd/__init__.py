@@ -468,10 +468,10 @@ class Problem:
                "cg_set_schedule")
 
     def set_level_forms(self, eager_max_tiles=-1, fused16_max_tiles=-1, pair_sweeps=-1):
-        """Level-size limits of the eager prolongation/restriction forms and of
-        the fused first 16-bit sweep, and whether red-black iterations after
-        the first run as one launch of both colours (cg_set_level_forms;
-        results unchanged; 0 never, negative the default)."""
+        """Level-size limit of the fused first 16-bit sweep, and whether
+        red-black iterations after the first run as one launch of both colours
+        (cg_set_level_forms; results unchanged; 0 never, negative the default;
+        eager_max_tiles changes nothing)."""
         _check(lib().cg_set_level_forms(self._h, int(eager_max_tiles), int(fused16_max_tiles), int(pair_sweeps)),
                "cg_set_level_forms")
 

@@ -3,7 +3,7 @@
 // Layout in HBM (structure of arrays, one problem or many in one pool):
 //   channel c of tile t, cell (i,j,k):  ch[c][t*512 + (i<<6 | j<<3 | k)]  (FP32)
 //   cell types:                        ctype[t*512 + ...]                (u8)
-//   worklists:                          arrays of 176-byte TileRec (one per tile
+//   worklists:                          arrays of 128-byte TileRec (one per tile
 //                                       and phase), so a workgroup finds its
 //                                       tile, neighbours and children in one
 //                                       scalar load
@@ -39,20 +39,26 @@ struct alignas(16) TileRec {
   int32_t parent;     // -1 on level 0
   int32_t prob;       // problem index in the pool
   int32_t leaf_slot;  // LEAF: slot of its dot partial; -1 otherwise
-  int32_t gslot;      // GHOST: slot in the 64-value ghost buffer; -1 otherwise
+  int32_t gslot;      // GHOST: slot in the 64-value ghost buffer; LEAF with ghost children: the slot of the
+                      // first of them, where its GhostKids entry is; -1 otherwise
   int32_t self;       // the tile's index
   float h;            // cell size of the tile's level
   uint32_t meta;      // level | type << 8 | octant << 16 | has_gchild << 24 | all_interior << 25 |
-                      // inert_candidate << 26 | all_open << 27
-  uint32_t ntypes;    // type of face neighbour f in bits 4f..4f+3 (0: none)
+                      // inert_candidate << 26 | all_open << 27 | uniform << 28 | h_pow2 << 29
+  uint32_t ntypes;    // type of face neighbour f in bits 4f..4f+3 (0: none), std_face f in bit 24 + f
   float bc[7];        // face coefficients of the smoothing view (subtree at the
                       // tile's own level): faces x-,y-,z-,x+,y+,z+, then inside
   int32_t nbr_parent[6];  // parent tile of face neighbour f (-1: no neighbour or level 0)
-  int32_t gch[8];     // LEAF: ghost child per octant (-1: none)
-  int32_t gcs[8];     // ... and its ghost slot
-  int32_t pad1;
+  float h3;           // (h * h) * h
+  double rdiag;       // 1 / D, D = the sweep's diagonal of a cell whose six faces have the inside coefficient
+  int32_t pad[2];
 };
-static_assert(sizeof(TileRec) == 176, "TileRec is 176 bytes");
+static_assert(sizeof(TileRec) == 128, "TileRec is 128 bytes");
+// The ghost children of a LEAF tile by octant (-1: none): tile and ghost slot.
+struct alignas(16) GhostKids {
+  int32_t tile[8];
+  int32_t slot[8];
+};
 // Fields packed in dwords so that a workgroup fetches them with scalar loads.
 __host__ __device__ __forceinline__ int tr_level(const TileRec& T) { return int(T.meta & 0xff); }
 __host__ __device__ __forceinline__ uint8_t tr_type(const TileRec& T) { return uint8_t((T.meta >> 8) & 0xff); }
@@ -67,6 +73,15 @@ __host__ __device__ __forceinline__ bool tr_inert_cand(const TileRec& T) { retur
 // every cell INTERIOR and no face cut by a NEUMANN cell: each face mask byte is
 // M_OPEN_INT (the masks need not be read)
 __host__ __device__ __forceinline__ bool tr_all_open(const TileRec& T) { return ((T.meta >> 27) & 1) != 0; }
+// every face of the tile has the inside coefficient: with all_open every cell's
+// diagonal is D (rdiag)
+__host__ __device__ __forceinline__ bool tr_uniform(const TileRec& T) { return ((T.meta >> 28) & 1) != 0; }
+// h is a power of two (and h3 its exact cube), so that a product with h3 rounds
+// as three products with h do
+__host__ __device__ __forceinline__ bool tr_h_pow2(const TileRec& T) { return ((T.meta >> 29) & 1) != 0; }
+// every face neighbour is missing, a GHOST tile, or all_open and uniform (so the
+// diagonal of its cells is D)
+__host__ __device__ __forceinline__ bool tr_std_faces(const TileRec& T) { return ((T.ntypes >> 24) & 0x3f) == 0x3f; }
 __host__ __device__ __forceinline__ uint8_t tr_ntype(const TileRec& T, int f) { return uint8_t((T.ntypes >> (4 * f)) & 0xf); }
 
 struct alignas(16) ProbState {
@@ -111,6 +126,7 @@ struct Ctx {
   double* part2; // second partial stream (mean counts)
   const float* diag;  // per cell, colour-split order: the V-cycle colour sweep's diagonal D (k_diag)
   const TileRec* tiles;  // every tile's record by tile index (null where the handle has none)
+  const GhostKids* kids;  // ghost children of LEAF tiles, by TileRec::gslot
   uint8_t* inert = nullptr;  // per tile: 1 while the current solve leaves the tile untouched (k_cg_init)
 };
 
@@ -277,6 +293,24 @@ __device__ __forceinline__ int pick4(int g, int a, int b, int c, int d) {
   const int lo = (g & 1) ? b : a;
   const int hi = (g & 1) ? d : c;
   return (g & 2) ? hi : lo;
+}
+
+// The quotient a / d, correctly rounded, from rd = 1/d in FP64 (within 2^-51
+// of it): the product's relative error is below 2^-50, and a quotient of two
+// 24-bit significands lies at least 2^-49 (relative) from every rounding
+// boundary of FP32, so the conversion rounds to the same value (results below
+// 2^-126, where FP32 has fewer bits, within one unit of their last place).
+// 4 issue slots against 15.5 for the FP32 division on gfx950.
+__device__ __forceinline__ float div_by(float a, double rd) { return float(double(a) * rd); }
+// 1/d in FP64 for finite d != 0: the FP32 reciprocal and two Newton steps (a
+// divisor beyond the range where that reciprocal is a normal number: the division).
+__device__ __forceinline__ double recip64(float d) {
+  const double dd = double(d);
+  const float a = __builtin_fabsf(d);
+  if (!(a >= 0x1p-100f && a <= 0x1p100f)) return 1.0 / dd;
+  double y = double(__builtin_amdgcn_rcpf(d));
+  y = __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
 }
 
 // Wavefront sum of a double in the fixed xor-butterfly order (masks 32..1);
@@ -514,8 +548,20 @@ struct Stencil {
   uint64_t m;          // own face masks, one byte per cell
   float xkm, xkp;      // k-halo values (z- neighbour cell (i,j,7), z+ neighbour cell (i,j,0))
   float b_int, b_f[6]; // base coefficients: inside the tile and across face f
-  float h;
+  float h, h3;
+  double rd;           // the record's rdiag, and what it says of the tile
+  bool open, uniform, p2;
 };
+__device__ __forceinline__ void stencil_coeffs(const TileRec& T, const float bcv[7], Stencil& S) {
+  S.h = T.h;
+  S.h3 = T.h3;
+  S.rd = T.rdiag;
+  S.open = tr_all_open(T);
+  S.uniform = tr_uniform(T);
+  S.p2 = tr_h_pow2(T);
+  S.b_int = bcv[6];
+  for (int f = 0; f < 6; f++) S.b_f[f] = bcv[f];
+}
 
 // Stage tile T's X values (zeros where the flags say so) and face masks.
 //   zero_all:   treat X as 0 everywhere (first sweep from a zero guess)
@@ -617,9 +663,7 @@ __device__ __forceinline__ void stage_commit(StageRaw<V>& r, const TileRec& T, c
   }
   S.xkm = single_f<V>(r.km);
   S.xkp = single_f<V>(r.kp);
-  S.h = T.h;
-  S.b_int = bcv[6];
-  for (int f = 0; f < 6; f++) S.b_f[f] = bcv[f];
+  stencil_coeffs(T, bcv, S);
 }
 
 // Stage tile T's X values (zeros where the flags say so) and face masks.
@@ -737,9 +781,7 @@ __device__ __forceinline__ void stage_commit_pg(StagePG& r, const TileRec& T, co
   const bool ghm = T.nbr[2] >= 0 && tr_ntype(T, 2) == T_GHOST, ghp = T.nbr[5] >= 0 && tr_ntype(T, 5) == T_GHOST;
   S.xkm = (ghm && !(r.km_ct & C_INT)) ? 0.f : r.km;
   S.xkp = (ghp && !(r.kp_ct & C_INT)) ? 0.f : r.kp;
-  S.h = T.h;
-  S.b_int = bcv[6];
-  for (int f = 0; f < 6; f++) S.b_f[f] = bcv[f];
+  stencil_coeffs(T, bcv, S);
 }
 
 // Face coefficients of tile T seen with the subtree view at level sl
@@ -805,19 +847,48 @@ __device__ __forceinline__ NbrPencils lds_nbrs(const TileLDS& L) {
   return N;
 }
 
-// A x (and its diagonal) on all 8 cells of the lane, given its neighbour pencils.
+// A x (and its diagonal) on all 8 cells of the lane, its i/j neighbours read from
+// the staged pencils.  Open tiles take the short rows, one half of the pencil at a
+// time (both at once need more registers than eight wavefronts a SIMD leave, and
+// HBM-bound passes need those wavefronts).  The apply of the refined 45,054-tile
+// scene 61 -> 55 us, of the 256-problem pool 1089 -> 1060 us (5.9 TB/s).
 template <bool WANT_AX, bool WANT_D>
-__device__ __forceinline__ void apply_pencil(const NbrPencils& N, const Stencil& S, float ax[8], float dg[8]) {
+__device__ __forceinline__ void apply_pencil(const TileLDS& L, const Stencil& S, float ax[8], float dg[8]) {
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
+  const float bim = (i == 0) ? S.b_f[0] : S.b_int;
+  const float bip = (i == 7) ? S.b_f[3] : S.b_int;
+  const float bjm = (j == 0) ? S.b_f[1] : S.b_int;
+  const float bjp = (j == 7) ? S.b_f[4] : S.b_int;
+  if (WANT_AX && !WANT_D && S.open) {
+    // every cell INTERIOR, no face cut: the base coefficients as they are
+    // (cell_row_m's sums; 13 or 15 operations a cell instead of about 30), one
+    // half of the pencil at a time
+    const int pc = (i + 1) * 10 + (j + 1);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const float4 im = L.xs[h][pc - 10], ip = L.xs[h][pc + 10], jm = L.xs[h][pc - 1], jp = L.xs[h][pc + 1];
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        const int k = 4 * h + m;
+        const float x0 = S.own[k];
+        float s = 0.f;
+        s = __builtin_fmaf(bim, x0 - comp4(im, m), s);
+        s = __builtin_fmaf(bip, x0 - comp4(ip, m), s);
+        s = __builtin_fmaf(bjm, x0 - comp4(jm, m), s);
+        s = __builtin_fmaf(bjp, x0 - comp4(jp, m), s);
+        s = __builtin_fmaf((k == 0) ? S.b_f[2] : S.b_int, x0 - ((k == 0) ? S.xkm : S.own[k - 1]), s);
+        s = __builtin_fmaf((k == 7) ? S.b_f[5] : S.b_int, x0 - ((k == 7) ? S.xkp : S.own[k + 1]), s);
+        ax[k] = ((s * S.h) * S.h) * S.h;
+      }
+    }
+    return;
+  }
+  const NbrPencils N = lds_nbrs(L);
   float xim[8], xip[8], xjm[8], xjp[8];
   unpack8(N.im0, N.im1, xim);
   unpack8(N.ip0, N.ip1, xip);
   unpack8(N.jm0, N.jm1, xjm);
   unpack8(N.jp0, N.jp1, xjp);
-  const float bim = (i == 0) ? S.b_f[0] : S.b_int;
-  const float bip = (i == 7) ? S.b_f[3] : S.b_int;
-  const float bjm = (j == 0) ? S.b_f[1] : S.b_int;
-  const float bjp = (j == 7) ? S.b_f[4] : S.b_int;
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     const float xn[6] = {xim[k], xip[k], xjm[k], xjp[k], (k == 0) ? S.xkm : S.own[k - 1], (k == 7) ? S.xkp : S.own[k + 1]};
@@ -829,123 +900,103 @@ __device__ __forceinline__ void apply_pencil(const NbrPencils& N, const Stencil&
   }
 }
 
-
-// One red-black colour update on the lane's four cells of that colour: cell
-// (i,j,k) is updated when (i+j+k) % 2 == color, i.e. k = 2m + p with the lane's
-// parity p.  The operands of those four rows are gathered with whole-vector
-// selects on p (no per-lane register indexing), so only the four rows are formed.
-__device__ __forceinline__ void gs_pencil(const NbrPencils& N, const Stencil& S, const float b[8], int color,
-                                          float4& out0, float4& out1) {
-  const int lane = lane_id(), i = lane >> 3, j = lane & 7;
-  const bool p = ((color + i + j) & 1) != 0;
-  auto pick = [&](float4 a, float4 c) { return sel4(p, even4(a, c), odd4(a, c)); };
-  const float4 XIM = pick(N.im0, N.im1);
-  const float4 XIP = pick(N.ip0, N.ip1);
-  const float4 XJM = pick(N.jm0, N.jm1);
-  const float4 XJP = pick(N.jp0, N.jp1);
-  const float4 o0 = make_float4(S.own[0], S.own[1], S.own[2], S.own[3]);
-  const float4 o1 = make_float4(S.own[4], S.own[5], S.own[6], S.own[7]);
-  const float4 EV = even4(o0, o1), OD = odd4(o0, o1);
-  const float4 X0 = sel4(p, EV, OD);
-  // k-1 and k+1 neighbours of cell 2m+p
-  const float4 XKM = sel4(p, make_float4(S.xkm, OD.x, OD.y, OD.z), EV);
-  const float4 XKP = sel4(p, OD, make_float4(EV.y, EV.z, EV.w, S.xkp));
-  const float4 B = sel4(p, make_float4(b[0], b[2], b[4], b[6]), make_float4(b[1], b[3], b[5], b[7]));
-  const float bim = (i == 0) ? S.b_f[0] : S.b_int;
-  const float bip = (i == 7) ? S.b_f[3] : S.b_int;
-  const float bjm = (j == 0) ? S.b_f[1] : S.b_int;
-  const float bjp = (j == 7) ? S.b_f[4] : S.b_int;
-  const int sh = p ? 8 : 0;
-  float nv[4];
-#pragma unroll
-  for (int m = 0; m < 4; m++) {
-    const uint32_t mb = (m < 2 ? uint32_t(S.m) : uint32_t(S.m >> 32)) >> (16 * (m & 1) + sh);  // bits 0..6 used
-    const float bkm = (!p && m == 0) ? S.b_f[2] : S.b_int;
-    const float bkp = (p && m == 3) ? S.b_f[5] : S.b_int;
-    const float x0 = comp4(X0, m);
-    const float xn[6] = {comp4(XIM, m), comp4(XIP, m), comp4(XJM, m), comp4(XJP, m), comp4(XKM, m), comp4(XKP, m)};
-    const float bc[6] = {bim, bip, bjm, bjp, bkm, bkp};
-    float ax, dg;
-    cell_row_m<true>(x0, mb, xn, bc, S.h, ax, dg);
-    float delta = 0.f;
-    if ((mb & M_INT) && dg != 0.f) delta = (comp4(B, m) - ax) / dg;
-    nv[m] = x0 + delta;
-  }
-  // put the four new values back at their parity positions
-  out0 = sel4(p, make_float4(nv[0], o0.y, nv[1], o0.w), make_float4(o0.x, nv[0], o0.z, nv[1]));
-  out1 = sel4(p, make_float4(nv[2], o1.y, nv[3], o1.w), make_float4(o1.x, nv[2], o1.z, nv[3]));
+// What a colour update needs of its tile besides values: the face coefficients
+// and sizes, and what the record says of the tile.
+struct GsCoef {
+  const float* bc;  // faces x-..z+, inside
+  float h, h3;
+  double rd;
+  bool open, uniform, p2;
+};
+__device__ __forceinline__ GsCoef gs_coef(const TileRec& T) {
+  return GsCoef{T.bc, T.h, T.h3, T.rdiag, tr_all_open(T), tr_uniform(T), tr_h_pow2(T)};
 }
-
-// ---------------------------------------------------------------------------
-// Per-tile bodies (one wavefront each)
-// ---------------------------------------------------------------------------
+// b - A x of an open cell from its row sum: ((s h) h) h, one exact product when h
+// is a power of two (then b - s h3 rounds once either way).
+__device__ __forceinline__ float open_residual(const GsCoef& G, float s, float b) {
+  return G.p2 ? __builtin_fmaf(-s, G.h3, b) : b - ((s * G.h) * G.h) * G.h;
+}
+// 1/D of a lane's open cells: those inside the pencil (mid) and at its ends
+// k = 0 (lo) and k = 7 (hi), the sums formed as cell_row_m forms them (0: D is 0).
+struct OpenDiag {
+  double mid, lo, hi;
+};
+__device__ __forceinline__ OpenDiag open_diag(const GsCoef& G, float bim, float bip, float bjm, float bjp) {
+  if (G.uniform) return OpenDiag{G.rd, G.rd, G.rd};
+  const float bi = G.bc[6], d4 = (((0.f + bim) + bip) + bjm) + bjp;
+  auto inv = [&](float d) {
+    const float g = ((d * G.h) * G.h) * G.h;
+    return g != 0.f ? recip64(g) : 0.0;
+  };
+  return OpenDiag{inv((d4 + bi) + bi), inv((d4 + G.bc[2]) + bi), inv((d4 + bi) + G.bc[5])};
+}
 
 // The four updated cells of a red-black colour pass, in split-layout quads:
 // cell k = 2m + p of lane (i,j) (p = (color+i+j)&1) with value X0.m, rhs B.m,
 // i/j neighbours XIM..XJP (component m: the neighbours' other-colour quads line
 // up with the lane's updated quad), the lane's other-colour quad XO and the
-// k-halo values xkm (cell (i,j,-1), used when p = 0) and xkp ((i,j,8), p = 1).
+// k-halo value xk (cell (i,j,-1) when p = 0, (i,j,8) when p = 1).
+// ZERO: every x is 0 (the first pass), so A x = 0.
+// A tile whose record says all_open (every cell INTERIOR, no face cut: two thirds
+// of the batched workload's) needs no masks, and D takes at most three values a
+// lane, one where no face neighbour is a GHOST: its quotients are products with
+// the 64-bit 1/D (div_by).  About 200 vector operations a tile instead of 290;
+// the other tiles take the general rows and the FP32 division.  The colour pass
+// of the 360,472-tile level of a 256-problem pool, in FP32: 319 -> 300 us; on a
+// level of 64 tiles, where a pass is one chain of waits: 2.61 -> 2.48 us.
+template <bool ZERO = false>
 __device__ __forceinline__ float4 gs_quad(float4 X0, float4 XO, float4 XIM, float4 XIP, float4 XJM, float4 XJP,
-                                          float xkm, float xkp, float4 B, uint32_t mq, const float bcv[7], float h,
-                                          int i, int j, bool p) {
+                                          float xk, float4 B, uint32_t mq, const GsCoef& G, int i, int j, bool p) {
   // k-1 and k+1 neighbours of cell 2m+p
-  const float4 XKM = sel4(p, make_float4(xkm, XO.x, XO.y, XO.z), XO);
-  const float4 XKP = sel4(p, XO, make_float4(XO.y, XO.z, XO.w, xkp));
-  const float bi = bcv[6];
-  const float bim = (i == 0) ? bcv[0] : bi;
-  const float bip = (i == 7) ? bcv[3] : bi;
-  const float bjm = (j == 0) ? bcv[1] : bi;
-  const float bjp = (j == 7) ? bcv[4] : bi;
+  const float4 XKM = sel4(p, make_float4(xk, XO.x, XO.y, XO.z), XO);
+  const float4 XKP = sel4(p, XO, make_float4(XO.y, XO.z, XO.w, xk));
+  const float bi = G.bc[6];
+  const float bim = (i == 0) ? G.bc[0] : bi;
+  const float bip = (i == 7) ? G.bc[3] : bi;
+  const float bjm = (j == 0) ? G.bc[1] : bi;
+  const float bjp = (j == 7) ? G.bc[4] : bi;
   float nv[4];
-  if (__all(mq == M_OPEN_INT * 0x01010101u)) {
-    // Every updated cell of the wavefront is INTERIOR with six uncut faces:
-    // each face coefficient is its base coefficient, so the diagonal sum
-    // depends on the cell only through the k faces.  Its sums are formed once
-    // per lane in the same order as cell_row_m forms them (faces x-, x+, y-,
-    // y+, z-, z+; adding a zero is exact), so every value is the general path's.
-    const float d4 = (((0.f + bim) + bip) + bjm) + bjp;
-    const float dmid = (d4 + bi) + bi;
-    const float dlo = (d4 + bcv[2]) + bi;   // cell k = 0 (p = 0, m = 0)
-    const float dhi = (d4 + bi) + bcv[5];   // cell k = 7 (p = 1, m = 3)
-    const float gmid = ((dmid * h) * h) * h;
-    const float glo = ((dlo * h) * h) * h;
-    const float ghi = ((dhi * h) * h) * h;
+  if (G.open) {
+    const OpenDiag D = open_diag(G, bim, bip, bjm, bjp);
+    const double dlo = p ? D.mid : D.lo, dhi = p ? D.hi : D.mid;  // of m = 0 and m = 3
+    const float bkm = p ? bi : G.bc[2], bkp = p ? G.bc[5] : bi;   // of m = 0 (k - 1) and m = 3 (k + 1)
 #pragma unroll
     for (int m = 0; m < 4; m++) {
-      const float bkm = (!p && m == 0) ? bcv[2] : bi;
-      const float bkp = (p && m == 3) ? bcv[5] : bi;
       const float x0 = comp4(X0, m);
       float s = 0.f;
-      s = __builtin_fmaf(bim, x0 - comp4(XIM, m), s);
-      s = __builtin_fmaf(bip, x0 - comp4(XIP, m), s);
-      s = __builtin_fmaf(bjm, x0 - comp4(XJM, m), s);
-      s = __builtin_fmaf(bjp, x0 - comp4(XJP, m), s);
-      s = __builtin_fmaf(bkm, x0 - comp4(XKM, m), s);
-      s = __builtin_fmaf(bkp, x0 - comp4(XKP, m), s);
-      const float ax = ((s * h) * h) * h;
-      const float dg = (!p && m == 0) ? glo : ((p && m == 3) ? ghi : gmid);
-      float delta = 0.f;
-      if (dg != 0.f) delta = (comp4(B, m) - ax) / dg;
-      nv[m] = x0 + delta;
+      if (!ZERO) {
+        s = __builtin_fmaf(bim, x0 - comp4(XIM, m), s);
+        s = __builtin_fmaf(bip, x0 - comp4(XIP, m), s);
+        s = __builtin_fmaf(bjm, x0 - comp4(XJM, m), s);
+        s = __builtin_fmaf(bjp, x0 - comp4(XJP, m), s);
+        s = __builtin_fmaf(m == 0 ? bkm : bi, x0 - comp4(XKM, m), s);
+        s = __builtin_fmaf(m == 3 ? bkp : bi, x0 - comp4(XKP, m), s);
+      }
+      const float res = ZERO ? comp4(B, m) - 0.f : open_residual(G, s, comp4(B, m));
+      nv[m] = x0 + div_by(res, m == 0 ? dlo : (m == 3 ? dhi : D.mid));
     }
     return make_float4(nv[0], nv[1], nv[2], nv[3]);
   }
 #pragma unroll
   for (int m = 0; m < 4; m++) {
     const uint32_t mb = mq >> (8 * m);  // bits 0..6 used
-    const float bkm = (!p && m == 0) ? bcv[2] : bi;
-    const float bkp = (p && m == 3) ? bcv[5] : bi;
+    const float bkm = (!p && m == 0) ? G.bc[2] : bi;
+    const float bkp = (p && m == 3) ? G.bc[5] : bi;
     const float x0 = comp4(X0, m);
     const float xn[6] = {comp4(XIM, m), comp4(XIP, m), comp4(XJM, m), comp4(XJP, m), comp4(XKM, m), comp4(XKP, m)};
     const float bc[6] = {bim, bip, bjm, bjp, bkm, bkp};
     float ax, dg;
-    cell_row_m<true>(x0, mb, xn, bc, h, ax, dg);
+    cell_row_m<true>(x0, mb, xn, bc, G.h, ax, dg);
     float delta = 0.f;
-    if ((mb & M_INT) && dg != 0.f) delta = (comp4(B, m) - ax) / dg;
+    if ((mb & M_INT) && dg != 0.f) delta = (comp4(B, m) - (ZERO ? 0.f : ax)) / dg;
     nv[m] = x0 + delta;
   }
   return make_float4(nv[0], nv[1], nv[2], nv[3]);
 }
+
+// ---------------------------------------------------------------------------
+// Per-tile bodies (one wavefront each)
+// ---------------------------------------------------------------------------
 
 struct GsLDS {
   float4 xo[100];  // other-colour quads of the tile's pencils and of the halo ring, index (i+1)*10 + (j+1)
@@ -968,13 +1019,13 @@ struct GsIn {
   float4 xc, xo, B, halo;
   float4 r0, r1;  // with F_DOT_RZ on a LEAF tile: r of the lane's pencil, cells 0..3 and 4..7
   uint32_t mask;  // the face masks of the lane's four cells of the pass's colour
-  float xkm, xkp;
+  float xk;       // k halo: cell (i,j,7) of the z- neighbour (p = 0) or (i,j,0) of the z+ one (p = 1)
   int32_t done;   // the problem's done flag, loaded with the tile's data (used with F_CHECK_DONE only)
 };
 template <class V>
 struct GsRaw {
   typename RawV<V>::Q xc, xo, B, halo;
-  typename RawV<V>::S xkm, xkp;
+  typename RawV<V>::S xk;
   float4 r0, r1;
   uint32_t mask;
   int32_t done;
@@ -1022,14 +1073,12 @@ __device__ __forceinline__ GsRaw<V> gs_issue(const Ctx& c, const TileRec& T, con
     const bool ok = lane < 32 && n >= 0 && !(zero_all || (ghost_zero && gh));
     g.halo = load_q_raw(ok ? X + size_t(n) * 512 + ho + src_pl * 4 : zp);
   }
-  // k halos: cell (i,j,7) of the z- neighbour and (i,j,0) of the z+ neighbour
+  // k halo, the one that the lane's cells of this colour reach (colour ho either way)
   {
-    int n = T.nbr[2];
-    bool ok = n >= 0 && !(zero_all || (ghost_zero && tr_ntype(T, 2) == T_GHOST));
-    g.xkm = load_s_raw(ok ? X + size_t(n) * 512 + split_cell(i, j, 7) : zp);
-    n = T.nbr[5];
-    ok = n >= 0 && !(zero_all || (ghost_zero && tr_ntype(T, 5) == T_GHOST));
-    g.xkp = load_s_raw(ok ? X + size_t(n) * 512 + split_cell(i, j, 0) : zp);
+    const bool p = ((color + i + j) & 1) != 0;
+    const int n = p ? uni(T.nbr[5]) : uni(T.nbr[2]);
+    const bool ok = n >= 0 && !(zero_all || (ghost_zero && tr_ntype(T, p ? 5 : 2) == T_GHOST));
+    g.xk = load_s_raw(ok ? X + size_t(n) * 512 + ho + lane * 4 + (p ? 0 : 3) : zp);
   }
   return g;
 }
@@ -1039,15 +1088,13 @@ __device__ __forceinline__ GsIn gs_convert(GsRaw<V>& r) {
   hold(r.xo);
   hold(r.B);
   hold(r.halo);
-  hold(r.xkm);
-  hold(r.xkp);
+  hold(r.xk);
   GsIn g;
   g.xc = quad_f<V>(r.xc);
   g.xo = quad_f<V>(r.xo);
   g.B = quad_f<V>(r.B);
   g.halo = quad_f<V>(r.halo);
-  g.xkm = single_f<V>(r.xkm);
-  g.xkp = single_f<V>(r.xkp);
+  g.xk = single_f<V>(r.xk);
   g.r0 = r.r0;
   g.r1 = r.r1;
   g.mask = r.mask;
@@ -1078,8 +1125,8 @@ __device__ __forceinline__ void gs_finish(const Ctx& c, const TileRec& T, V* X, 
   V* tile = X + size_t(T.self) * 512;
   const int pc = (i + 1) * 10 + (j + 1);
   const bool p = ((color + i + j) & 1) != 0;
-  const float4 nv = gs_quad(g.xc, g.xo, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], g.xkm, g.xkp, g.B,
-                            g.mask, T.bc, T.h, i, j, p);
+  const float4 nv = gs_quad(g.xc, g.xo, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], g.xk, g.B, g.mask,
+                            gs_coef(T), i, j, p);
   store4(tile + hc + lane * 4, nv);
   if (flags & F_ZERO_X) store4(tile + ho + lane * 4, make_float4(0.f, 0.f, 0.f, 0.f));  // the zero guess of the other colour
   if (DOT && tr_type(T) == T_LEAF) {
@@ -1110,8 +1157,7 @@ __device__ __forceinline__ void tile_gs(const Ctx& c, const TileRec& T, int leve
 
 // stage_tile on the V-cycle arrays plus the tile's rhs b (natural order; 0 with
 // zero_b), the rhs loaded with the stage's loads, ahead of the one wait.
-// EAGER (the host's choice for small levels) stages the same way.
-template <class V, bool EAGER = false>
+template <class V>
 __device__ __forceinline__ void stage_with_rhs(const Ctx& c, const TileRec& T, const V* X, const V* XG, const V* F,
                                                int flags, bool zero_b, TileLDS& L, Stencil& S, float b[8]) {
   const V* src = zero_b ? zero_page<V>() : ((flags & F_VCYCLE) ? vc_rhs<V>(c) : F) + size_t(T.self) * 512;
@@ -1135,9 +1181,21 @@ __device__ __forceinline__ void tile_jacobi(const Ctx& c, const TileRec& T, int 
   stage_with_rhs(c, T, X, XG, F, flags, false, L, S, b);
   if (prob_done(c, T, flags)) return;
   wave_sync();
-  float ax[8], dg[8];
-  apply_pencil<true, true>(lds_nbrs(L), S, ax, dg);
-  float out[8];
+  float ax[8], dg[8], out[8];
+  if (S.open) {  // as gs_quad's open tiles: no masks, quotients as products with 1/D
+    apply_pencil<true, false>(L, S, ax, dg);
+    const int i = lane_id() >> 3, j = lane_id() & 7;
+    const OpenDiag D = open_diag(gs_coef(T), i == 0 ? T.bc[0] : T.bc[6], i == 7 ? T.bc[3] : T.bc[6],
+                                 j == 0 ? T.bc[1] : T.bc[6], j == 7 ? T.bc[4] : T.bc[6]);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const double rd = k == 0 ? D.lo : (k == 7 ? D.hi : D.mid);
+      out[k] = rd != 0.0 ? S.own[k] + div_by(omega * (b[k] - ax[k]), rd) : 0.f;
+    }
+    store8_split(Y + size_t(T.self) * 512, lane_id(), out);
+    return;
+  }
+  apply_pencil<true, true>(L, S, ax, dg);
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     out[k] = S.own[k];
@@ -1176,17 +1234,17 @@ __device__ __forceinline__ size_t parent_cell_split(const TileRec& T, int q) {
 // (GMGSolver.cu:284-339).  Output channel CO (rhsv in V-cycle mode): the
 // parent cell = sum * one_over_alpha, or += sum for a GHOST fine tile (whose
 // LEAF parent's rhs already holds r).  In V-cycle mode a ghost's rhs is 0.
-template <class V, bool EAGER = false>
+template <class V>
 __device__ __forceinline__ void tile_restrict(const Ctx& c, const TileRec& T, int level, const V* X, const V* F,
                                               V* CO, float one_over_alpha, int flags, TileLDS& L, float* res) {
   Stencil S;
   const int lane = lane_id();
   float b[8];
-  stage_with_rhs<V, EAGER>(c, T, X, X, F, flags, (flags & F_VCYCLE) && tr_type(T) == T_GHOST, L, S, b);
+  stage_with_rhs<V>(c, T, X, X, F, flags, (flags & F_VCYCLE) && tr_type(T) == T_GHOST, L, S, b);
   if (prob_done(c, T, flags)) return;
   wave_sync();
   float ax[8], dg[8];
-  apply_pencil<true, false>(lds_nbrs(L), S, ax, dg);
+  apply_pencil<true, false>(L, S, ax, dg);
   for (int k = 0; k < 8; k++) res[lane * 8 + k] = b[k] - ax[k];
   wave_sync();
   float s = octet_sum(res, lane);
@@ -1225,119 +1283,10 @@ __device__ __forceinline__ void tile_prolong(const Ctx& c, const TileRec& T, int
   }
 }
 
-// Prolongation fused into the first colour pass of the up-sweep on a level
-// (GMGSolver.cu:345-376 then :216-269): every value the pass reads -- own cells
-// and the face halos -- is formed on the fly as the prolongation would leave
-// it (x + pcoef * parent on INTERIOR cells of active tiles, the parent value on
-// INTERIOR cells of GHOST tiles, 0 elsewhere), so no separate launch is needed.
-// XD holds the down-sweep values, XO receives the level's result; GHOST tiles
-// in the list only store their prolongated values.
-// parent cells of pencil (i,j) of a child in octant oct (colour-split array)
-template <class V>
-__device__ __forceinline__ float4 parent_quad(const V* XC, int parent, int oct, int i, int j) {
-  const int ox = oct & 1, oy = (oct >> 1) & 1, oz = (oct >> 2) & 1;
-  return load_quad_split(XC + size_t(parent) * 512, (ox * 4 + (i >> 1)) * 8 + (oy * 4 + (j >> 1)), oz * 4);
-}
-// prolongated values of one pencil: active (fma with the down-sweep values) or
-// ghost; m: the pencil's face masks (their INTERIOR bits).  Values are rounded
-// as a store to V-typed memory would leave them.
-template <class V>
-__device__ __forceinline__ void prolong_pencil(float4 xa, float4 xb, float4 pq, uint64_t m, bool ghost, float pcoef,
-                                               float4& oa, float4& ob) {
-  const float cz[4] = {pq.x, pq.y, pq.z, pq.w};
-  float xo[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-  float o[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const bool in = ct_at(m, k) & M_INT;
-    o[k] = in ? vround<V>(ghost ? cz[k >> 1] : __builtin_fmaf(pcoef, cz[k >> 1], xo[k])) : 0.f;
-  }
-  oa = make_float4(o[0], o[1], o[2], o[3]);
-  ob = make_float4(o[4], o[5], o[6], o[7]);
-}
-
-// Prolongated k-halo value of lane (i,j): cell (i,j,KN) of face neighbour F.
-template <int F, int KN, class V>
-__device__ __forceinline__ void khalo_prolong(const Ctx& c, const TileRec& T, const V* XD, const V* XO, float pcoef,
-                                              int oct, int lane, float& xv) {
-  const int n = T.nbr[F];
-  if (n < 0) { xv = 0.f; return; }
-  const int i = lane >> 3, j = lane & 7;
-  const uint8_t mv = c.fmask[size_t(n) * 512 + lane * 8 + KN];
-  const bool gh = tr_ntype(T, F) == T_GHOST;
-  const int noct = oct ^ 4;
-  const int ox = noct & 1, oy = (noct >> 1) & 1, oz = (noct >> 2) & 1;
-  const float pz = to_f(XO[size_t(T.nbr_parent[F]) * 512 + split_cell(ox * 4 + (i >> 1), oy * 4 + (j >> 1), oz * 4 + (KN >> 1))]);
-  const float xo = gh ? 0.f : to_f(XD[size_t(n) * 512 + split_cell(i, j, KN)]);
-  xv = (mv & M_INT) ? vround<V>(gh ? pz : __builtin_fmaf(pcoef, pz, xo)) : 0.f;
-}
-
-template <class V>
-__device__ __forceinline__ void tile_gs_prolong(const Ctx& c, const TileRec& T, const V* XD, V* XO, float pcoef,
-                                                int color, int flags, TileLDS& L) {
-  const int lane = lane_id(), i = lane >> 3, j = lane & 7;
-  const int oct = tr_octant(T);
-  const bool own_ghost = tr_type(T) == T_GHOST;
-  const uint64_t mown = load_ct8(own_masks(c, T) + lane * 8);
-  const float4 pq = parent_quad(XO, T.parent, oct, i, j);
-  float4 xa = make_float4(0.f, 0.f, 0.f, 0.f), xb = xa;
-  if (!own_ghost) load_pencil_split(XD + size_t(T.self) * 512, lane, xa, xb);
-  float4 oa, ob;
-  prolong_pencil<V>(xa, xb, pq, mown, own_ghost, pcoef, oa, ob);
-  if (own_ghost) {  // GHOST tile: its prolongated values only
-    if (prob_done(c, T, flags)) return;
-    store_pencil_split(XO + size_t(T.self) * 512, lane, oa, ob);
-    return;
-  }
-  Stencil S;
-  S.own[0] = oa.x; S.own[1] = oa.y; S.own[2] = oa.z; S.own[3] = oa.w;
-  S.own[4] = ob.x; S.own[5] = ob.y; S.own[6] = ob.z; S.own[7] = ob.w;
-  S.m = mown;
-  const int pc = (i + 1) * 10 + (j + 1);
-  L.xs[0][pc] = oa;
-  L.xs[1][pc] = ob;
-  // halo ring, lanes 0..31 (as stage_tile), prolongated in the neighbour's frame
-  if (lane < 32) {
-    const int g = lane >> 3, t = lane & 7;
-    const int f = (g == 0) ? 0 : (g == 1) ? 3 : (g == 2) ? 1 : 4;
-    // the record's fields as uniform values, so that the per-lane choice below is
-    // a register select and not an indexed access to the record
-    const int n = pick4(g, uni(T.nbr[0]), uni(T.nbr[3]), uni(T.nbr[1]), uni(T.nbr[4]));
-    const int pn = pick4(g, uni(T.nbr_parent[0]), uni(T.nbr_parent[3]), uni(T.nbr_parent[1]), uni(T.nbr_parent[4]));
-    const int ni = (g == 0) ? 7 : (g == 1) ? 0 : t, nj = (g == 2) ? 7 : (g == 3) ? 0 : t;  // pencil in the neighbour
-    const int dst = (g == 0) ? (t + 1) : (g == 1) ? (91 + t) : (g == 2) ? ((t + 1) * 10) : ((t + 1) * 10 + 9);
-    const int noct = oct ^ (1 << (f % 3));
-    float4 va = make_float4(0.f, 0.f, 0.f, 0.f), vb = va;  // x = 0 outside the grid (GMGSolver.cu:120-122)
-    if (n >= 0) {
-      const bool gh = tr_ntype(T, f) == T_GHOST;
-      const uint64_t w = load_ct8(c.fmask + size_t(n) * 512 + (ni * 8 + nj) * 8);
-      float4 ya = make_float4(0.f, 0.f, 0.f, 0.f), yb = ya;
-      if (!gh) load_pencil_split(XD + size_t(n) * 512, ni * 8 + nj, ya, yb);
-      prolong_pencil<V>(ya, yb, parent_quad(XO, pn, noct, ni, nj), w, gh, pcoef, va, vb);
-    }
-    L.xs[0][dst] = va;
-    L.xs[1][dst] = vb;
-  }
-  // k halos: cell (i,j,7) of the z- neighbour and (i,j,0) of the z+ neighbour
-  khalo_prolong<2, 7>(c, T, XD, XO, pcoef, oct, lane, S.xkm);
-  khalo_prolong<5, 0>(c, T, XD, XO, pcoef, oct, lane, S.xkp);
-  S.h = T.h;
-  S.b_int = T.bc[6];
-  for (int f = 0; f < 6; f++) S.b_f[f] = T.bc[f];
-  float b[8];
-  load8_split(vc_rhs<V>(c) + size_t(T.self) * 512, lane, b);
-  if (prob_done(c, T, flags)) return;
-  wave_sync();
-  float4 out0, out1;
-  gs_pencil(lds_nbrs(L), S, b, color, out0, out1);
-  store_pencil_split(XO + size_t(T.self) * 512, lane, out0, out1);
-}
-
 // ---------------------------------------------------------------------------
 // One-tile-per-workgroup kernels over a worklist
 // ---------------------------------------------------------------------------
-// The first 128 bytes of a tile's record (everything but the ghost children's
-// slots), fetched by two scalar loads that nothing else waits behind: the held
+// A tile's record, fetched by two scalar loads that nothing else waits behind: the held
 // words keep the compiler from splitting the fetch into pieces that it would
 // load, wait for and test one after another.  A wavefront's cost on a small
 // level is its chain of memory round trips: with the launch's n and flags
@@ -1361,6 +1310,8 @@ __device__ __forceinline__ TileRec unpack_rec(RecWords a, RecWords b) {
   T.bc[1] = __int_as_float(a[15]);
   for (int f = 2; f < 7; f++) T.bc[f] = __int_as_float(b[f - 2]);
   for (int f = 0; f < 6; f++) T.nbr_parent[f] = b[5 + f];
+  T.h3 = __int_as_float(b[11]);
+  T.rdiag = __hiloint2double(b[13], b[12]);
   return T;
 }
 __device__ __forceinline__ TileRec load_rec(const TileRec* __restrict__ list, int w) {
@@ -1386,11 +1337,6 @@ __device__ __forceinline__ TileRec load_rec(const TileRec* __restrict__ list, in
   const int w = work_index(flags & F_SWIZZLE, n);                                      \
   if (w >= n) return;                                                                  \
   const TileRec T = load_rec(list, w, c);
-// The whole record, the ghost children's slots among it.
-#define TILE_KERNEL_PROLOGUE_ALL                                                       \
-  const int w = work_index(flags & F_SWIZZLE, n);                                      \
-  if (w >= n) return;                                                                  \
-  const TileRec T = list[w];
 // In a CG iteration's launch, a tile that k_cg_init found inert exits: the
 // launch would write the values its arrays already hold.
 #define SKIP_INERT \
@@ -1419,8 +1365,8 @@ __global__ __launch_bounds__(64) void k_gs_color_to(const TileRec* __restrict__ 
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const int pc = (i + 1) * 10 + (j + 1);
   const bool p = ((color + i + j) & 1) != 0;
-  const float4 nv = gs_quad(g.xc, g.xo, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], g.xkm, g.xkp, g.B,
-                            g.mask, T.bc, T.h, i, j, p);
+  const float4 nv = gs_quad(g.xc, g.xo, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], g.xk, g.B, g.mask,
+                            gs_coef(T), i, j, p);
   V* tile = Y + size_t(T.self) * 512;
   store4(tile + (color << 8) + lane * 4, nv);
   store4(tile + ((color ^ 1) << 8) + lane * 4, g.xo);
@@ -1545,13 +1491,22 @@ __device__ __forceinline__ float first_red(float b, float d) {
   const float delta = (d != 0.f) ? (b - 0.f) / d : 0.f;
   return vround<V>(0.f + delta);
 }
+// the same for a cell whose 1/D is rd
+template <class V>
+__device__ __forceinline__ float first_red_by(float b, double rd) {
+  return vround<V>(0.f + div_by(b - 0.f, rd));
+}
 
 // The first red-black iteration of a down-sweep level from the zero guess in
 // one launch: both colour passes of GMGSolver.cu:216-269 (colour 0 from x = 0,
 // the other colour written 0; then colour 1).  After the first pass a colour-0
 // cell depends on its own rhs and diagonal only, so the colour-0 values of the
-// halo are formed from the neighbours' rhs and stored diagonals and the second
-// pass needs no grid-wide wait.  Every value is the one the two passes give.
+// halo are formed from the neighbours' rhs and diagonals and the second pass
+// needs no grid-wide wait.  Every value is the one the two passes give.
+// Where every face neighbour's diagonals are the record's D (tr_std_faces: most
+// tiles) the halo's diagonals are not read (their loads go to the zero page) and
+// its five quotients are products with 1/D: 256 problems in bfloat16, the level of
+// 360,472 tiles as two passes 222.1 ms a solve, as this one launch 216.6.
 template <class V>
 __global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ list, int n, int flags, V* X, Ctx c) {
   TILE_KERNEL_PROLOGUE_C
@@ -1559,42 +1514,34 @@ __global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ lis
   __shared__ GsLDS L;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const bool ghost_zero = flags & F_GHOST_ZERO;
+  const bool std_faces = tr_std_faces(T);
   const V* R = vc_rhs<V>(c);
+  const V* zp = zero_page<V>();
+  const float* zf = zero_page<float>();
   // ---- loads, all issued before the first wait
   const int32_t* dp = (flags & F_CHECK_DONE) ? &c.ps[T.prob].done : reinterpret_cast<const int32_t*>(c.fmask);
   const int32_t done = *dp;
-  const uint64_t mask = load_ct8(own_masks(c, T) + lane * 8);
+  const uint32_t* masks = own_split_masks(c, T);
+  const uint32_t mq0 = masks[lane], mq1 = masks[64 + lane];
   typename RawV<V>::Q rb0 = load_q_raw(R + size_t(T.self) * 512 + lane * 4);        // colour-0 rhs quad
   typename RawV<V>::Q rb1 = load_q_raw(R + size_t(T.self) * 512 + 256 + lane * 4);  // colour-1 rhs quad
-  // halo ring of the colour-1 pass: lanes 0..31, the colour-0 quad of one neighbour pencil
-  // (a missing or ghost neighbour is read at the tile itself and its value
-  // taken as 0 afterwards, so that the loads need no inner branch)
-  typename RawV<V>::Q hb{};
-  float4 hd = make_float4(0.f, 0.f, 0.f, 0.f);
-  int dst = 0;
-  bool hok = false;
-  if (lane < 32) {
-    const int q = lane >> 3, t = lane & 7;
-    const int f = (q == 0) ? 0 : (q == 1) ? 3 : (q == 2) ? 1 : 4;
-    const int nb = pick4(q, uni(T.nbr[0]), uni(T.nbr[3]), uni(T.nbr[1]), uni(T.nbr[4]));
-    const int src_pl = (q == 0) ? (56 + t) : (q == 1) ? t : (q == 2) ? (t * 8 + 7) : (t * 8);
-    dst = (q == 0) ? (t + 1) : (q == 1) ? (91 + t) : (q == 2) ? ((t + 1) * 10) : ((t + 1) * 10 + 9);
-    const bool gh = tr_ntype(T, f) == T_GHOST;
-    hok = nb >= 0 && !(ghost_zero && gh);  // x = 0 outside the grid and on ghosts in the down-sweep
-    const int ln = hok ? nb : T.self;
-    hb = load_q_raw(R + size_t(ln) * 512 + src_pl * 4);
-    hd = *reinterpret_cast<const float4*>(c.diag + size_t(ln) * 512 + src_pl * 4);
-  }
-  // k halos: cell (i,j,7) of the z- neighbour and (i,j,0) of the z+ neighbour;
-  // their value after the first pass is 0 unless they are colour-0 cells
-  const int nzm = T.nbr[2], nzp = T.nbr[5];
-  const bool kokm = nzm >= 0 && !(ghost_zero && tr_ntype(T, 2) == T_GHOST) && ((i + j + 7) & 1) == 0;
-  const bool kokp = nzp >= 0 && !(ghost_zero && tr_ntype(T, 5) == T_GHOST) && ((i + j) & 1) == 0;
-  const int lzm = nzm >= 0 ? nzm : T.self, lzp = nzp >= 0 ? nzp : T.self;
-  typename RawV<V>::S kbm = load_s_raw(R + size_t(lzm) * 512 + split_cell(i, j, 7));
-  typename RawV<V>::S kbp = load_s_raw(R + size_t(lzp) * 512 + split_cell(i, j, 0));
-  float kdm = c.diag[size_t(lzm) * 512 + split_cell(i, j, 7)];
-  float kdp = c.diag[size_t(lzp) * 512 + split_cell(i, j, 0)];
+  // halo ring of the colour-1 pass: lanes 0..31, the colour-0 quad of one
+  // neighbour pencil; x = 0 outside the grid and on ghosts in the down-sweep
+  // (rhs and diagonal from the zero page)
+  const int q = (lane >> 3) & 3, t = lane & 7, f = ring_face(q);
+  const int nb = pick4(q, uni(T.nbr[0]), uni(T.nbr[3]), uni(T.nbr[1]), uni(T.nbr[4]));
+  const int src = ring_src(q, t) * 4;
+  const bool hok = lane < 32 && nb >= 0 && !(ghost_zero && tr_ntype(T, f) == T_GHOST);
+  typename RawV<V>::Q hb = load_q_raw(hok ? R + size_t(nb) * 512 + src : zp);
+  float4 hd = *reinterpret_cast<const float4*>(hok && !std_faces ? c.diag + size_t(nb) * 512 + src : zf);
+  // k halo of the colour-1 pass: cell (i,j,7) of the z- neighbour (i + j odd) or
+  // (i,j,0) of the z+ one (i + j even), a colour-0 cell either way
+  const bool p0 = ((i + j) & 1) != 0, p1 = !p0;
+  const int nz = p1 ? uni(T.nbr[5]) : uni(T.nbr[2]);
+  const bool kok = nz >= 0 && !(ghost_zero && tr_ntype(T, p1 ? 5 : 2) == T_GHOST);
+  const int kcell = lane * 4 + (p1 ? 0 : 3);
+  typename RawV<V>::S kb = load_s_raw(kok ? R + size_t(nz) * 512 + kcell : zp);
+  float kd = *(kok && !std_faces ? c.diag + size_t(nz) * 512 + kcell : zf);
   hold(rb0);
   hold(rb1);
   hold(hb);
@@ -1602,32 +1549,36 @@ __global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ lis
   hold_f(hd.y);
   hold_f(hd.z);
   hold_f(hd.w);
-  hold(kbm);
-  hold(kbp);
-  hold_f(kdm);
-  hold_f(kdp);
-  if (!hok) hd = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (!kokm) kdm = 0.f;
-  if (!kokp) kdp = 0.f;
+  hold(kb);
+  hold_f(kd);
   // ---- pass 1: the tile's colour-0 cells from x = 0 (gs_quad as the colour-0 pass runs it)
+  const GsCoef G = gs_coef(T);
   const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool p0 = ((i + j) & 1) != 0, p1 = !p0;
-  const float4 n0 = gs_quad(z4, z4, z4, z4, z4, z4, 0.f, 0.f, quad_f<V>(rb0), quad_mask(mask, p0), T.bc, T.h, i, j, p0);
+  const float4 n0 = gs_quad<true>(z4, z4, z4, z4, z4, z4, 0.f, quad_f<V>(rb0), mq0, G, i, j, p0);
   const float4 xr = make_float4(vround<V>(n0.x), vround<V>(n0.y), vround<V>(n0.z), vround<V>(n0.w));
-  // the halo's colour-0 values as that pass leaves them
+  // the halo's colour-0 values as that pass leaves them (a value that counts as
+  // 0 has rhs 0)
   const float4 hbf = quad_f<V>(hb);
-  const float4 hv = make_float4(first_red<V>(hbf.x, hd.x), first_red<V>(hbf.y, hd.y), first_red<V>(hbf.z, hd.z),
-                                first_red<V>(hbf.w, hd.w));
-  const float xkm = first_red<V>(single_f<V>(kbm), kdm);
-  const float xkp = first_red<V>(single_f<V>(kbp), kdp);
+  const float bk = single_f<V>(kb);
+  float4 hv;
+  float xk;
+  if (std_faces) {
+    hv = make_float4(first_red_by<V>(hbf.x, T.rdiag), first_red_by<V>(hbf.y, T.rdiag), first_red_by<V>(hbf.z, T.rdiag),
+                     first_red_by<V>(hbf.w, T.rdiag));
+    xk = first_red_by<V>(bk, T.rdiag);
+  } else {
+    hv = make_float4(first_red<V>(hbf.x, hd.x), first_red<V>(hbf.y, hd.y), first_red<V>(hbf.z, hd.z),
+                     first_red<V>(hbf.w, hd.w));
+    xk = first_red<V>(bk, kd);
+  }
   L.xo[(i + 1) * 10 + (j + 1)] = xr;
-  if (lane < 32) L.xo[dst] = hv;
+  if (lane < 32) L.xo[ring_dst(q, t)] = hv;
   wave_sync();
   if ((flags & F_CHECK_DONE) && done) return;
   // ---- pass 2: colour 1, its own values 0 before the update
   const int pc = (i + 1) * 10 + (j + 1);
-  const float4 n1 = gs_quad(z4, xr, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], xkm, xkp,
-                            quad_f<V>(rb1), quad_mask(mask, p1), T.bc, T.h, i, j, p1);
+  const float4 n1 = gs_quad(z4, xr, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], xk, quad_f<V>(rb1), mq1,
+                            G, i, j, p1);
   V* tile = X + size_t(T.self) * 512;
   store4(tile + lane * 4, xr);
   store4(tile + 256 + lane * 4, n1);
@@ -1635,49 +1586,6 @@ __global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ lis
 
 #include "gs_pair.hpp"
 
-// The same pass with every global load issued first, as raw bits (own pencil,
-// parent quad, face masks, halo pencils and their parents' quads, k halos, rhs,
-// done flag) and one wait before the values are formed.  Missing neighbours
-// and lanes 32..63 read the tile itself and its parent (values dropped), so no
-// load sits in a branch.  Faster on small levels, where each launch waits on
-// memory latency; slower on big ones (more loads and registers), so the host
-// picks it by level size.  Every value is the one tile_gs_prolong forms.
-template <class V>
-struct KHaloRaw {
-  uint32_t mv;
-  typename RawV<V>::S pz, xo;
-};
-// The raw loads of one prolongated k-halo value: face mask, parent value and
-// down-sweep value of cell (i,j,KN) of face neighbour F, each from the zero
-// page where it does not exist (no neighbour, a ghost neighbour's down-sweep
-// value, a ghost tile's own stage).
-template <int F, int KN, class V>
-__device__ __forceinline__ KHaloRaw<V> khalo_prolong_issue(const Ctx& c, const TileRec& T, const V* XD, const V* XO,
-                                                           int oct, int lane, bool skip) {
-  KHaloRaw<V> k;
-  const int n = T.nbr[F];
-  const bool gh = tr_ntype(T, F) == T_GHOST;
-  const bool ok = !skip && n >= 0;
-  const V* zp = zero_page<V>();
-  const int i = lane >> 3, j = lane & 7;
-  k.mv = (ok ? c.fmask + size_t(n) * 512 + lane * 8 : reinterpret_cast<const uint8_t*>(zp))[ok ? KN : 0];
-  const int noct = oct ^ 4;
-  const int ox = noct & 1, oy = (noct >> 1) & 1, oz = (noct >> 2) & 1;
-  k.pz = load_s_raw(ok ? XO + size_t(T.nbr_parent[F]) * 512 +
-                             split_cell(ox * 4 + (i >> 1), oy * 4 + (j >> 1), oz * 4 + (KN >> 1))
-                       : zp);
-  k.xo = load_s_raw(ok && !gh ? XD + size_t(n) * 512 + split_cell(i, j, KN) : zp);
-  return k;
-}
-// khalo_prolong's value from the raw loads (a missing neighbour's zero mask
-// gives 0)
-template <int F, class V>
-__device__ __forceinline__ float khalo_prolong_value(const TileRec& T, KHaloRaw<V> k, float pcoef) {
-  const bool gh = tr_ntype(T, F) == T_GHOST;
-  const float pz = single_f<V>(k.pz);
-  const float xo = single_f<V>(k.xo);
-  return (k.mv & M_INT) ? vround<V>(gh ? pz : __builtin_fmaf(pcoef, pz, xo)) : 0.f;
-}
 template <class V> struct RawQuadS { typename RawV<V>::S2 h0, h1; };
 template <class V>
 __device__ __forceinline__ RawQuadS<V> load_quad_split_raw(const V* __restrict__ tile, int pl, int K0) {
@@ -1694,105 +1602,112 @@ __device__ __forceinline__ float4 quad_split_f(const RawQuadS<V>& r, int pl) {
   const float2 E = q0 ? h1 : h0, O = q0 ? h0 : h1;
   return make_float4(E.x, O.x, E.y, O.y);
 }
+// The prolongated values of a pencil's four cells of one colour (split quad): x +
+// pcoef * parent on INTERIOR cells of active tiles, the parent value on those of
+// GHOST tiles, 0 elsewhere, rounded as a store to V-typed memory would leave
+// them.  Cells k = 2 e and 2 e + 1 have parent cell e, so a quad of either colour
+// lines up with the parent quad; m: the quad's face masks (their INTERIOR bits).
 template <class V>
-__device__ __forceinline__ void tile_gs_prolong_eager(const Ctx& c, const TileRec& T, const V* XD, V* XO, float pcoef,
-                                                      int color, int flags, TileLDS& L) {
+__device__ __forceinline__ float4 prolong_quad(float4 x, float4 pq, uint32_t m, bool ghost, float pcoef) {
+  auto one = [&](float xv, float pv, int e) {
+    return ((m >> (8 * e)) & M_INT) ? vround<V>(ghost ? pv : __builtin_fmaf(pcoef, pv, xv)) : 0.f;
+  };
+  return make_float4(one(x.x, pq.x, 0), one(x.y, pq.y, 1), one(x.z, pq.z, 2), one(x.w, pq.w, 3));
+}
+
+// Prolongation fused into the first colour pass of the up-sweep on a level
+// (GMGSolver.cu:345-376 then :216-269): every value the pass reads -- the tile's
+// cells and the other-colour halo -- is formed on the fly as the prolongation
+// would leave it, so no separate launch is needed.  XD holds the down-sweep
+// values, XO receives the level's result; GHOST tiles in the list only store
+// their prolongated values.
+// Every load is issued before the first wait (what does not exist comes from the
+// zero page), and the pass works on colour-split quads throughout: of a
+// neighbour pencil only the four cells the update reads are formed, of the two k
+// halos the one the lane's cells reach, and only the updated colour's rhs is read
+// (2.5 s + t + s/8 bytes a cell, s the stored size, instead of 3 s + t + s/8).
+// The 532,926-tile level of the 256-problem pool in FP32 769 -> 649 us, in
+// bfloat16 469 -> 366; the refined 45,054-tile scene's in bfloat16 34.3 -> 26.2;
+// a level of 64 tiles 3.72 -> 2.85.
+template <class V>
+__global__ __launch_bounds__(64) void k_gs_prolong(const TileRec* __restrict__ list, int n, int flags, const V* XD, V* XO,
+                                                   float pcoef, int color, Ctx c) {
+  TILE_KERNEL_PROLOGUE_C
+  SKIP_INERT
+  __shared__ GsLDS L;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const int oct = tr_octant(T);
   const bool own_ghost = tr_type(T) == T_GHOST;
   const V* zp = zero_page<V>();
-  // ---- loads, none in a branch (values that do not exist come from the zero page)
+  const uint32_t* zw = reinterpret_cast<const uint32_t*>(kZeroPage);
+  const int hc = color << 8, ho = hc ^ 256;
+  const bool p = ((color + i + j) & 1) != 0;
+  // the parent pencil of pencil (a,b) of a child in octant o
+  auto parent_pencil = [](int o, int a, int b) { return ((o & 1) * 4 + (a >> 1)) * 8 + ((o >> 1) & 1) * 4 + (b >> 1); };
   const int32_t* dp = (flags & F_CHECK_DONE) ? &c.ps[T.prob].done : reinterpret_cast<const int32_t*>(c.fmask);
   const int32_t done = *dp;
-  const uint64_t mown = load_ct8(own_masks(c, T) + lane * 8);
-  const int ppl = ((oct & 1) * 4 + (i >> 1)) * 8 + (((oct >> 1) & 1) * 4 + (j >> 1));  // parent pencil
+  const uint32_t* masks = own_split_masks(c, T);
+  const uint32_t mc = masks[(hc >> 2) + lane], mo = masks[(ho >> 2) + lane];
+  const int ppl = parent_pencil(oct, i, j);
   RawQuadS<V> rpq = load_quad_split_raw(XO + size_t(T.parent) * 512, ppl, ((oct >> 2) & 1) * 4);
-  RawPencil<V> rown = load_pencil_split_raw(own_ghost ? zp : XD + size_t(T.self) * 512, lane);
-  RawPencil<V> rrhs = load_pencil_split_raw(own_ghost ? zp : vc_rhs<V>(c) + size_t(T.self) * 512, lane);
-  // halo ring of lanes 0..31 as in tile_gs_prolong; every lane loads
-  const int g = (lane >> 3) & 3, t = lane & 7;
-  const int f = ring_face(g);
+  const V* xd = own_ghost ? zp : XD + size_t(T.self) * 512;
+  typename RawV<V>::Q rxc = load_q_raw(xd + hc + lane * 4);
+  typename RawV<V>::Q rxo = load_q_raw(xd + ho + lane * 4);
+  typename RawV<V>::Q rB = load_q_raw((own_ghost ? zp : vc_rhs<V>(c) + size_t(T.self) * 512) + hc + lane * 4);
+  // halo ring of lanes 0..31 (x = 0 outside the grid: a missing neighbour's zero
+  // masks make every value 0)
+  const int g = (lane >> 3) & 3, t = lane & 7, f = ring_face(g);
   const int hn = pick4(g, uni(T.nbr[0]), uni(T.nbr[3]), uni(T.nbr[1]), uni(T.nbr[4]));
   const int pn = pick4(g, uni(T.nbr_parent[0]), uni(T.nbr_parent[3]), uni(T.nbr_parent[1]), uni(T.nbr_parent[4]));
-  const int ni = pick4(g, 7, 0, t, t), nj = pick4(g, t, t, 7, 0);  // pencil in the neighbour
-  const int noct = oct ^ (1 << (f % 3));
-  const int hpl = ni * 8 + nj;
-  const int hppl = ((noct & 1) * 4 + (ni >> 1)) * 8 + (((noct >> 1) & 1) * 4 + (nj >> 1));
+  const int hpl = ring_src(g, t), noct = oct ^ (g < 2 ? 1 : 2);
+  const int hppl = parent_pencil(noct, hpl >> 3, hpl & 7);
   const bool hgh = tr_ntype(T, f) == T_GHOST;
   const bool hok = !own_ghost && lane < 32 && hn >= 0;
-  const uint64_t hw = load_ct8(hok ? c.fmask + size_t(hn) * 512 + hpl * 8 : reinterpret_cast<const uint8_t*>(zp));
-  RawPencil<V> rh = load_pencil_split_raw(hok && !hgh ? XD + size_t(hn) * 512 : zp, hpl);
+  uint32_t hm = *(hok ? c.fsplit + size_t(hn) * 128 + (ho >> 2) + hpl : zw);
+  typename RawV<V>::Q rh = load_q_raw(hok && !hgh ? XD + size_t(hn) * 512 + ho + hpl * 4 : zp);
   RawQuadS<V> rhpq = load_quad_split_raw(hok ? XO + size_t(pn) * 512 : zp, hppl, ((noct >> 2) & 1) * 4);
-  KHaloRaw<V> km = khalo_prolong_issue<2, 7>(c, T, XD, XO, oct, lane, own_ghost);
-  KHaloRaw<V> kp = khalo_prolong_issue<5, 0>(c, T, XD, XO, oct, lane, own_ghost);
-  // ---- one wait, then the values
+  // k halo: cell (i,j,7) of the z- neighbour (p = 0) or (i,j,0) of the z+ one
+  const int kn = p ? uni(T.nbr[5]) : uni(T.nbr[2]), kpn = p ? uni(T.nbr_parent[5]) : uni(T.nbr_parent[2]);
+  const bool kgh = tr_ntype(T, p ? 5 : 2) == T_GHOST;
+  const bool kok = !own_ghost && kn >= 0;
+  const int kcell = ho + lane * 4 + (p ? 0 : 3);
+  const int kpl = parent_pencil(oct ^ 4, i, j);
+  const int kpcell = split_cell(kpl >> 3, kpl & 7, (((oct ^ 4) >> 2) & 1) * 4 + (p ? 0 : 3));
+  uint32_t km = *(kok ? reinterpret_cast<const uint8_t*>(c.fsplit) + size_t(kn) * 512 + kcell
+                      : reinterpret_cast<const uint8_t*>(zw));
+  typename RawV<V>::S rkp = load_s_raw(kok ? XO + size_t(kpn) * 512 + kpcell : zp);
+  typename RawV<V>::S rkx = load_s_raw(kok && !kgh ? XD + size_t(kn) * 512 + kcell : zp);
   hold_all(rpq.h0);
   hold_all(rpq.h1);
-  hold_all(rown);
-  hold_all(rrhs);
+  hold_all(rxc);
+  hold_all(rxo);
+  hold_all(rB);
   hold_all(rh);
   hold_all(rhpq.h0);
   hold_all(rhpq.h1);
-  hold_all(km.mv);
-  hold_all(km.pz);
-  hold_all(km.xo);
-  hold_all(kp.mv);
-  hold_all(kp.pz);
-  hold_all(kp.xo);
-  float4 xa, xb;
-  pencil_split_f(rown, lane, xa, xb);
-  float4 oa, ob;
-  prolong_pencil<V>(xa, xb, quad_split_f(rpq, ppl), mown, own_ghost, pcoef, oa, ob);
-  if (own_ghost) {  // GHOST tile: its prolongated values only
-    if ((flags & F_CHECK_DONE) && done) return;
-    store_pencil_split(XO + size_t(T.self) * 512, lane, oa, ob);
+  hold_all(hm);
+  hold_all(km);
+  hold_all(rkp);
+  hold_all(rkx);
+  if ((flags & F_CHECK_DONE) && done) return;
+  const float4 pq = quad_split_f(rpq, ppl);
+  const float4 vc = prolong_quad<V>(quad_f<V>(rxc), pq, mc, own_ghost, pcoef);
+  const float4 vo = prolong_quad<V>(quad_f<V>(rxo), pq, mo, own_ghost, pcoef);
+  V* tile = XO + size_t(T.self) * 512;
+  store4(tile + ho + lane * 4, vo);
+  if (own_ghost) {
+    store4(tile + hc + lane * 4, vc);
     return;
   }
-  Stencil S;
-  S.own[0] = oa.x; S.own[1] = oa.y; S.own[2] = oa.z; S.own[3] = oa.w;
-  S.own[4] = ob.x; S.own[5] = ob.y; S.own[6] = ob.z; S.own[7] = ob.w;
-  S.m = mown;
-  const int pc = (i + 1) * 10 + (j + 1);
-  L.xs[0][pc] = oa;
-  L.xs[1][pc] = ob;
-  if (lane < 32) {
-    // x = 0 outside the grid (GMGSolver.cu:120-122): a missing neighbour's
-    // zero masks make every value 0
-    float4 ya, yb, va, vb;
-    pencil_split_f(rh, hpl, ya, yb);
-    prolong_pencil<V>(ya, yb, quad_split_f(rhpq, hppl), hw, hgh, pcoef, va, vb);
-    L.xs[0][ring_dst(g, t)] = va;
-    L.xs[1][ring_dst(g, t)] = vb;
-  }
-  S.xkm = khalo_prolong_value<2>(T, km, pcoef);
-  S.xkp = khalo_prolong_value<5>(T, kp, pcoef);
-  S.h = T.h;
-  S.b_int = T.bc[6];
-  for (int e = 0; e < 6; e++) S.b_f[e] = T.bc[e];
-  float4 ba, bb;
-  pencil_split_f(rrhs, lane, ba, bb);
-  const float b[8] = {ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, bb.z, bb.w};
-  if ((flags & F_CHECK_DONE) && done) return;
+  L.xo[(i + 1) * 10 + (j + 1)] = vo;
+  if (lane < 32)
+    L.xo[ring_dst(g, t)] = prolong_quad<V>(quad_f<V>(rh), quad_split_f(rhpq, hppl), hm, hgh, pcoef);
+  const float kp = single_f<V>(rkp);
+  const float xk = (km & M_INT) ? vround<V>(kgh ? kp : __builtin_fmaf(pcoef, kp, single_f<V>(rkx))) : 0.f;
   wave_sync();
-  float4 out0, out1;
-  gs_pencil(lds_nbrs(L), S, b, color, out0, out1);
-  store_pencil_split(XO + size_t(T.self) * 512, lane, out0, out1);
-}
-template <class V>
-__global__ __launch_bounds__(64) void k_gs_prolong_eager(const TileRec* __restrict__ list, int n, int flags,
-                                                         const V* XD, V* XO, float pcoef, int color, Ctx c) {
-  TILE_KERNEL_PROLOGUE_C
-  SKIP_INERT
-  __shared__ TileLDS L;
-  tile_gs_prolong_eager(c, T, XD, XO, pcoef, color, flags, L);
-}
-template <class V>
-__global__ __launch_bounds__(64) void k_gs_prolong(const TileRec* __restrict__ list, int n, int flags, const V* XD,
-                                                   V* XO, float pcoef, int color, Ctx c) {
-  TILE_KERNEL_PROLOGUE_C
-  SKIP_INERT
-  __shared__ TileLDS L;
-  tile_gs_prolong(c, T, XD, XO, pcoef, color, flags, L);
+  const int pc = (i + 1) * 10 + (j + 1);
+  store4(tile + hc + lane * 4, gs_quad(vc, vo, L.xo[pc - 10], L.xo[pc + 10], L.xo[pc - 1], L.xo[pc + 1], xk, quad_f<V>(rB),
+                                       mc, gs_coef(T), i, j, p));
 }
 template <class V>
 __global__ __launch_bounds__(64) void k_jacobi(const TileRec* __restrict__ list, int n, int flags, int level,
@@ -1802,14 +1717,14 @@ __global__ __launch_bounds__(64) void k_jacobi(const TileRec* __restrict__ list,
   __shared__ TileLDS L;
   tile_jacobi(c, T, level, X, XG, Y, F, omega, flags, L);
 }
-template <class V, bool EAGER = false>
+template <class V>
 __global__ __launch_bounds__(64) void k_restrict(const TileRec* __restrict__ list, int n, int flags, int level,
                                                  const V* X, const V* F, V* CO, float one_over_alpha, Ctx c) {
   TILE_KERNEL_PROLOGUE_C
   SKIP_INERT
   __shared__ TileLDS L;
   __shared__ float res[512];
-  tile_restrict<V, EAGER>(c, T, level, X, F, CO, one_over_alpha, flags, L, res);
+  tile_restrict<V>(c, T, level, X, F, CO, one_over_alpha, flags, L, res);
 }
 template <class V>
 __global__ __launch_bounds__(64) void k_prolong(const TileRec* __restrict__ list, int n, int flags, int level,
@@ -1863,24 +1778,6 @@ struct CoarseLDS {
   float t[CL_CHILDREN * 512];   // level 1: residuals (restriction) or new values (damped Jacobi)
   float b0[CL_ROOTS * 512];     // V-cycle rhs of level 0
 };
-
-// The quotient a / d, correctly rounded, from rd = 1/d in FP64 (within 2^-51
-// of it): the product's relative error is below 2^-50, and a quotient of two
-// 24-bit significands lies at least 2^-49 (relative) from every rounding
-// boundary of FP32, so the conversion rounds to the same value (results below
-// 2^-126, where FP32 has fewer bits, within one unit of their last place).
-// 4 issue slots against 15.5 for the FP32 division on gfx950.
-__device__ __forceinline__ float div_by(float a, double rd) { return float(double(a) * rd); }
-// 1/d in FP64 for finite d != 0: the FP32 reciprocal and two Newton steps (a
-// divisor beyond the range where that reciprocal is a normal number: the division).
-__device__ __forceinline__ double recip64(float d) {
-  const double dd = double(d);
-  const float a = __builtin_fabsf(d);
-  if (!(a >= 0x1p-100f && a <= 0x1p100f)) return 1.0 / dd;
-  double y = double(__builtin_amdgcn_rcpf(d));
-  y = __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
-  return __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
-}
 
 // One cell of a level: LDS byte addresses of its six neighbours (faces x-, x+,
 // y-, y+, z-, z+; CL_ZERO outside the grid, the cell itself across a face cut by
@@ -2391,7 +2288,14 @@ __global__ __launch_bounds__(64) void k_apply(const TileRec* __restrict__ list, 
   __shared__ float gl[512];
   Stencil S;
   float bcv[7];
-  view_coeffs(T, sl, bcv);
+  if (PG) {
+    // the view of LEAF and GHOST tiles with no subtree level, from the record's
+    // (its level's): the same but for NONLEAF neighbours, which count there as LEAF
+    for (int f = 0; f < 6; f++) bcv[f] = tr_ntype(T, f) == T_NONLEAF ? 0.f : T.bc[f];
+    bcv[6] = T.bc[6];
+  } else {
+    view_coeffs(T, sl, bcv);
+  }
   if (PG) {
     StagePG r = stage_issue_pg(c, T, X);
     stage_commit_pg(r, T, bcv, L, S);
@@ -2401,8 +2305,8 @@ __global__ __launch_bounds__(64) void k_apply(const TileRec* __restrict__ list, 
   if (prob_done(c, T, flags)) return;
   wave_sync();
   float ax[8], dg[8];
-  if (diag) apply_pencil<false, true>(lds_nbrs(L), S, dg, ax);
-  else apply_pencil<true, false>(lds_nbrs(L), S, ax, dg);
+  if (diag) apply_pencil<false, true>(L, S, dg, ax);
+  else apply_pencil<true, false>(L, S, ax, dg);
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   if (tr_type(T) == T_GHOST && dot) {
@@ -2432,7 +2336,7 @@ __global__ __launch_bounds__(64) void k_ghost_gather(const TileRec* __restrict__
   float4 e[2];
   int gs[2];
   for (int h = 0; h < 2; h++) {
-    gs[h] = list[w].gcs[(i >> 2) | ((j >> 2) << 1) | (h << 2)];  // lane-dependent index: read from memory
+    gs[h] = c.kids[T.gslot].slot[(i >> 2) | ((j >> 2) << 1) | (h << 2)];
     if (gs[h] >= 0) e[h] = *reinterpret_cast<const float4*>(c.gsum + size_t(gs[h]) * 64 + (i & 3) * 16 + (j & 3) * 4);
   }
   if (prob_done(c, T, flags)) return;
@@ -3047,9 +2951,10 @@ __global__ __launch_bounds__(64) void k_amg_restrict(const TileRec* __restrict__
 __global__ __launch_bounds__(64) void k_amg_leaf_rhs(const TileRec* __restrict__ list, int n, int flags,
                                                      const float* __restrict__ TMP, const float* __restrict__ F,
                                                      float* __restrict__ RHS, Ctx c) {
-  TILE_KERNEL_PROLOGUE_ALL
+  TILE_KERNEL_PROLOGUE_C
   const uint8_t ty = tr_type(T);
   if (ty == T_NONLEAF || prob_done(c, T, flags)) return;
+  const GhostKids* kids = tr_has_gchild(T) ? c.kids + T.gslot : nullptr;
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t b = size_t(T.self) * 512 + lane * 8;
   float out[8];
@@ -3060,9 +2965,7 @@ __global__ __launch_bounds__(64) void k_amg_leaf_rhs(const TileRec* __restrict__
     load8(F + b, f);
     for (int k = 0; k < 8; k++) {
       const int o = (i >> 2) | ((j >> 2) << 1) | ((k >> 2) << 2);
-      // the ghost child of octant o, by register selects (no indexed private array)
-      const int g = (o & 4) ? ((o & 2) ? ((o & 1) ? T.gch[7] : T.gch[6]) : ((o & 1) ? T.gch[5] : T.gch[4]))
-                            : ((o & 2) ? ((o & 1) ? T.gch[3] : T.gch[2]) : ((o & 1) ? T.gch[1] : T.gch[0]));
+      const int g = kids ? kids->tile[o] : -1;  // the ghost child of octant o
       float sum = 0.f;
       if (g >= 0)
         for (int cid = 0; cid < 8; cid++)
@@ -3688,8 +3591,11 @@ __device__ __forceinline__ void tile_accumulate_children(const Ctx& c, const Til
   load8(X + base, x);
   // ghost children of the pencil's two octants (k 0..3, k 4..7)
   const int o0 = (i >> 2) | ((j >> 2) << 1);
-  const int g[2] = {pick4(o0, uni(T.gch[0]), uni(T.gch[1]), uni(T.gch[2]), uni(T.gch[3])),
-                    pick4(o0, uni(T.gch[4]), uni(T.gch[5]), uni(T.gch[6]), uni(T.gch[7]))};
+  int g[2] = {-1, -1};
+  if (tr_has_gchild(T)) {
+    g[0] = c.kids[T.gslot].tile[o0];
+    g[1] = c.kids[T.gslot].tile[4 + o0];
+  }
   float fv[2][2][2][8];  // [oz][ii][jj][fine k]
   uint8_t fc[2][2][2][8];
 #pragma unroll
@@ -3725,7 +3631,7 @@ __device__ __forceinline__ void tile_accumulate_children(const Ctx& c, const Til
 __global__ __launch_bounds__(64) void k_accumulate_children(Ctx c, const TileRec* __restrict__ list, int n,
                                                             float* __restrict__ X, uint8_t mask, float coeff) {
   const int flags = 0;
-  TILE_KERNEL_PROLOGUE_ALL
+  TILE_KERNEL_PROLOGUE_C
   tile_accumulate_children(c, T, X, mask, coeff);
 }
 // The same for the three face-velocity channels in one launch (one after the
@@ -3733,7 +3639,7 @@ __global__ __launch_bounds__(64) void k_accumulate_children(Ctx c, const TileRec
 __global__ __launch_bounds__(64) void k_accumulate_children_vel(Ctx c, const TileRec* __restrict__ list, int n, Vel U,
                                                                 uint8_t mask, float coeff) {
   const int flags = 0;
-  TILE_KERNEL_PROLOGUE_ALL
+  TILE_KERNEL_PROLOGUE_C
   for (int a = 0; a < 3; a++) tile_accumulate_children(c, T, U.u[a], mask, coeff);
 }
 

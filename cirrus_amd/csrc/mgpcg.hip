@@ -83,6 +83,7 @@ struct cg_problem {
   std::vector<int> leaf_count;   // per problem: LEAF tiles
   std::vector<int> coarse_C;     // per problem: deepest LDS-resident level (-1: none)
   std::vector<TileRec> tiles;    // one record per tile (internal order)
+  std::vector<GhostKids> kids;   // by ghost slot (build only)
   DList leaf, gather, applyl, ghosts, all;
   std::vector<DList> act, lvl;   // per level, all problems (operator API)
   std::vector<DList> actg, lvlg; // per level, tiles the V-cycle smooths with grid-wide launches
@@ -94,8 +95,7 @@ struct cg_problem {
   bool rz_in_vcycle = false;     // every LEAF tile is on a grid-wide level >= 1 (its up-sweep can sum r.z)
   int gs_block = 1;
   int device = 0;           // the HIP device current when the handle was created
-  int eager_max = 16384;    // levels of at most this many tiles: every load before one wait (prolongation pass, restriction)
-  int fused16_max = 16384;  // 16-bit levels of at most this many tiles: first down-sweep iteration in one launch
+  int fused16_max = INT32_MAX;  // 16-bit levels of at most this many tiles: first down-sweep iteration in one launch
   int gs_pair = 0;          // RB-GS iterations after the first as one launch (k_gs_pair; needs d_tiles; slower, off)
   std::vector<int> lev, tbase, coarse_auto;
   std::vector<uint8_t> ty;
@@ -121,6 +121,7 @@ struct cg_problem {
   float* d_api[3] = {nullptr, nullptr, nullptr};  // colour-split copies of channels for the operator API
   float* d_vel[3] = {nullptr, nullptr, nullptr};  // face velocities u, v, w (channels 6-8, allocated on first use)
   float* d_gsum = nullptr;
+  GhostKids* d_kids = nullptr;   // by ghost slot (behind d_gsum in its allocation)
   ProbState* d_ps = nullptr;
   int32_t* d_dflag = nullptr;
   const int32_t* d_pmap = nullptr;  // finalize workgroup -> problem (pools whose problems are a subset)
@@ -164,6 +165,7 @@ struct cg_problem {
     c.rhsvf = reinterpret_cast<f16*>(d_rhsvh);
     c.zbf = reinterpret_cast<f16*>(d_zbh);
     c.gsum = d_gsum;
+    c.kids = d_kids;
     c.ps = d_ps;
     c.dflag = d_dflag;
     c.pmap = d_pmap;
@@ -221,6 +223,7 @@ struct TreeBuild {
   std::vector<TileRec> tiles;
   std::vector<int> ext, lev;
   std::vector<uint8_t> ty;
+  std::vector<GhostKids> kids;  // by local ghost slot (the first child's)
   int nleaf = 0, nghost = 0;
 };
 void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int ghost_base, TreeBuild& B) {
@@ -275,6 +278,9 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
   }
   B.nleaf = nleaf;
   B.nghost = nghost;
+  GhostKids none;
+  for (int o = 0; o < 8; o++) none.tile[o] = none.slot[o] = -1;
+  B.kids.assign(nghost, none);
   if (nleaf == 0) fail(CG_ERR_INVALID, "tree has no LEAF tiles");
   for (int i = 0; i < n; i++) {
     TileRec& T = B.tiles[i];
@@ -305,7 +311,6 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
     T.self = base + i;
     T.h = float(d->h0 / double(1u << l));
     T.meta = uint32_t(l) | (uint32_t(my) << 8) | (octant << 16);
-    for (int o = 0; o < 8; o++) { T.gch[o] = -1; T.gcs[o] = -1; }
     if (my != GHOST) {
       for (int o = 0; o < 8; o++) {
         const int ch = find(l + 1, 2 * cd[i][0] + (o & 1), 2 * cd[i][1] + ((o >> 1) & 1), 2 * cd[i][2] + ((o >> 2) & 1));
@@ -313,14 +318,35 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
           fail(CG_ERR_INVALID, "a NONLEAF tile must have 8 LEAF/NONLEAF children");
         if (my == LEAF && ch >= 0) {
           if (ty[ch] != GHOST) fail(CG_ERR_INVALID, "a LEAF tile can only have GHOST children");
-          T.gch[o] = base + ch;
-          T.gcs[o] = gslot[ch];
-          T.meta |= 1u << 24;
+          if (T.gslot < 0) {
+            T.gslot = gslot[ch];
+            T.meta |= 1u << 24;
+          }
+          GhostKids& kids = B.kids[T.gslot - ghost_base];
+          kids.tile[o] = base + ch;
+          kids.slot[o] = gslot[ch];
         }
       }
     }
     // smoothing-view coefficients (subtree at the tile's own level)
     view_coeffs(T, l, T.bc);
+    // the sweep's diagonal of a cell with six inside coefficients, summed as the
+    // kernels sum it, and its reciprocal
+    T.h3 = (T.h * T.h) * T.h;
+    if (my != GHOST) {
+      const float ci = T.bc[6];
+      float d = 0.f;
+      for (int e = 0; e < 6; e++) d = d + ci;
+      d = ((d * T.h) * T.h) * T.h;
+      bool uniform = d != 0.f;
+      for (int f = 0; f < 6; f++) uniform = uniform && T.bc[f] == ci;
+      T.rdiag = d != 0.f ? 1.0 / double(d) : 0.0;
+      if (uniform) T.meta |= 1u << 28;
+    }
+    // a power of two whose third power is a normal number
+    uint32_t hb;
+    std::memcpy(&hb, &T.h, 4);
+    if ((hb & 0x7fffffu) == 0 && T.h > 0x1p-40f && T.h < 0x1p40f) T.meta |= 1u << 29;
     // the cell types as 64 words of 8 cells (cell index i*64 + j*8 + k)
     constexpr uint64_t kOnes = 0x0101010101010101ull;
     auto words = [&](int t) {
@@ -359,7 +385,11 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
   }
   for (int i = 0; i < n; i++) {
     TileRec& T = B.tiles[i];
-    for (int f = 0; f < 6; f++) T.nbr_parent[f] = T.nbr[f] < 0 ? -1 : B.tiles[T.nbr[f] - base].parent;
+    for (int f = 0; f < 6; f++) {
+      const TileRec* N = T.nbr[f] < 0 ? nullptr : &B.tiles[T.nbr[f] - base];
+      T.nbr_parent[f] = N ? N->parent : -1;
+      if (!N || tr_type(*N) == T_GHOST || (tr_all_open(*N) && tr_uniform(*N))) T.ntypes |= 1u << (24 + f);
+    }
   }
 }
 
@@ -539,6 +569,7 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
     leaf_base[q + 1] = leaf_base[q] + nl;
     ghost_base[q + 1] = ghost_base[q] + ng;
   }
+  P.kids.resize(ghost_base[nprob]);
   auto build_one = [&](int q) {
     TreeBuild B;
     build_tree(&descs[q], q, tbase[q], leaf_base[q], ghost_base[q], B);
@@ -548,6 +579,7 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
       lev[tbase[q] + i] = B.lev[i];
       ty[tbase[q] + i] = B.ty[i];
     }
+    std::copy(B.kids.begin(), B.kids.end(), P.kids.begin() + ghost_base[q]);
     P.leaf_begin[q] = leaf_base[q];
     P.leaf_count[q] = B.nleaf;
     P.coarse_C[q] = coarse_depth(B.lev, B.ty);
@@ -609,9 +641,12 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
   HIPC(hipMemsetAsync(P.d_zb, 0, cells * sizeof(float), P.stream));
   HIPC(hipMalloc(&P.d_inert, size_t(n)));
   HIPC(hipMemsetAsync(P.d_inert, 0, size_t(n), P.stream));
-  size_t g64 = size_t(std::max(1, ghost_total)) * 64 * sizeof(float);
-  HIPC(hipMalloc(&P.d_gsum, g64));
+  const size_t g64 = size_t(std::max(1, ghost_total)) * 64 * sizeof(float);
+  HIPC(hipMalloc(&P.d_gsum, g64 + size_t(ghost_total) * sizeof(GhostKids)));
   HIPC(hipMemsetAsync(P.d_gsum, 0, g64, P.stream));
+  P.d_kids = reinterpret_cast<GhostKids*>(reinterpret_cast<char*>(P.d_gsum) + g64);
+  if (ghost_total)
+    HIPC(hipMemcpyAsync(P.d_kids, P.kids.data(), sizeof(GhostKids) * size_t(ghost_total), hipMemcpyHostToDevice, P.stream));
   HIPC(hipMalloc(&P.d_ps, sizeof(ProbState) * nprob));
   HIPC(hipMemsetAsync(P.d_ps, 0, sizeof(ProbState) * nprob, P.stream));
   HIPC(hipMalloc(&P.d_dflag, sizeof(int32_t) * nprob));
@@ -843,16 +878,13 @@ void ensure_bf16(cg_problem& P) {
 // V is the storage type of Z, ZO, the scratch buffer and the V-cycle rhs (R is
 // only a placeholder: in V-cycle mode the rhs comes from the V-cycle rhs array).
 // The fused first iteration (k_gs_first) saves a launch and the first pass's
-// traffic, but reads the halo's diagonals, which no other kernel brings into
-// the cache; with 16-bit storage on a level of many tiles that costs more than
-// the second launch saves (measured on the 256-problem pool), so large 16-bit
-// levels keep the two passes.  Results are the same either way.
-constexpr int kFirstFused16Max = 16384;
-// Levels of at most this many tiles use k_gs_prolong_eager and the eager
-// k_restrict (all loads before one wait: faster where a launch waits on
-// latency, slower on big levels).
-constexpr int kProlongEagerMax = 16384;
-// Both limits are per handle (cg_set_level_forms), defaulting to these.
+// traffic on levels of every size.  With 16-bit storage it used to lose to the
+// two passes beyond 16,384 tiles, by the halo diagonals it read; on tiles with
+// uniform faces it reads none now, and on every level it is the faster form
+// (RB-GS solves in bfloat16, two-pass beyond 16,384 tiles against one launch
+// everywhere: 256 problems 222.1 against 216.6 ms, the 45,054-tile refined scene
+// 49.9 against 49.1 ms).  The limit is per handle (cg_set_level_forms).
+constexpr int kFirstFused16Max = INT32_MAX;
 
 // last_flags is added to the last colour pass of each grid-wide level's
 // up-sweep (RB-GS with nu >= 1), the pass after which that level's z is final.
@@ -896,10 +928,7 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
     }
     const DList& al = P.lvlg[l];
     int fl = base | F_GHOST_ZERO | (v.nu == 0 ? F_ZERO_X : 0);
-    if (al.n > P.eager_max)
-      k_restrict<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
-    else if (al.n)
-      k_restrict<V, true><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
+    if (al.n) k_restrict<V><<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, l, Z, R, nullptr, v.ooa, c);
   }
   launch_coarse<V>(P, c, VCycleArgs{v.nu, v.coarsest, v.smoother, v.omega, v.ooa, v.pcoef}, ZO, base & ~F_SWIZZLE);
   {
@@ -922,10 +951,7 @@ void enqueue_vcycle(cg_problem& P, V* Z, V* ZO, const V* R, const VParams& v, in
     const bool jac = v.smoother != CG_SMOOTH_RBGS;
     if (!jac && v.nu > 0) {
       // prolongation fused into the first (black) pass; the level's result goes to ZO
-      if (al.n > P.eager_max)
-        k_gs_prolong<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, Z, ZO, v.pcoef, 1, c);
-      else if (al.n)
-        k_gs_prolong_eager<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, Z, ZO, v.pcoef, 1, c);
+      if (al.n) k_gs_prolong<V><<<grid_for(al.n, base), 64, 0, P.stream>>>(P.L(al), al.n, base, Z, ZO, v.pcoef, 1, c);
       if (c.tiles == nullptr || v.nu < 2) {
         launch_gs(P, a, c, l, ZO, R, 0, base | (v.nu == 1 ? last_flags : 0));
         for (int s = 1; s < v.nu; s++) {
@@ -1962,7 +1988,7 @@ cg_status cg_set_level_forms(cg_problem* p, int32_t eager_max_tiles, int32_t fus
   return guard([&] {
     if (!p) fail(CG_ERR_INVALID, "null problem");
     if (!p->owner) fail(CG_ERR_INVALID, "cg_set_level_forms: not an owning handle");
-    p->eager_max = eager_max_tiles < 0 ? kProlongEagerMax : eager_max_tiles;
+    (void)eager_max_tiles;  // one form for every size now
     p->fused16_max = fused16_max_tiles < 0 ? kFirstFused16Max : fused16_max_tiles;
     p->gs_pair = pair_sweeps > 0 ? 1 : 0;
     HIPC(hipStreamSynchronize(p->stream));

@@ -141,6 +141,7 @@ struct cg_server {
   bf16* d_rhsvh = nullptr;
   bf16* d_zbh = nullptr;
   float* d_gsum = nullptr;
+  GhostKids* d_kids = nullptr;
   ProbState* d_ps = nullptr;
   int32_t* d_dflag = nullptr;
   int32_t* d_dflag_init = nullptr;
@@ -195,7 +196,7 @@ cg_server::~cg_server() {
   for (auto& row : ev_gtab)
     for (auto e : row) if (e) (void)hipEventDestroy(e);
   if (h_ver) (void)hipHostFree(h_ver);
-  void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_b, d_x64, d_r64, d_ver, d_zh, d_rhsvh, d_zbh, d_gsum, d_ps, d_dflag,
+  void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_b, d_x64, d_r64, d_ver, d_zh, d_rhsvh, d_zbh, d_gsum, d_kids, d_ps, d_dflag,
                   d_dflag_init, d_pmap, d_part, d_part2, d_asm, d_recs, d_gasm, d_gtab, d_plans,
                   (void*)d_srcs, d_offs, d_counts};
   for (void* q : ptrs) if (q) (void)hipFree(q);
@@ -211,14 +212,14 @@ namespace {
 
 // Device bytes one tile costs: 6 channels, the V-cycle scratch, the kept rhs
 // and the colour sweep's diagonal (FP32), cell types, inert flags and face masks, ghost row
-// sums, dot partials and room for its records: the instance's own lists, the
+// sums, ghost children, dot partials and room for its records: the instance's own lists, the
 // assembled active worklists and the group worklists; BF16 storage adds three
 // bfloat16 vectors, verify_f64 two FP64 vectors.
 constexpr int kRecKindsPerTile = 5;  // leaf, gather, applyl, actg, lvlg: at most 5 records per tile
 // An instance's own lists (leaf, gather, applyl, ghosts, all, actg, lvlg) hold
 // 3 leaf + ghost + 3 n <= 6 n records; a group's (leaf, ghosts, applyl) <= 2 n.
 constexpr int kOwnRecsPerTile = 6, kGroupRecsPerTile = 2;
-constexpr int64_t kBytesPerTile = (CG_NUM_CHANNELS + 3) * 512 * 4 + 2 * 512 + 1 + 64 * 4 + 2 * 8 +
+constexpr int64_t kBytesPerTile = (CG_NUM_CHANNELS + 3) * 512 * 4 + 2 * 512 + 1 + 64 * 4 + int64_t(sizeof(GhostKids)) + 2 * 8 +
                                   (kRecKindsPerTile + kOwnRecsPerTile + kGroupRecsPerTile) * int64_t(sizeof(TileRec));
 
 void server_create(const cg_server_config* cfg, cg_server& S) {
@@ -280,6 +281,7 @@ void server_create(const cg_server_config* cfg, cg_server& S) {
     }
   }
   HIPC(hipMalloc(&S.d_gsum, size_t(S.cap_ghost) * 64 * sizeof(float)));
+  HIPC(hipMalloc(&S.d_kids, size_t(S.cap_ghost) * sizeof(GhostKids)));
   HIPC(hipMalloc(&S.d_ps, sizeof(ProbState) * S.nslots));
   HIPC(hipMemsetAsync(S.d_ps, 0, sizeof(ProbState) * S.nslots, S.stream));
   HIPC(hipMalloc(&S.d_dflag, sizeof(int32_t) * S.nslots));
@@ -333,6 +335,7 @@ void server_create(const cg_server_config* cfg, cg_server& S) {
   P.d_rhsvh = S.d_rhsvh;
   P.d_zbh = S.d_zbh;
   P.d_gsum = S.d_gsum;
+  P.d_kids = S.d_kids;
   P.d_ps = S.d_ps;
   P.d_dflag = S.d_dflag;
   P.d_pmap = S.d_pmap;
@@ -531,13 +534,14 @@ void admit_upload(cg_server& S, const cg_tree_desc* d, const TreeBuild& B, const
   I->rec_begin = rb;
   I->rec_count = int(W.size());
   I->d_recs = S.d_recs + rb;
-  // records and cell types through the admission ring, copied on
+  // records, cell types and ghost children through the admission ring, copied on
   // the stream (the host does not wait for a device that is busy with other
   // requests); a tree too large for the ring goes through its own staging
   // buffer with synchronous copies
   const size_t rec_bytes = sizeof(TileRec) * W.size(), ct_bytes = size_t(n) * 512;
-  const size_t o_ct = (rec_bytes + 255) & ~size_t(255);
-  const size_t total = o_ct + ct_bytes;
+  const size_t kid_bytes = sizeof(GhostKids) * B.kids.size();
+  const size_t o_ct = (rec_bytes + 255) & ~size_t(255), o_kid = o_ct + ((ct_bytes + 255) & ~size_t(255));
+  const size_t total = o_kid + kid_bytes;
   char* ring = ring_take(S, total);
   char* stage = ring ? ring : reinterpret_cast<char*>(I->h_buf);
   if (!ring && total > I->h_bytes) fail(CG_ERR_INVALID, "cg_server_admit: staging buffer too small");
@@ -548,6 +552,10 @@ void admit_upload(cg_server& S, const cg_tree_desc* d, const TreeBuild& B, const
     else HIPC(hipMemcpy(dst, stage + off, bytes, hipMemcpyHostToDevice));
   };
   up(I->d_recs, 0, rec_bytes);
+  if (kid_bytes) {
+    std::memcpy(stage + o_kid, B.kids.data(), kid_bytes);
+    up(S.d_kids + inst.ghost_begin, o_kid, kid_bytes);
+  }
   // cell types in internal order; x = 0 so that a first warm start is a cold one
   up(S.d_ctype + size_t(tb) * 512, o_ct, ct_bytes);
   if (ring) ring_release_after_copies(S, ring, total);

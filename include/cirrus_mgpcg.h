@@ -200,17 +200,16 @@ cg_status cg_get_solution_f64(cg_problem* p, double* host);
  * tiles with the next tile's loads issued before the current one is updated
  * (on levels with more tiles than that; others as 1). */
 cg_status cg_set_schedule(cg_problem* p, int32_t coarse_shift, int32_t swizzle, int32_t tile_block);
-/* Two more kernel forms chosen by level size, also without effect on results:
- * levels (all problems of the handle together) of at most eager_max_tiles
- * tiles run the prolongation-fused colour pass and the restriction with every
- * load issued before one wait (shorter latency chain; more registers); with
- * 16-bit storage, levels of at most fused16_max_tiles tiles run the first
- * down-sweep iteration as one launch (it reads the halo's diagonals).  0: never,
- * a negative value: the default 16384.  pair_sweeps: 1 runs every red-black
+/* Two more kernel forms, also without effect on results: with 16-bit storage,
+ * levels (all problems of the handle together) of at most fused16_max_tiles
+ * tiles run the first down-sweep iteration as one launch (0: never, a negative
+ * value: the default, every level).  pair_sweeps: 1 runs every red-black
  * iteration after the first as one launch of both colours (the halo's first
  * colour formed again from the neighbours' data; bit-identical, but slower
  * than the two passes on every level measured), 0 or a negative value as two
- * colour passes (the default).  No reference counterpart. */
+ * colour passes (the default).  eager_max_tiles is accepted and changes nothing
+ * (one form of the prolongation and restriction passes serves every size).  No
+ * reference counterpart. */
 cg_status cg_set_level_forms(cg_problem* p, int32_t eager_max_tiles, int32_t fused16_max_tiles, int32_t pair_sweeps);
 typedef struct {
   int32_t candidates;        /* parameter sets timed */
