@@ -2399,46 +2399,94 @@ __global__ __launch_bounds__(64) void k_cg_finish_x(const TileRec* __restrict__ 
   store8(c.x + base, xv);
 }
 
-// Sum of a problem's per-tile partials in the fixed order (lane q adds
-// partials q, q+64, ... in sequence, then the butterfly), staged through LDS by
-// the whole workgroup.  Each thread issues all its loads of a chunk before the
-// first wait (addresses clamped into the range, so every load is in bounds),
-// and the summing wave reads its LDS values in groups of FIN_GROUP before
-// adding them in sequence: a chunk costs one memory round trip, not one per
-// element.
-constexpr int FIN_THREADS = 256;
-constexpr int FIN_CHUNK = 4096;
-constexpr int FIN_PER_THREAD = FIN_CHUNK / FIN_THREADS;
+// Sum of a problem's per-tile partials in the fixed order (lane q of the first
+// wavefront adds partials q, q + 64, ... in sequence, then the butterfly), by a
+// workgroup of NT threads.  The sequence is a chain of count / 64 dependent
+// additions, so what can be saved is the wait for the data:
+// NT = FIN_WAVE: one wavefront, each lane loading its own sequence, FIN_ROWS
+//   values in flight while the FIN_ROWS before them are added; no LDS, no barrier.
+// NT = FIN_BLOCK: the whole workgroup loads a chunk into LDS while the first
+//   wavefront adds the chunk before it.
+// Addresses are clamped into the range; what lies beyond it adds -0.0, which
+// leaves every sum as it is.
+constexpr int FIN_WAVE = 64;
+constexpr int FIN_BLOCK = 1024;
+constexpr int FIN_ROWS = 32;
+constexpr int FIN_CHUNK = 16384;
+constexpr int FIN_PER_THREAD = FIN_CHUNK / FIN_BLOCK;
 constexpr int FIN_GROUP = 16;
-__device__ __forceinline__ double block_sum_partials(const double* __restrict__ part, int begin, int count, double* lds) {
+template <int NT>
+__device__ __forceinline__ double block_sum_partials(const double* __restrict__ part, int begin, int count) {
   const int tid = threadIdx.x;
+  const double* src = part + begin;
   double a = 0.0;
-  for (int c0 = 0; c0 < count; c0 += FIN_CHUNK) {
-    const int m = min(FIN_CHUNK, count - c0);  // >= 1
-    const double* src = part + begin + c0;
+  if constexpr (NT == FIN_WAVE) {
+    auto fetch = [&](int r0, double (&v)[FIN_ROWS]) {
+#pragma unroll
+      for (int u = 0; u < FIN_ROWS; u++) v[u] = src[min((r0 + u) * 64 + tid, count - 1)];
+    };
+    double v[FIN_ROWS], w[FIN_ROWS];
+    const int rows = (count + 63) >> 6;
+    fetch(0, v);
+    for (int r0 = 0; r0 < rows; r0 += FIN_ROWS) {
+      if (r0 + FIN_ROWS < rows) fetch(r0 + FIN_ROWS, w);
+#pragma unroll
+      for (int u = 0; u < FIN_ROWS; u++) a += (r0 + u) * 64 + tid < count ? v[u] : -0.0;
+#pragma unroll
+      for (int u = 0; u < FIN_ROWS; u++) v[u] = w[u];
+    }
+    return wave_sum(a);
+  } else {
+    __shared__ double lds[FIN_CHUNK];
     double v[FIN_PER_THREAD];
+    auto fetch = [&](int c0) {
 #pragma unroll
-    for (int u = 0; u < FIN_PER_THREAD; u++) v[u] = src[min(tid + u * FIN_THREADS, m - 1)];
-    __syncthreads();  // the previous chunk's sums are done with lds
+      for (int u = 0; u < FIN_PER_THREAD; u++) v[u] = src[min(c0 + tid + u * NT, count - 1)];
+    };
+    fetch(0);
+    for (int c0 = 0; c0 < count; c0 += FIN_CHUNK) {
+      __syncthreads();  // the previous chunk's sums are done with lds
 #pragma unroll
-    for (int u = 0; u < FIN_PER_THREAD; u++)
-      if (tid + u * FIN_THREADS < m) lds[tid + u * FIN_THREADS] = v[u];
-    __syncthreads();
-    if (tid < 64) {
-      // lane tid continues its sequence tid, tid+64, ... across chunks (FIN_CHUNK is a multiple of 64)
-      const int len = (m - tid + 63) >> 6;  // values of this lane in the chunk
-      for (int g0 = 0; g0 < len; g0 += FIN_GROUP) {
-        double w[FIN_GROUP];
+      for (int u = 0; u < FIN_PER_THREAD; u++) lds[tid + u * NT] = c0 + tid + u * NT < count ? v[u] : -0.0;
+      __syncthreads();
+      if (c0 + FIN_CHUNK < count) fetch(c0 + FIN_CHUNK);
+      if (tid < 64) {
+        // lane tid continues its sequence tid, tid + 64, ... across chunks (FIN_CHUNK is a multiple of 64 FIN_GROUP)
+        const int rows = (min(FIN_CHUNK, count - c0) + 63) >> 6;
+        double w[FIN_GROUP], x[FIN_GROUP];
 #pragma unroll
-        for (int u = 0; u < FIN_GROUP; u++) w[u] = lds[min(tid + (g0 + u) * 64, FIN_CHUNK - 1)];
+        for (int u = 0; u < FIN_GROUP; u++) w[u] = lds[tid + u * 64];
+        for (int g0 = 0; g0 < rows; g0 += FIN_GROUP) {
+          const int g1 = g0 + FIN_GROUP < rows ? g0 + FIN_GROUP : 0;
 #pragma unroll
-        for (int u = 0; u < FIN_GROUP; u++)
-          if (g0 + u < len) a += w[u];
+          for (int u = 0; u < FIN_GROUP; u++) x[u] = lds[tid + (g1 + u) * 64];
+#pragma unroll
+          for (int u = 0; u < FIN_GROUP; u++) a += w[u];
+#pragma unroll
+          for (int u = 0; u < FIN_GROUP; u++) w[u] = x[u];
+        }
       }
     }
+    if (tid < 64) a = wave_sum(a);
+    return a;
   }
-  if (tid < 64) a = wave_sum(a);
-  return a;
+}
+// A problem's state as one load of the wavefront (word `lane` of it), its fields
+// taken from the lanes once they are needed: the load goes out with the partials'.
+__device__ __forceinline__ uint32_t state_word(const ProbState* ps) {
+  constexpr int kWords = int(sizeof(ProbState) / 4);
+  static_assert(kWords <= 64, "one word a lane");
+  return reinterpret_cast<const uint32_t*>(ps)[min(lane_id(), kWords - 1)];
+}
+__device__ __forceinline__ ProbState state_of(uint32_t word) {
+  union {
+    uint32_t w[sizeof(ProbState) / 4];
+    ProbState s;
+  } u;
+  hold(word);
+#pragma unroll
+  for (int i = 0; i < int(sizeof(ProbState) / 4); i++) u.w[i] = uint32_t(__builtin_amdgcn_readlane(int(word), i));
+  return u.s;
 }
 
 // Per-problem finalisation of a reduction over the LEAF-tile partials.
@@ -2446,56 +2494,63 @@ enum : int { FIN_BB = 0, FIN_RZ = 1, FIN_PAP = 2, FIN_RR = 3, FIN_MEAN = 4, FIN_
 // range_count >= 0: the launch's one problem has its partials at range_begin ..
 // range_begin + range_count - 1 (its leaf range), given by the host so that
 // their loads go out with the problem state's rather than after it.
-__global__ __launch_bounds__(FIN_THREADS) void k_finalize(Ctx c, int mode, int flags, int range_begin = 0,
-                                                          int range_count = -1) {
-  __shared__ double lds[FIN_CHUNK];
-  ProbState* ps = c.ps + (c.pmap ? c.pmap[blockIdx.x] : int(blockIdx.x));
+template <int NT>
+__global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_begin, int range_count,
+                                                 const double* part, ProbState* states, const int32_t* pmap,
+                                                 const double* part2, int32_t* dflag) {
+  ProbState* ps = states + (pmap ? pmap[blockIdx.x] : int(blockIdx.x));
+  const uint32_t word = state_word(ps);
   const bool given = range_count >= 0;
+  int begin = range_begin, count = range_count;
   if (!given) {
-    if (mode != FIN_BB && (flags & F_CHECK_DONE) && ps->done) return;
-    if (mode == FIN_MEAN && !ps->pure_neumann) return;
+    const ProbState st = state_of(word);
+    if (mode != FIN_BB && (flags & F_CHECK_DONE) && st.done) return;
+    if (mode == FIN_MEAN && !st.pure_neumann) return;
+    begin = st.leaf_begin;
+    count = st.leaf_count;
   }
-  const int begin = given ? range_begin : ps->leaf_begin;
-  const int count = given ? range_count : ps->leaf_count;
-  const double s = block_sum_partials(c.part, begin, count, lds);
+  const double s = block_sum_partials<NT>(part, begin, count);
+  const ProbState st = state_of(word);
   if (given) {  // the same tests, after the sum (whose value is then dropped)
-    if (mode != FIN_BB && (flags & F_CHECK_DONE) && ps->done) return;
-    if (mode == FIN_MEAN && !ps->pure_neumann) return;
+    if (mode != FIN_BB && (flags & F_CHECK_DONE) && st.done) return;
+    if (mode == FIN_MEAN && !st.pure_neumann) return;
   }
   double q = 0.0;
-  if (mode == FIN_MEAN) q = block_sum_partials(c.part2, begin, count, lds);
+  if (mode == FIN_MEAN) q = block_sum_partials<NT>(part2, begin, count);
   if (threadIdx.x != 0) return;
   switch (mode) {
     case FIN_BB: {  // GMGSolver.cu:542-554
       ps->bb = s;
       ps->rr = s;
-      double thr = ps->tol2 * s;
-      thr = thr > ps->thr_abs ? thr : ps->thr_abs;
+      double thr = st.tol2 * s;
+      thr = thr > st.thr_abs ? thr : st.thr_abs;
+      const int done = (s == 0.0 || st.max_iters <= 0) ? 1 : 0;
       ps->thr = thr > 2.2250738585072014e-308 ? thr : 2.2250738585072014e-308;
       ps->iter = 0;
       ps->converged = (s == 0.0) ? 1 : 0;
-      ps->done = (s == 0.0 || ps->max_iters <= 0) ? 1 : 0;
+      ps->done = done;
       ps->gamma = 0.0;
-      c.dflag[blockIdx.x] = ps->done;
+      dflag[blockIdx.x] = done;
       break;
     }
     case FIN_RZ:  // gamma_old = gamma; gamma = r.z; beta = gamma / gamma_old (GMGSolver.cu:629-638)
-      ps->gamma_old = ps->gamma;
+      ps->gamma_old = st.gamma;
       ps->gamma = s;
-      ps->beta = (ps->iter == 0) ? 0.0 : s / ps->gamma_old;
+      ps->beta = (st.iter == 0) ? 0.0 : s / st.gamma;
       break;
     case FIN_PAP:  // alpha = gamma / p.Ap (GMGSolver.cu:580-582)
       ps->pAp = s;
-      ps->alpha = ps->gamma / s;
+      ps->alpha = st.gamma / s;
       break;
     case FIN_RR: {  // GMGSolver.cu:611-619 (checked every sync_stride iterations)
       ps->rr = s;
-      int it = ps->iter + 1;
+      const int it = st.iter + 1, cs = st.check_stride;
+      const bool converged = cs > 0 && it % cs == 0 && s < st.thr;
+      const int done = (converged || it >= st.max_iters) ? 1 : st.done;
       ps->iter = it;
-      const int cs = ps->check_stride;
-      if (cs > 0 && it % cs == 0 && s < ps->thr) { ps->converged = 1; ps->done = 1; }
-      else if (it >= ps->max_iters) ps->done = 1;
-      c.dflag[blockIdx.x] = ps->done;
+      if (converged) ps->converged = 1;
+      ps->done = done;
+      dflag[blockIdx.x] = done;
       break;
     }
     case FIN_MEAN:
@@ -2503,18 +2558,18 @@ __global__ __launch_bounds__(FIN_THREADS) void k_finalize(Ctx c, int mode, int f
       break;
     case FIN_IRBB:  // |b|^2 of an FP64 refinement's right-hand side and the inner solves' threshold floor
       ps->bb_b = s;
-      ps->thr_abs = ps->tol_abs2 * s;
+      ps->thr_abs = st.tol_abs2 * s;
       break;
     case FIN_SCALE: {  // float16 storage: the right-hand side's scale 2^k, from |b|^2 / cells = 2^e f,
                        // f in [1, 2): k = -floor(e/2) - 4 (root mean square near 2^-4)
       int k = 0;
       if (s > 0.0) {
-        const int e = ilogb(s / (512.0 * double(ps->leaf_count)));
+        const int e = ilogb(s / (512.0 * double(st.leaf_count)));
         const int half = (e >= 0) ? e / 2 : -((-e + 1) / 2);
         k = min(120, max(-120, -half - 4));
       }
       ps->scale_exp = k;
-      ps->thr_abs = ldexp(ps->thr_abs, 2 * k);
+      ps->thr_abs = ldexp(st.thr_abs, 2 * k);
       break;
     }
   }
@@ -2650,9 +2705,9 @@ __global__ __launch_bounds__(64) void k_dot_selected(const int32_t* __restrict__
   const double s = tile_dot(A, Bv, sel[q]);
   if (lane_id() == 0) part[q] = s;
 }
-__global__ __launch_bounds__(FIN_THREADS) void k_sum_partials(const double* __restrict__ part, int n, double* __restrict__ out) {
-  __shared__ double lds[FIN_CHUNK];
-  double s = block_sum_partials(part, 0, n, lds);
+template <int NT>
+__global__ __launch_bounds__(NT) void k_sum_partials(const double* __restrict__ part, int n, double* __restrict__ out) {
+  const double s = block_sum_partials<NT>(part, 0, n);
   if (threadIdx.x == 0) *out = s;
 }
 // Copy whole tiles of a list from one channel to another.
@@ -3455,21 +3510,21 @@ __global__ __launch_bounds__(64) void k_ir_accumulate(Ctx c, const TileRec* __re
 // Per problem q (workgroup -> problem through pmap, else the identity): its
 // |r64|^2 (the leaf-slot partials) and |b|^2 (ProbState::bb_b) into
 // out[2q], out[2q + 1].
-__global__ __launch_bounds__(FIN_THREADS) void k_ir_verdict(Ctx c, double* __restrict__ out) {
-  __shared__ double lds[FIN_CHUNK];
+template <int NT>
+__global__ __launch_bounds__(NT) void k_ir_verdict(Ctx c, double* __restrict__ out) {
   const int q = c.pmap ? c.pmap[blockIdx.x] : int(blockIdx.x);
   const ProbState* ps = c.ps + q;
-  const double s = block_sum_partials(c.part, ps->leaf_begin, ps->leaf_count, lds);
+  const double s = block_sum_partials<NT>(c.part, ps->leaf_begin, ps->leaf_count);
   if (threadIdx.x == 0) {
     out[2 * q] = s;
     out[2 * q + 1] = ps->bb_b;
   }
 }
 // Per-problem totals of the leaf-slot partials, in the fixed order.
-__global__ __launch_bounds__(FIN_THREADS) void k_prob_sums(Ctx c, double* __restrict__ out) {
-  __shared__ double lds[FIN_CHUNK];
+template <int NT>
+__global__ __launch_bounds__(NT) void k_prob_sums(Ctx c, double* __restrict__ out) {
   const ProbState* ps = c.ps + blockIdx.x;
-  const double s = block_sum_partials(c.part, ps->leaf_begin, ps->leaf_count, lds);
+  const double s = block_sum_partials<NT>(c.part, ps->leaf_begin, ps->leaf_count);
   if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 

@@ -78,6 +78,7 @@ struct cg_problem {
   int n = 0;  // tiles of all problems
   int max_level = 0;
   int n_leaf = 0, n_ghost = 0;
+  int max_leaf = 0;              // LEAF tiles of the largest problem
   std::vector<int> ext_of;       // internal -> caller index (problems concatenated)
   std::vector<int> leaf_begin;   // per problem: first leaf slot
   std::vector<int> leaf_count;   // per problem: LEAF tiles
@@ -613,6 +614,7 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
   }
   const int leaf_total = leaf_base[nprob], ghost_total = ghost_base[nprob];
   P.n_leaf = leaf_total;
+  for (int q = 0; q < nprob; q++) P.max_leaf = std::max(P.max_leaf, P.leaf_count[q]);
   P.n_ghost = ghost_total;
   P.max_level = 0;
   for (int i = 0; i < n; i++) P.max_level = std::max(P.max_level, lev[i]);
@@ -799,6 +801,28 @@ int loop_waves() {
   }();
   return w;
 }
+// Which form of the partial sums (block_sum_partials) a launch takes, by the
+// largest problem's LEAF tiles.  A k_finalize launch, by one wavefront against by
+// 16: 64 tiles 2.2 against 4.4 us, 4,096 tiles 3.5 against 4.7, 45,054 tiles 25
+// against 12.2; the two meet near 7,000.  (One workgroup of four wavefronts that
+// loaded a chunk, waited and added it took 3.4, 4.4 and 27.2 us.)
+constexpr int kFinWaveMax = 6144;
+inline bool fin_by_wave(int max_leaf) { return max_leaf <= kFinWaveMax; }
+// One finalize workgroup per problem of c (through its problem map).
+void launch_finalize(hipStream_t st, int nprob, int max_leaf, const Ctx& c, int mode, int flags, int range_begin = 0,
+                     int range_count = -1) {
+  if (fin_by_wave(max_leaf))
+    k_finalize<FIN_WAVE><<<unsigned(nprob), FIN_WAVE, 0, st>>>(mode, flags, range_begin, range_count, c.part, c.ps, c.pmap,
+                                                               c.part2, c.dflag);
+  else
+    k_finalize<FIN_BLOCK><<<unsigned(nprob), FIN_BLOCK, 0, st>>>(mode, flags, range_begin, range_count, c.part, c.ps,
+                                                                 c.pmap, c.part2, c.dflag);
+}
+void launch_sum(hipStream_t st, const double* part, int n, double* out) {
+  if (fin_by_wave(n)) k_sum_partials<FIN_WAVE><<<1, FIN_WAVE, 0, st>>>(part, n, out);
+  else k_sum_partials<FIN_BLOCK><<<1, FIN_BLOCK, 0, st>>>(part, n, out);
+}
+
 template <class V, bool DOT>
 void launch_gs_as(cg_problem& P, const DList& a, const Ctx& c, int l, V* Z, const V* R, int color, int flags) {
   const int lw = P.gs_block == 8 ? loop_waves<V, DOT>() : 0;
@@ -1083,7 +1107,7 @@ void enqueue_cg_iteration(cg_problem& P, const VParams& vp, int pure_neumann) {
   const int rb = one ? P.leaf_begin[0] : 0, rc = one ? P.leaf_count[0] : -1;
   if (pure_neumann) {
     k_mean<<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl & ~F_INERT, c.r, c);
-    k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_MEAN, fl);
+    launch_finalize(P.stream, int(np), P.max_leaf, c, FIN_MEAN, fl);
     k_subtract_mean<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl & ~F_INERT, c.r, 1, c);
   }
   // RB-GS: down-sweep in the scratch buffer, z assembled in z by the up-sweep
@@ -1094,13 +1118,13 @@ void enqueue_cg_iteration(cg_problem& P, const VParams& vp, int pure_neumann) {
   if (v.amg) enqueue_amg_vcycle(P, v);
   else enqueue_vcycle<V>(P, v.smoother == CG_SMOOTH_RBGS ? pool_zb<V>(P) : Z, Z, nullptr, v, rz_fused ? F_DOT_RZ : 0);
   if (!rz_fused) k_cg_dot_rz<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
-  k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_RZ, fl, rb, rc);
+  launch_finalize(P.stream, int(np), P.max_leaf, c, FIN_RZ, fl, rb, rc);
   k_cg_update_p<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
   k_apply<true><<<grid_for(P.applyl.n, fl), 64, 0, P.stream>>>(P.L(P.applyl), P.applyl.n, fl, c.p, c.ap, -1, 0, 1, c);
   if (P.gather.n) k_ghost_gather<<<grid_for(P.gather.n, fl), 64, 0, P.stream>>>(P.L(P.gather), P.gather.n, fl, c);
-  k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_PAP, fl, rb, rc);
+  launch_finalize(P.stream, int(np), P.max_leaf, c, FIN_PAP, fl, rb, rc);
   k_cg_update_xr<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
-  k_finalize<<<np, FIN_THREADS, 0, P.stream>>>(c, FIN_RR, fl, rb, rc);
+  launch_finalize(P.stream, int(np), P.max_leaf, c, FIN_RR, fl, rb, rc);
 }
 void enqueue_cg_iteration(cg_problem& P, const VParams& v, int pure_neumann, int storage) {
   if (storage == CG_STORE_BF16) enqueue_cg_iteration<bf16>(P, v, pure_neumann);
@@ -1132,7 +1156,7 @@ double dot_types(cg_problem& P, const float* A, const float* B, int types) {
   const TileRec* dl = tmp_list(P, l);
   const Ctx c = P.ctx();
   k_dot_tiles<<<unsigned(l.size()), 64, 0, P.stream>>>(c, dl, int(l.size()), A, B, P.d_part);
-  k_sum_partials<<<1, FIN_THREADS, 0, P.stream>>>(P.d_part, int(l.size()), P.d_scalar);
+  launch_sum(P.stream, P.d_part, int(l.size()), P.d_scalar);
   double out = 0;
   HIPC(hipMemcpyAsync(&out, P.d_scalar, sizeof(double), hipMemcpyDeviceToHost, P.stream));
   HIPC(hipStreamSynchronize(P.stream));
@@ -1182,7 +1206,8 @@ void ensure_f64(cg_problem& P) {
 // Per-problem totals of the leaf-slot partials in c.part, to the host.
 std::vector<double> prob_sums(cg_problem& P) {
   const Ctx c = P.ctx();
-  k_prob_sums<<<unsigned(P.nprob), FIN_THREADS, 0, P.stream>>>(c, P.d_psum);
+  if (fin_by_wave(P.max_leaf)) k_prob_sums<FIN_WAVE><<<unsigned(P.nprob), FIN_WAVE, 0, P.stream>>>(c, P.d_psum);
+  else k_prob_sums<FIN_BLOCK><<<unsigned(P.nprob), FIN_BLOCK, 0, P.stream>>>(c, P.d_psum);
   std::vector<double> out(P.nprob);
   HIPC(hipMemcpyAsync(out.data(), P.d_psum, sizeof(double) * P.nprob, hipMemcpyDeviceToHost, P.stream));
   HIPC(hipStreamSynchronize(P.stream));
@@ -1199,7 +1224,7 @@ std::vector<double> residual64(cg_problem& P, const float* B, int pure_neumann, 
   if (P.ghosts.n) k_accumulate_ghosts64<<<P.ghosts.n, 64, 0, P.stream>>>(c, P.L(P.ghosts), P.ghosts.n, P.d_r64);
   if (pure_neumann) {
     k_ir_residual<<<gl, 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, B, P.d_r64, 1);
-    k_finalize<<<unsigned(P.nprob), FIN_THREADS, 0, P.stream>>>(c, FIN_MEAN, 0);
+    launch_finalize(P.stream, P.nprob, P.max_leaf, c, FIN_MEAN, 0);
     k_ir_recenter<<<gl, 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, P.d_r64, write_r ? 1 : 0);
   } else {
     k_ir_residual<<<gl, 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, B, P.d_r64, write_r ? 0 : 2);
@@ -1238,7 +1263,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   const bool f16s = prm.storage == CG_STORE_F16;
   if (f16s) {  // float16 storage: solve for 2^k b, k from |b|^2 per problem (FIN_SCALE)
     k_ir_norm<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r);
-    k_finalize<<<unsigned(P.nprob), FIN_THREADS, 0, P.stream>>>(c, FIN_SCALE, 0);
+    launch_finalize(P.stream, P.nprob, P.max_leaf, c, FIN_SCALE, 0);
     k_scale_leaf<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, 1);
   }
   if (prm.storage == CG_STORE_BF16)
@@ -1247,7 +1272,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
     k_cg_init<f16><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz, c);
   else
     k_cg_init<float><<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz, c);
-  k_finalize<<<unsigned(P.nprob), FIN_THREADS, 0, P.stream>>>(c, FIN_BB, 0);
+  launch_finalize(P.stream, P.nprob, P.max_leaf, c, FIN_BB, 0);
   HIPC(hipGetLastError());
 
   char keybuf[160];
@@ -2257,7 +2282,7 @@ cg_status cg_dot_noalloc(cg_problem* p, int32_t a_channel, int32_t b_channel, in
     double* res = reinterpret_cast<double*>(s + kScrOut);
     k_select_tiles<<<1, SEL_THREADS, 0, P.stream>>>(P.d_tiles, P.n, tile_types, sel);
     k_dot_selected<<<unsigned(count), 64, 0, P.stream>>>(sel, count, P.d_ch[a_channel], P.d_ch[b_channel], part);
-    k_sum_partials<<<1, FIN_THREADS, 0, P.stream>>>(part, count, res);
+    launch_sum(P.stream, part, count, res);
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(out, res, sizeof(double), hipMemcpyDeviceToHost, P.stream));
     HIPC(hipStreamSynchronize(P.stream));
@@ -2271,7 +2296,7 @@ cg_status cg_recenter_leaf_voxels(cg_problem* p, int32_t channel) {
     set_prob_state(*p, 0.0, 0, 1);
     const Ctx c = p->ctx();
     k_mean<<<p->leaf.n, 64, 0, p->stream>>>(p->L(p->leaf), p->leaf.n, 0, p->d_ch[channel], c);
-    k_finalize<<<1, FIN_THREADS, 0, p->stream>>>(c, FIN_MEAN, 0);
+    launch_finalize(p->stream, 1, p->max_leaf, c, FIN_MEAN, 0);
     k_subtract_mean<float><<<p->leaf.n, 64, 0, p->stream>>>(p->L(p->leaf), p->leaf.n, 0, p->d_ch[channel], 0, c);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(p->stream));

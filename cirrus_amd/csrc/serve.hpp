@@ -711,7 +711,7 @@ void group_residual64(cg_server& S, const Group& G, bool write_r) {
   if (G.ghosts.n) k_accumulate_ghosts64<<<G.ghosts.n, 64, 0, st>>>(c, GL(S, G.ghosts), G.ghosts.n, S.d_r64);
   if (S.prm.pure_neumann) {
     k_ir_residual<<<gl, 64, 0, st>>>(c, GL(S, G.leaf_full), G.leaf_full.n, S.d_b, S.d_r64, 1);
-    k_finalize<<<unsigned(G.nfull), FIN_THREADS, 0, st>>>(group_ctx(S), FIN_MEAN, 0);
+    launch_finalize(st, G.nfull, S.view.max_leaf, group_ctx(S), FIN_MEAN, 0);
     k_ir_recenter<<<gl, 64, 0, st>>>(c, GL(S, G.leaf_full), G.leaf_full.n, S.d_r64, write_r ? 1 : 0);
   } else {
     k_ir_residual<<<gl, 64, 0, st>>>(c, GL(S, G.leaf_full), G.leaf_full.n, S.d_b, S.d_r64, write_r ? 0 : 2);
@@ -744,6 +744,7 @@ void server_start_queued(cg_server& S, int k) {
     ps.max_iters = S.prm.max_iters;
     ps.leaf_begin = int32_t(I.leaf_begin);
     ps.leaf_count = I.nleaf;
+    S.view.max_leaf = std::max(S.view.max_leaf, I.nleaf);
     ps.pure_neumann = S.prm.pure_neumann;
     ps.check_stride = S.prm.sync_stride;
     if (!I.dev_rhs && !I.ir_cont)
@@ -765,7 +766,7 @@ void server_start_queued(cg_server& S, int k) {
     if (G.nfull) {  // |b|^2 and the threshold floor
       group_residual64(S, G, true);
       k_ir_norm<<<grid_for(G.leaf_full.n, kSwizzle), 64, 0, st>>>(c, GL(S, G.leaf_full), G.leaf_full.n, S.d_b);
-      k_finalize<<<unsigned(G.nfull), FIN_THREADS, 0, st>>>(group_ctx(S), FIN_IRBB, 0);
+      launch_finalize(st, G.nfull, S.view.max_leaf, group_ctx(S), FIN_IRBB, 0);
     }
     // the step solves A d = float(r) from d = 0
     if (S.prm.storage == CG_STORE_BF16) k_cg_init<bf16><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, c);
@@ -781,7 +782,7 @@ void server_start_queued(cg_server& S, int k) {
   }
   Ctx ci = group_ctx(S);
   ci.dflag = S.d_dflag_init;
-  k_finalize<<<unsigned(G.n), FIN_THREADS, 0, st>>>(ci, FIN_BB, 0);
+  launch_finalize(st, G.n, S.view.max_leaf, ci, FIN_BB, 0);
   HIPC(hipGetLastError());
 }
 
@@ -873,7 +874,8 @@ void enqueue_verify(cg_server& S, const Group& G, const std::vector<int>& slots)
   if (S.refine) k_ir_accumulate<<<gl, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, S.d_x64, 0);
   else k_ir_load_x<<<gl, 64, 0, st>>>(c, GL(S, G.leaf), G.leaf.n, S.d_ch[CG_CH_X], S.d_x64);
   group_residual64(S, G, S.refine != 0);
-  k_ir_verdict<<<unsigned(G.n), FIN_THREADS, 0, st>>>(group_ctx(S), S.d_ver);
+  if (fin_by_wave(S.view.max_leaf)) k_ir_verdict<FIN_WAVE><<<unsigned(G.n), FIN_WAVE, 0, st>>>(group_ctx(S), S.d_ver);
+  else k_ir_verdict<FIN_BLOCK><<<unsigned(G.n), FIN_BLOCK, 0, st>>>(group_ctx(S), S.d_ver);
   // one copy over the group's slot range (the other slots' entries in it are
   // rewritten with the values their own checks left)
   const int lo = *std::min_element(slots.begin(), slots.end()), hi = *std::max_element(slots.begin(), slots.end());
