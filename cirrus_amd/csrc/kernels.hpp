@@ -120,7 +120,7 @@ struct Ctx {
   f16* zbf;
   float* gsum;   // 64 per ghost: 2x2x2 sums of the ghost rows of A p
   ProbState* ps;
-  int32_t* dflag; // per-problem copy of ProbState::done, polled by the host
+  int32_t* progress;  // per problem 2 * iterations + done, in host memory, which the host polls (null: nobody does)
   const int32_t* pmap;  // finalize workgroup -> problem (null: identity)
   double* part;  // per-leaf-slot dot partials
   double* part2; // second partial stream (mean counts)
@@ -2494,10 +2494,13 @@ enum : int { FIN_BB = 0, FIN_RZ = 1, FIN_PAP = 2, FIN_RR = 3, FIN_MEAN = 4, FIN_
 // range_count >= 0: the launch's one problem has its partials at range_begin ..
 // range_begin + range_count - 1 (its leaf range), given by the host so that
 // their loads go out with the problem state's rather than after it.
+__device__ __forceinline__ void report_progress(int32_t* progress, int iters, int done) {
+  if (progress) __hip_atomic_store(progress + blockIdx.x, 2 * iters + done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <int NT>
 __global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_begin, int range_count,
                                                  const double* part, ProbState* states, const int32_t* pmap,
-                                                 const double* part2, int32_t* dflag) {
+                                                 const double* part2, int32_t* progress) {
   ProbState* ps = states + (pmap ? pmap[blockIdx.x] : int(blockIdx.x));
   const uint32_t word = state_word(ps);
   const bool given = range_count >= 0;
@@ -2530,7 +2533,7 @@ __global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_
       ps->converged = (s == 0.0) ? 1 : 0;
       ps->done = done;
       ps->gamma = 0.0;
-      dflag[blockIdx.x] = done;
+      report_progress(progress, 0, done);
       break;
     }
     case FIN_RZ:  // gamma_old = gamma; gamma = r.z; beta = gamma / gamma_old (GMGSolver.cu:629-638)
@@ -2550,7 +2553,7 @@ __global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_
       ps->iter = it;
       if (converged) ps->converged = 1;
       ps->done = done;
-      dflag[blockIdx.x] = done;
+      report_progress(progress, it, done);
       break;
     }
     case FIN_MEAN:

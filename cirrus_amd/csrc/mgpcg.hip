@@ -124,7 +124,6 @@ struct cg_problem {
   float* d_gsum = nullptr;
   GhostKids* d_kids = nullptr;   // by ghost slot (behind d_gsum in its allocation)
   ProbState* d_ps = nullptr;
-  int32_t* d_dflag = nullptr;
   const int32_t* d_pmap = nullptr;  // finalize workgroup -> problem (pools whose problems are a subset)
   CoarsePlan* d_plans = nullptr;
   double* d_part = nullptr;
@@ -136,11 +135,10 @@ struct cg_problem {
   int tmp_list_cap = 0;
   int32_t* d_ext = nullptr;      // internal tile -> caller index (channel moves from and to device buffers)
   hipStream_t stream = nullptr;
-  int* h_pin = nullptr;
-  ProbState* h_ps = nullptr;     // pinned staging of the ProbState uploads
+  ProbState* h_ps = nullptr;     // pinned staging of the ProbState uploads and of the final states
+  int32_t* h_prog = nullptr;     // Ctx::progress (pinned, behind h_ps in its allocation)
   hipEvent_t ev_ps = nullptr;    // recorded after the last upload from h_ps
   bool ps_pending = false;
-  hipEvent_t ev[2] = {nullptr, nullptr};
   hipEvent_t ev_io[2] = {nullptr, nullptr};  // orders device channel moves against the caller's stream
   hipGraphExec_t graph = nullptr;
   std::string graph_key;
@@ -168,7 +166,7 @@ struct cg_problem {
     c.gsum = d_gsum;
     c.kids = d_kids;
     c.ps = d_ps;
-    c.dflag = d_dflag;
+    c.progress = h_prog;
     c.pmap = d_pmap;
     c.part = d_part;
     c.part2 = d_part2;
@@ -182,14 +180,13 @@ struct cg_problem {
 
 cg_problem::~cg_problem() {
   if (!owner) return;
+  if (stream) (void)hipStreamSynchronize(stream);  // nothing writes to the memory below any more
   if (graph) (void)hipGraphExecDestroy(graph);
-  for (auto e : ev) if (e) (void)hipEventDestroy(e);
   for (auto e : ev_io) if (e) (void)hipEventDestroy(e);
-  if (h_pin) (void)hipHostFree(h_pin);
   if (h_ps) (void)hipHostFree(h_ps);
   if (ev_ps) (void)hipEventDestroy(ev_ps);
   void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_zh, d_rhsvh, d_zbh, d_x64, d_r64, d_bsave, d_psum, d_gsum, d_ps,
-                  d_dflag, d_plans, d_part, d_part2, d_scalar, d_lists, d_tiles, d_tmp_list, d_amgc, d_amgct, d_ext};
+                  d_plans, d_part, d_part2, d_scalar, d_lists, d_tiles, d_tmp_list, d_amgc, d_amgct, d_ext};
   for (void* q : ptrs) if (q) (void)hipFree(q);
   for (auto q : d_ch) if (q) (void)hipFree(q);
   for (auto q : d_api) if (q) (void)hipFree(q);
@@ -651,8 +648,6 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
     HIPC(hipMemcpyAsync(P.d_kids, P.kids.data(), sizeof(GhostKids) * size_t(ghost_total), hipMemcpyHostToDevice, P.stream));
   HIPC(hipMalloc(&P.d_ps, sizeof(ProbState) * nprob));
   HIPC(hipMemsetAsync(P.d_ps, 0, sizeof(ProbState) * nprob, P.stream));
-  HIPC(hipMalloc(&P.d_dflag, sizeof(int32_t) * nprob));
-  HIPC(hipMemsetAsync(P.d_dflag, 0, sizeof(int32_t) * nprob, P.stream));
   size_t np = size_t(std::max(n, 64));
   HIPC(hipMalloc(&P.d_part, np * sizeof(double)));
   HIPC(hipMalloc(&P.d_part2, np * sizeof(double)));
@@ -673,11 +668,9 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
   k_face_mask<<<P.all.n, 64, 0, P.stream>>>(P.d_ctype, P.d_fmask, P.d_fsplit, P.L(P.all), P.all.n);
   k_diag<<<P.all.n, 64, 0, P.stream>>>(P.ctx(), P.L(P.all), P.all.n, P.d_diag);
   HIPC(hipGetLastError());
-  HIPC(hipHostMalloc(&P.h_pin, 2 * sizeof(int) * nprob, hipHostMallocDefault));
-  HIPC(hipHostMalloc(&P.h_ps, sizeof(ProbState) * nprob, hipHostMallocDefault));
+  HIPC(hipHostMalloc(&P.h_ps, (sizeof(ProbState) + sizeof(int32_t)) * nprob, hipHostMallocCoherent));
+  P.h_prog = reinterpret_cast<int32_t*>(P.h_ps + nprob);
   HIPC(hipEventCreateWithFlags(&P.ev_ps, hipEventDisableTiming));
-  HIPC(hipEventCreateWithFlags(&P.ev[0], hipEventDisableTiming));
-  HIPC(hipEventCreateWithFlags(&P.ev[1], hipEventDisableTiming));
   HIPC(hipEventCreateWithFlags(&P.ev_io[0], hipEventDisableTiming));
   HIPC(hipEventCreateWithFlags(&P.ev_io[1], hipEventDisableTiming));
   HIPC(hipStreamSynchronize(P.stream));
@@ -766,7 +759,6 @@ void set_prob_state(cg_problem& P, double tol, int max_iters, int pure_neumann, 
     s.check_stride = check_stride;
   }
   HIPC(hipMemcpyAsync(P.d_ps, st, sizeof(ProbState) * P.nprob, hipMemcpyHostToDevice, P.stream));
-  HIPC(hipMemsetAsync(P.d_dflag, 0, sizeof(int32_t) * P.nprob, P.stream));
   if (P.h_ps) {
     HIPC(hipEventRecord(P.ev_ps, P.stream));
     P.ps_pending = true;
@@ -813,10 +805,10 @@ void launch_finalize(hipStream_t st, int nprob, int max_leaf, const Ctx& c, int 
                      int range_count = -1) {
   if (fin_by_wave(max_leaf))
     k_finalize<FIN_WAVE><<<unsigned(nprob), FIN_WAVE, 0, st>>>(mode, flags, range_begin, range_count, c.part, c.ps, c.pmap,
-                                                               c.part2, c.dflag);
+                                                               c.part2, c.progress);
   else
     k_finalize<FIN_BLOCK><<<unsigned(nprob), FIN_BLOCK, 0, st>>>(mode, flags, range_begin, range_count, c.part, c.ps,
-                                                                 c.pmap, c.part2, c.dflag);
+                                                                 c.pmap, c.part2, c.progress);
 }
 void launch_sum(hipStream_t st, const double* part, int n, double* out) {
   if (fin_by_wave(n)) k_sum_partials<FIN_WAVE><<<1, FIN_WAVE, 0, st>>>(part, n, out);
@@ -1170,11 +1162,52 @@ void full_negative_laplacian(cg_problem& P, float* X, float* AX, int diag) {
   if (P.ghosts.n) k_accumulate_ghosts<<<P.ghosts.n, 64, 0, P.stream>>>(c, P.L(P.ghosts), P.ghosts.n, AX);
 }
 
-std::vector<ProbState> read_states(cg_problem& P) {
-  std::vector<ProbState> s(P.nprob);
-  HIPC(hipMemcpyAsync(s.data(), P.d_ps, sizeof(ProbState) * P.nprob, hipMemcpyDeviceToHost, P.stream));
+// Waits for the stream's work; the problems' states as it leaves them.
+std::vector<ProbState> finish_states(cg_problem& P) {
+  HIPC(hipMemcpyAsync(P.h_ps, P.d_ps, sizeof(ProbState) * P.nprob, hipMemcpyDeviceToHost, P.stream));
   HIPC(hipStreamSynchronize(P.stream));
-  return s;
+  P.ps_pending = false;
+  return std::vector<ProbState>(P.h_ps, P.h_ps + P.nprob);
+}
+
+// Waits until every problem is done or past iteration `iters`; true when all are
+// done.  The kernels write their progress to host memory (Ctx::progress), so an
+// iteration needs no copy and no event for it: those cost 8 to 12 us between two
+// iterations, more than its own host wait.  A stream that has ended or failed
+// ends the wait too.
+bool wait_progress(cg_problem& P, int iters) {
+  using clock = std::chrono::steady_clock;
+  bool all = true;
+  for (int q = 0; q < P.nprob; q++) {
+    clock::time_point since{}, checked{};
+    for (unsigned spin = 0;; spin++) {
+      const int32_t w = __atomic_load_n(&P.h_prog[q], __ATOMIC_ACQUIRE);
+      if (w & 1) break;
+      if ((w >> 1) >= iters) {
+        all = false;
+        break;
+      }
+      if (spin % 64 != 63) {
+        __builtin_ia32_pause();
+        continue;
+      }
+      const auto now = clock::now();
+      if (spin == 63) since = checked = now;
+      if (now - checked > std::chrono::milliseconds(20)) {  // is the device still at it?
+        checked = now;
+        const hipError_t e = hipStreamQuery(P.stream);
+        if (e != hipErrorNotReady) {
+          HIPC(e);
+          const int32_t last = __atomic_load_n(&P.h_prog[q], __ATOMIC_ACQUIRE);
+          if (!(last & 1) && (last >> 1) < iters) fail(CG_ERR_HIP, "cg_solve: the device ended without its iterations");
+        }
+        (void)hipGetLastError();  // "not ready" is no error
+      }
+      if (now - since > std::chrono::milliseconds(2)) std::this_thread::sleep_for(std::chrono::microseconds(50));
+      else std::this_thread::yield();
+    }
+  }
+  return all;
 }
 
 // All problems of the pool, one graph replay per CG iteration for all of them;
@@ -1255,6 +1288,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   v.pcoef = prm.prolong_coeff;
   const int stride = std::max(1, prm.sync_stride);
   auto t0 = std::chrono::steady_clock::now();
+  for (int q = 0; q < P.nprob; q++) P.h_prog[q] = 0;  // the stream is idle: every entry point waits for its work
   set_prob_state(P, prm.rel_tol, prm.max_iters, prm.pure_neumann, prm.sync_stride, tol_q, maxit_q, thr_abs_q);
   int max_iters = prm.max_iters;
   if (maxit_q) for (int q = 0; q < P.nprob; q++) max_iters = std::max(max_iters, maxit_q[q]);
@@ -1279,11 +1313,13 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   v.amg = amg ? 1 : 0;
   std::snprintf(keybuf, sizeof(keybuf), "%d/%d/%d/%a/%a/%a/%d/%d/%d/%d", v.nu, v.coarsest, v.smoother, double(v.omega),
                 double(v.ooa), double(v.pcoef), prm.pure_neumann, prm.storage, P.swz, v.amg);
-  // -1: replay where launches dominate an iteration (the AMG V-cycle; handles
-  // of fewer than kStreamMinTiles tiles), stream launches otherwise, which
-  // measured faster on larger single problems (a graph node costs less when
-  // empty, more once its kernel moves data)
-  constexpr int kStreamMinTiles = 4096;
+  // -1: replay where the host could not keep up with the device (the AMG V-cycle;
+  // handles of fewer than kStreamMinTiles tiles), stream launches otherwise.  A
+  // launch costs the host 3.5 to 5 us, a replayed node less, and the device 2 us
+  // more an iteration.  5,505 tiles (41 launches of 3.7 us an iteration): 4.9 ms a
+  // solve by stream launches with a busy host, 2 % less than by replay with an idle
+  // one, 4.0 ms by replay; 14,345 tiles (5.3 us a launch): 3.47 ms and 3.53.
+  constexpr int kStreamMinTiles = 8192;
   const bool use_graph = prm.use_graph > 0 || (prm.use_graph < 0 && (amg || P.n < kStreamMinTiles));
   if (use_graph && P.graph_key != keybuf) {
     if (P.graph) HIPC(hipGraphExecDestroy(P.graph));
@@ -1300,31 +1336,13 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
     if (use_graph) HIPC(hipGraphLaunch(P.graph, P.stream));
     else enqueue_cg_iteration(P, v, prm.pure_neumann, prm.storage);
   };
-  // Poll the done flags one chunk behind the enqueue front, so the device never
-  // waits for the host; iterations after convergence exit at their first load.
-  const int npb = P.nprob;
-  auto all_done = [&](int sl) {
-    for (int q = 0; q < npb; q++) if (!P.h_pin[sl * npb + q]) return false;
-    return true;
-  };
-  int enq = 0, slot = 0;
-  bool have_prev = false;
-  while (true) {
-    if (max_iters == 0) break;
-    for (int s = 0; s < stride; s++) { one_iter(); enq++; }
+  // Follow the device one chunk behind the enqueue front, so it never waits for
+  // the host; iterations after convergence exit at their first load.
+  for (int enq = 0; enq < max_iters;) {
+    for (int s = 0; s < stride; s++) one_iter();
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(&P.h_pin[slot * npb], P.d_dflag, sizeof(int32_t) * npb, hipMemcpyDeviceToHost, P.stream));
-    HIPC(hipEventRecord(P.ev[slot], P.stream));
-    if (have_prev) {
-      HIPC(hipEventSynchronize(P.ev[1 - slot]));
-      if (all_done(1 - slot)) break;
-    }
-    if (enq >= max_iters) {
-      HIPC(hipEventSynchronize(P.ev[slot]));
-      break;
-    }
-    have_prev = true;
-    slot = 1 - slot;
+    if (enq > 0 && wait_progress(P, enq)) break;
+    enq += stride;
   }
   // the last iteration's x update (k_cg_update_p applies each earlier one)
   k_cg_finish_x<<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz | (c.inert ? F_INERT : 0), c);
@@ -1333,9 +1351,8 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
     k_scale_leaf<<<grid_for(P.leaf.n, kSwizzle), 64, 0, P.stream>>>(c, P.L(P.leaf), P.leaf.n, c.r, -1);
   }
   if (tail) (*tail)();
-  HIPC(hipStreamSynchronize(P.stream));
+  std::vector<ProbState> st = finish_states(P);
   auto t1 = std::chrono::steady_clock::now();
-  std::vector<ProbState> st = read_states(P);
   for (ProbState& s : st) {  // |b|^2 and |r|^2 at the caller's scale (exact: powers of two)
     s.bb = std::ldexp(s.bb, -2 * s.scale_exp);
     s.rr = std::ldexp(s.rr, -2 * s.scale_exp);

@@ -143,8 +143,6 @@ struct cg_server {
   float* d_gsum = nullptr;
   GhostKids* d_kids = nullptr;
   ProbState* d_ps = nullptr;
-  int32_t* d_dflag = nullptr;
-  int32_t* d_dflag_init = nullptr;
   int32_t* d_pmap = nullptr;
   double* d_part = nullptr;
   double* d_part2 = nullptr;
@@ -196,8 +194,8 @@ cg_server::~cg_server() {
   for (auto& row : ev_gtab)
     for (auto e : row) if (e) (void)hipEventDestroy(e);
   if (h_ver) (void)hipHostFree(h_ver);
-  void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_b, d_x64, d_r64, d_ver, d_zh, d_rhsvh, d_zbh, d_gsum, d_kids, d_ps, d_dflag,
-                  d_dflag_init, d_pmap, d_part, d_part2, d_asm, d_recs, d_gasm, d_gtab, d_plans,
+  void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_b, d_x64, d_r64, d_ver, d_zh, d_rhsvh, d_zbh, d_gsum, d_kids, d_ps,
+                  d_pmap, d_part, d_part2, d_asm, d_recs, d_gasm, d_gtab, d_plans,
                   (void*)d_srcs, d_offs, d_counts};
   for (void* q : ptrs) if (q) (void)hipFree(q);
   for (auto q : d_ch) if (q) (void)hipFree(q);
@@ -284,8 +282,6 @@ void server_create(const cg_server_config* cfg, cg_server& S) {
   HIPC(hipMalloc(&S.d_kids, size_t(S.cap_ghost) * sizeof(GhostKids)));
   HIPC(hipMalloc(&S.d_ps, sizeof(ProbState) * S.nslots));
   HIPC(hipMemsetAsync(S.d_ps, 0, sizeof(ProbState) * S.nslots, S.stream));
-  HIPC(hipMalloc(&S.d_dflag, sizeof(int32_t) * S.nslots));
-  HIPC(hipMalloc(&S.d_dflag_init, sizeof(int32_t) * S.nslots));
   HIPC(hipMalloc(&S.d_pmap, sizeof(int32_t) * S.max_probs));
   HIPC(hipMalloc(&S.d_part, sizeof(double) * S.cap_leaf));
   HIPC(hipMalloc(&S.d_part2, sizeof(double) * S.cap_leaf));
@@ -337,7 +333,6 @@ void server_create(const cg_server_config* cfg, cg_server& S) {
   P.d_gsum = S.d_gsum;
   P.d_kids = S.d_kids;
   P.d_ps = S.d_ps;
-  P.d_dflag = S.d_dflag;
   P.d_pmap = S.d_pmap;
   P.d_part = S.d_part;
   P.d_part2 = S.d_part2;
@@ -780,9 +775,7 @@ void server_start_queued(cg_server& S, int k) {
         c);
     else k_cg_init_warm<float><<<G.leaf.n, 64, 0, st>>>(GL(S, G.leaf), G.leaf.n, 0, S.d_b, c);
   }
-  Ctx ci = group_ctx(S);
-  ci.dflag = S.d_dflag_init;
-  launch_finalize(st, G.n, S.view.max_leaf, ci, FIN_BB, 0);
+  launch_finalize(st, G.n, S.view.max_leaf, group_ctx(S), FIN_BB, 0);
   HIPC(hipGetLastError());
 }
 
