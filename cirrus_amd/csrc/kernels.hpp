@@ -298,10 +298,44 @@ __device__ __forceinline__ int pick4(int g, int a, int b, int c, int d) {
 // The quotient a / d, correctly rounded, from rd = 1/d in FP64 (within 2^-51
 // of it): the product's relative error is below 2^-50, and a quotient of two
 // 24-bit significands lies at least 2^-49 (relative) from every rounding
-// boundary of FP32, so the conversion rounds to the same value (results below
-// 2^-126, where FP32 has fewer bits, within one unit of their last place).
-// 4 issue slots against 15.5 for the FP32 division on gfx950.
+// boundary of FP32, so the conversion rounds to the same value.  Below 2^-126,
+// where FP32 has fewer bits, a quotient can lie on a boundary, a multiple of
+// 2^-150 (else it is at least 2^-48 away from one): where the product is within
+// 2^-49 of such a multiple, that is the quotient (div_again, run for subnormal
+// results; a result of 0 is right as it is).  4 issue slots and one for the test
+// against 15.5 for the FP32 division on gfx950.
 __device__ __forceinline__ float div_by(float a, double rd) { return float(double(a) * rd); }
+__device__ __forceinline__ bool subnormal(float q) { return __builtin_amdgcn_classf(q, 0x90); }
+__device__ __forceinline__ float div_again(float q, float a, double rd) {
+  constexpr double kToGrid = 0x1.8p-98;  // adding it leaves a multiple of 2^-150
+  const double v = double(a) * rd, t = (v + kToGrid) - kToGrid;
+  return subnormal(q) && __builtin_fabs(v - t) <= __builtin_fabs(v) * 0x1p-49 ? float(t) : q;
+}
+__device__ __forceinline__ float div_by_checked(float a, double rd) {
+  float q = div_by(a, rd);
+  if (__builtin_expect(subnormal(q), 0)) q = div_again(q, a, rd);
+  return q;
+}
+// The same without a test, where a branch is on the critical path: the product
+// rounded to 50 bits (9 v - (9 v - v)) is still on its side of every boundary that
+// it is not on, and is the quotient where that has 25 bits (rd within 2^-52 of 1/d).
+__device__ __forceinline__ float div_by_rounded(float a, double rd) {
+  const double v = double(a) * rd, c = 9.0 * v;
+  return float(c - (c - v));
+}
+// Four quotients with one test for all.
+__device__ __forceinline__ void div4_by(const float a[4], double r0, double r1, double r2, double r3, float q[4]) {
+  q[0] = div_by(a[0], r0);
+  q[1] = div_by(a[1], r1);
+  q[2] = div_by(a[2], r2);
+  q[3] = div_by(a[3], r3);
+  if (__builtin_expect(int(subnormal(q[0])) | int(subnormal(q[1])) | int(subnormal(q[2])) | int(subnormal(q[3])), 0)) {
+    q[0] = div_again(q[0], a[0], r0);
+    q[1] = div_again(q[1], a[1], r1);
+    q[2] = div_again(q[2], a[2], r2);
+    q[3] = div_again(q[3], a[3], r3);
+  }
+}
 // 1/d in FP64 for finite d != 0: the FP32 reciprocal and two Newton steps (a
 // divisor beyond the range where that reciprocal is a normal number: the division).
 __device__ __forceinline__ double recip64(float d) {
@@ -911,10 +945,10 @@ struct GsCoef {
 __device__ __forceinline__ GsCoef gs_coef(const TileRec& T) {
   return GsCoef{T.bc, T.h, T.h3, T.rdiag, tr_all_open(T), tr_uniform(T), tr_h_pow2(T)};
 }
-// b - A x of an open cell from its row sum: ((s h) h) h, one exact product when h
-// is a power of two (then b - s h3 rounds once either way).
+// b - A x of an open cell from its row sum: ((s h) h) h, one product when h is a
+// power of two (all three are then exact but where the last leaves FP32's range).
 __device__ __forceinline__ float open_residual(const GsCoef& G, float s, float b) {
-  return G.p2 ? __builtin_fmaf(-s, G.h3, b) : b - ((s * G.h) * G.h) * G.h;
+  return b - (G.p2 ? s * G.h3 : ((s * G.h) * G.h) * G.h);
 }
 // 1/D of a lane's open cells: those inside the pencil (mid) and at its ends
 // k = 0 (lo) and k = 7 (hi), the sums formed as cell_row_m forms them (0: D is 0).
@@ -960,6 +994,7 @@ __device__ __forceinline__ float4 gs_quad(float4 X0, float4 XO, float4 XIM, floa
     const OpenDiag D = open_diag(G, bim, bip, bjm, bjp);
     const double dlo = p ? D.mid : D.lo, dhi = p ? D.hi : D.mid;  // of m = 0 and m = 3
     const float bkm = p ? bi : G.bc[2], bkp = p ? G.bc[5] : bi;   // of m = 0 (k - 1) and m = 3 (k + 1)
+    float res[4], q[4];
 #pragma unroll
     for (int m = 0; m < 4; m++) {
       const float x0 = comp4(X0, m);
@@ -972,10 +1007,10 @@ __device__ __forceinline__ float4 gs_quad(float4 X0, float4 XO, float4 XIM, floa
         s = __builtin_fmaf(m == 0 ? bkm : bi, x0 - comp4(XKM, m), s);
         s = __builtin_fmaf(m == 3 ? bkp : bi, x0 - comp4(XKP, m), s);
       }
-      const float res = ZERO ? comp4(B, m) - 0.f : open_residual(G, s, comp4(B, m));
-      nv[m] = x0 + div_by(res, m == 0 ? dlo : (m == 3 ? dhi : D.mid));
+      res[m] = ZERO ? comp4(B, m) - 0.f : open_residual(G, s, comp4(B, m));
     }
-    return make_float4(nv[0], nv[1], nv[2], nv[3]);
+    div4_by(res, dlo, D.mid, D.mid, dhi, q);
+    return make_float4(X0.x + q[0], X0.y + q[1], X0.z + q[2], X0.w + q[3]);
   }
 #pragma unroll
   for (int m = 0; m < 4; m++) {
@@ -1187,10 +1222,15 @@ __device__ __forceinline__ void tile_jacobi(const Ctx& c, const TileRec& T, int 
     const int i = lane_id() >> 3, j = lane_id() & 7;
     const OpenDiag D = open_diag(gs_coef(T), i == 0 ? T.bc[0] : T.bc[6], i == 7 ? T.bc[3] : T.bc[6],
                                  j == 0 ? T.bc[1] : T.bc[6], j == 7 ? T.bc[4] : T.bc[6]);
+    float res[8], q[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) res[k] = omega * (b[k] - ax[k]);
+    div4_by(res, D.lo, D.mid, D.mid, D.mid, q);
+    div4_by(res + 4, D.mid, D.mid, D.mid, D.hi, q + 4);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       const double rd = k == 0 ? D.lo : (k == 7 ? D.hi : D.mid);
-      out[k] = rd != 0.0 ? S.own[k] + div_by(omega * (b[k] - ax[k]), rd) : 0.f;
+      out[k] = rd != 0.0 ? S.own[k] + q[k] : 0.f;
     }
     store8_split(Y + size_t(T.self) * 512, lane_id(), out);
     return;
@@ -1491,11 +1531,6 @@ __device__ __forceinline__ float first_red(float b, float d) {
   const float delta = (d != 0.f) ? (b - 0.f) / d : 0.f;
   return vround<V>(0.f + delta);
 }
-// the same for a cell whose 1/D is rd
-template <class V>
-__device__ __forceinline__ float first_red_by(float b, double rd) {
-  return vround<V>(0.f + div_by(b - 0.f, rd));
-}
 
 // The first red-black iteration of a down-sweep level from the zero guess in
 // one launch: both colour passes of GMGSolver.cu:216-269 (colour 0 from x = 0,
@@ -1563,9 +1598,12 @@ __global__ __launch_bounds__(64) void k_gs_first(const TileRec* __restrict__ lis
   float4 hv;
   float xk;
   if (std_faces) {
-    hv = make_float4(first_red_by<V>(hbf.x, T.rdiag), first_red_by<V>(hbf.y, T.rdiag), first_red_by<V>(hbf.z, T.rdiag),
-                     first_red_by<V>(hbf.w, T.rdiag));
-    xk = first_red_by<V>(bk, T.rdiag);
+    const double rd = T.rdiag;
+    const float hb4[4] = {hbf.x - 0.f, hbf.y - 0.f, hbf.z - 0.f, hbf.w - 0.f};
+    float q4[4];
+    div4_by(hb4, rd, rd, rd, rd, q4);
+    hv = make_float4(vround<V>(0.f + q4[0]), vround<V>(0.f + q4[1]), vround<V>(0.f + q4[2]), vround<V>(0.f + q4[3]));
+    xk = vround<V>(0.f + div_by_checked(bk - 0.f, rd));
   } else {
     hv = make_float4(first_red<V>(hbf.x, hd.x), first_red<V>(hbf.y, hd.y), first_red<V>(hbf.z, hd.z),
                      first_red<V>(hbf.w, hd.w));
@@ -1892,41 +1930,19 @@ __device__ __forceinline__ void cl_gs(CoarseLDS& M, const CoarseCells& L, int co
     const CoarseCell& Q = L.P[col][m];
     const float x0 = cl_at(M, at);
     const float res = cl_residual(M, Q, x0, true, L.cf, L.h);  // used on INTERIOR cells only
-    nv[m] = vround<V>(x0 + (Q.rd != 0.0 ? div_by(res, Q.rd) : 0.f));
+    nv[m] = vround<V>(x0 + (Q.rd != 0.0 ? div_by_rounded(res, Q.rd) : 0.f));
   });
   cl_each<FULL>(L, col, [&](int m, uint32_t at) { cl_at(M, at) = nv[m]; });
   __syncthreads();
 }
 
-// Latency bound on one CU (a scalar round trip for the plan, one for the cells,
-// then about 30 passes with a barrier each), so what counts is the length of a
-// pass: the rows are prepared once and kept for the down- and the up-sweep,
-// neighbours are read without bank conflicts, and the division is a product with
-// the prepared reciprocal.  Nine tiles, two sweeps per level, ten bottom
-// iterations: 21.4 -> 13.5 us; six roots alone: 14.2 -> 10.2 us.  (Sixteen tiles
-// on level 1 were measured too: 27 us, no better than that level's grid-wide
-// launches.)
+// The V-cycle of the resident levels on prepared cells: z from 0, the rhs in the
+// cells of the finest level (and in M.b0 where level 0 has more than level 1
+// restricts to).  Leaves z in M.z; ends with a barrier if it did anything.
 template <class V>
-__global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __restrict__ plans, int flags, V* Z,
-                                                           VCycleArgs v, Ctx c) {
-  __shared__ CoarseLDS M;
+__device__ __forceinline__ void cl_vcycle(CoarseLDS& M, const CoarsePlan& cp, int n1, CoarseCells& L0, CoarseCells& L1,
+                                          const VCycleArgs& v) {
   const int tid = threadIdx.x;
-  const CoarsePlan& cp = plans[blockIdx.x];
-  const int n0 = cp.n0, n1 = cp.n1;
-  CoarseCells L0, L1;
-  {
-    const int32_t done = (flags & F_CHECK_DONE) ? c.ps[cp.prob].done : 0;
-    CoarseRaw R0, R1;
-    cl_issue<V>(c, cp, CL_ROOTS, n1, R1);
-    cl_issue<V>(c, cp, 0, n0, R0);
-    if (done) return;
-    if (tid < 4) M.z[CL_ZERO + tid] = 0.f;
-    cl_commit(cp, CL_ROOTS, n1, R1, M, L1);
-    cl_commit(cp, 0, n0, R0, M, L0);
-  }
-#pragma unroll
-  for (int col = 0; col < 2; col++) cl_each<false>(L0, col, [&](int m, uint32_t at) { M.b0[at >> 2] = L0.P[col][m].b; });
-  __syncthreads();
   constexpr uint32_t T0 = CL_ROOTS * 512;  // M.t starts at level 1's first cell
   // one damped-Jacobi sweep of level 1
   auto jacobi1 = [&]() {
@@ -1937,7 +1953,7 @@ __global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __r
         const bool in = (L1.in >> (2 * m + col)) & 1;
         const float x0 = cl_at(M, at);
         const float res = cl_residual(M, Q, x0, in, L1.cf, L1.h);
-        M.t[(at >> 2) - T0] = in ? (Q.rd != 0.0 ? x0 + div_by(v.omega * res, Q.rd) : 0.f) : x0;
+        M.t[(at >> 2) - T0] = in ? (Q.rd != 0.0 ? x0 + div_by_rounded(v.omega * res, Q.rd) : 0.f) : x0;
       });
     __syncthreads();
 #pragma unroll
@@ -1978,8 +1994,8 @@ __global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __r
   }
   for (int it = 0; it < it0; it++) { cl_gs<V, false>(M, L0, 0); cl_gs<V, false>(M, L0, 1); }
   for (int it = 0; it < it0; it++) { cl_gs<V, false>(M, L0, 1); cl_gs<V, false>(M, L0, 0); }
-  const int q0 = uni(tid >> 8), r = tid & 255;
   if (n1) {
+    const int q0 = uni(tid >> 8), r = tid & 255;
     // prolongation: x += pcoef * parent on INTERIOR cells, 0 elsewhere (the two
     // cells of a pair k = 2 e, 2 e + 1 have one parent cell)
     const int i = r >> 5, j = (r >> 2) & 7, e = r & 3;
@@ -1998,6 +2014,41 @@ __global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __r
       if (v.smoother != 0) jacobi1();
       else { cl_gs<V, true>(M, L1, 1); cl_gs<V, true>(M, L1, 0); }
     }
+  }
+}
+
+// Latency bound on one CU (a scalar round trip for the plan, one for the cells,
+// then about 30 passes with a barrier each), so what counts is the length of a
+// pass: the rows are prepared once and kept for the down- and the up-sweep,
+// neighbours are read without bank conflicts, and the division is a product with
+// the prepared reciprocal.  Nine tiles, two sweeps per level, ten bottom
+// iterations: 21.4 -> 13.5 us; six roots alone: 14.2 -> 10.2 us.  (Sixteen tiles
+// on level 1 were measured too: 27 us, no better than that level's grid-wide
+// launches.)
+template <class V>
+__global__ __launch_bounds__(CL_THREADS) void k_coarse_lds(const CoarsePlan* __restrict__ plans, int flags, V* Z,
+                                                           VCycleArgs v, Ctx c) {
+  __shared__ CoarseLDS M;
+  const int tid = threadIdx.x;
+  const CoarsePlan& cp = plans[blockIdx.x];
+  const int n0 = cp.n0, n1 = cp.n1;
+  CoarseCells L0, L1;
+  {
+    const int32_t done = (flags & F_CHECK_DONE) ? c.ps[cp.prob].done : 0;
+    CoarseRaw R0, R1;
+    cl_issue<V>(c, cp, CL_ROOTS, n1, R1);
+    cl_issue<V>(c, cp, 0, n0, R0);
+    if (done) return;
+    if (tid < 4) M.z[CL_ZERO + tid] = 0.f;
+    cl_commit(cp, CL_ROOTS, n1, R1, M, L1);
+    cl_commit(cp, 0, n0, R0, M, L0);
+  }
+#pragma unroll
+  for (int col = 0; col < 2; col++) cl_each<false>(L0, col, [&](int m, uint32_t at) { M.b0[at >> 2] = L0.P[col][m].b; });
+  __syncthreads();
+  cl_vcycle<V>(M, cp, n1, L0, L1, v);
+  const int q0 = uni(tid >> 8), r = tid & 255;
+  if (n1) {
 #pragma unroll
     for (int col = 0; col < 2; col++)
       cl_each<true>(L1, col, [&](int m, uint32_t at) {
@@ -3151,7 +3202,7 @@ __device__ __forceinline__ void amg_cl_gs(CoarseLDS& M, const AmgCells& L, int c
     const AmgCell& Q = L.P[col][m];
     const float x0 = cl_at(M, at);
     const float res = amg_cell_residual(M, Q, x0);
-    cl_at(M, at) = x0 + (Q.rd != 0.0 ? div_by(res, Q.rd) : 0.f);
+    cl_at(M, at) = x0 + (Q.rd != 0.0 ? div_by_rounded(res, Q.rd) : 0.f);
   });
   __syncthreads();
 }

@@ -12,8 +12,6 @@ import pytest
 import cirrus_amd as ca
 import pyoracle as po
 
-pytestmark = pytest.mark.gpu
-
 SCENES = {
     "uniform": dict(kind=po.SCENE_UNIFORM, uniform_level=2, has_solid=0),
     "band": dict(kind=po.SCENE_SPHERE_BAND, band_level=[4, 3, 2], band_r=0.15),
@@ -22,6 +20,7 @@ SCENES = {
 }
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("scene", sorted(SCENES))
 @pytest.mark.parametrize("h0", [0.125, 0.1, 0.3])
 @pytest.mark.parametrize("smoother,storage,nu", [(ca.SMOOTH_RBGS, ca.STORE_F32, 2), (ca.SMOOTH_RBGS, ca.STORE_F32, 3),
@@ -43,6 +42,7 @@ def test_open_tiles_give_the_oracle_solve(scene, h0, smoother, storage, nu):
         assert np.array_equal(P.get(ca.CH_X)[typ == po.LEAF], xo), fused16
 
 
+@pytest.mark.gpu
 def test_open_tiles_of_several_cell_sizes_in_one_batch():
     items = []
     for h0 in (0.125, 0.1, 0.25, 0.3):
@@ -59,3 +59,68 @@ def test_open_tiles_of_several_cell_sizes_in_one_batch():
         assert (res[k]["iters"], res[k]["rr"]) == (ro["iters"], ro["rr"]), k
         m = typ == po.LEAF
         assert np.array_equal(X[k][m], o.get(po.CH_X).astype(np.float32)[m]), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h0", [0.125, 0.3])
+def test_subnormal_quotients_round_as_division(h0):
+    """A sweep from x = 0 leaves b / D; with b near the lowest FP32 values the
+    quotients are subnormal, where many lie halfway between two."""
+    o = po.Oracle(h0=h0, seed=7, **SCENES["band"])
+    lev, crd, typ, nbr = o.topology()
+    P = ca.Problem(ca.Tree(o.params.h0, lev, crd, typ, o.celltypes()))
+    b = np.random.default_rng(1).integers(-1 << 14, 1 << 14, (P.n, 512)).astype(np.float32) * np.float32(2.0 ** -149)
+    for level in range(P.max_level + 1):
+        for sweep in ("rbgs", "jacobi"):
+            for X in (o, P):
+                X.set(po.CH_Z, np.zeros((P.n, 512), np.float32))
+                X.set(po.CH_TMP, b)
+            if sweep == "rbgs":
+                o.gs_color(level, po.CH_Z, po.CH_TMP, 0)
+                ca.GaussSeidelColor(P, level, ca.CH_Z, ca.CH_TMP, 0)
+            else:
+                o.jacobi_sweep(level, po.CH_Z, po.CH_TMP, 1.0)
+                ca.JacobiSweep(P, level, ca.CH_Z, ca.CH_TMP, 1.0)
+            assert np.array_equal(P.get(ca.CH_Z), o.get(po.CH_Z).astype(np.float32)), (level, sweep)
+
+
+@pytest.mark.parametrize("err", [0.0, 2.0 ** -52, -(2.0 ** -52), 2.0 ** -51, -(2.0 ** -51)])
+def test_subnormal_quotients_from_a_reciprocal(err):
+    """The kernels' steps in numpy: a quotient below 2^-126 from a 64-bit
+    reciprocal off by err, taken to the multiple of 2^-150 within 2^-49 of it,
+    rounds as the exact quotient does (halfway cases made on purpose)."""
+    rng = np.random.default_rng(9)
+    n = 1 << 20
+    d = np.ldexp(rng.integers(1 << 23, 1 << 24, n).astype(np.float64), rng.integers(-30, 2, n)).astype(np.float32)
+    a = np.ldexp(rng.integers(1, 1 << 24, n).astype(np.float64), -149).astype(np.float32)  # any subnormal or small normal value
+    m = n // 2  # halfway: a = d (k + 1/2) 2^-149, d a small integer times a power of two
+    d[:m] = rng.integers(1, 64, m) * np.float32(0.5)
+    a[:m] = (d[:m].astype(np.float64) * (rng.integers(0, 1 << 12, m) + 0.5) * 2.0 ** -149).astype(np.float32)
+    rd = (1.0 / d.astype(np.float64)) * (1.0 + err)
+    v = a.astype(np.float64) * rd
+    q = v.astype(np.float32)
+    t = (v + 1.5 * 2.0 ** -98) - 1.5 * 2.0 ** -98
+    sub = (q != 0) & (np.abs(q) < np.float32(2.0 ** -126))
+    q = np.where(sub & (np.abs(v - t) <= np.abs(v) * 2.0 ** -49), t.astype(np.float32), q)
+    assert sub.mean() > 0.4
+    assert np.array_equal(q, a / d)
+
+
+@pytest.mark.parametrize("err", [0.0, 2.0 ** -53, -(2.0 ** -53)])
+@pytest.mark.parametrize("low", [False, True])
+def test_quotients_rounded_to_fifty_bits(err, low):
+    """The branch-free form: the product with a reciprocal (one unit of its last
+    place off at most) rounded to 50 bits, then to FP32."""
+    rng = np.random.default_rng(10)
+    n = 1 << 20
+    d = np.ldexp(rng.integers(1 << 23, 1 << 24, n).astype(np.float64), rng.integers(-30, 2, n)).astype(np.float32)
+    if low:
+        a = np.ldexp(rng.integers(1, 1 << 24, n).astype(np.float64), -149).astype(np.float32)
+        m = n // 2
+        d[:m] = rng.integers(1, 64, m) * np.float32(0.5)
+        a[:m] = (d[:m].astype(np.float64) * (rng.integers(0, 1 << 12, m) + 0.5) * 2.0 ** -149).astype(np.float32)
+    else:
+        a = np.ldexp(rng.integers(1 << 23, 1 << 24, n).astype(np.float64), rng.integers(-60, 20, n)).astype(np.float32)
+    v = a.astype(np.float64) * ((1.0 / d.astype(np.float64)) * (1.0 + err))
+    c = 9.0 * v
+    assert np.array_equal((c - (c - v)).astype(np.float32), a / d)
