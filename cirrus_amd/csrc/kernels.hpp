@@ -2629,6 +2629,223 @@ __global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_
   }
 }
 
+// ---------------------------------------------------------------------------
+// CG of a problem whose every level is LDS-resident: up to `iters` iterations in
+// one launch of one workgroup.  Launch by launch such an iteration was one of this
+// kernel's V-cycles and seven launches of 2.2 to 3.7 us for eight tiles of vector
+// work each.  Here r, p, A p and z stay in LDS (colour-split, so that the rows are
+// those of the V-cycle), x in registers, and an iteration is the V-cycle's passes
+// and seven barriers: the vector part's cells are the threads' own cells of the
+// finest level, and for a tile's dot partial one wavefront reads its pencils and
+// adds them in the order of the per-tile kernels.  One 16^3 box (9 tiles, two
+// sweeps a level), 19 iterations: 790 -> 360 us a solve, 10 us of it an iteration,
+// bound by the V-cycle's chain of some forty passes with a barrier each.
+// ---------------------------------------------------------------------------
+struct SmallLDS {
+  float p[CL_ZERO + 4];        // in v.z's layout, so that a cell's neighbour addresses serve both
+  CoarseLDS v;                 // v.t: A p outside the V-cycle
+  float r[CL_CHILDREN * 512];  // from the finest level's first slot
+  double part[3][CL_CHILDREN];
+  ProbState out;               // the state to leave (thread 0's)
+};
+// A tile's sum over the 64 pencils (lanes) of f(cell values of the pencil in order).
+__device__ __forceinline__ void sm_pencil(const float* a, float o[8]) {  // a: the tile's colour-split cells
+  float4 q0, q1;
+  load_pencil_split(a, lane_id(), q0, q1);
+  o[0] = q0.x; o[1] = q0.y; o[2] = q0.z; o[3] = q0.w;
+  o[4] = q1.x; o[5] = q1.y; o[6] = q1.z; o[7] = q1.w;
+}
+__device__ __forceinline__ double sm_dot(const float* a, const float* b) {
+  float x[8], y[8];
+  sm_pencil(a, x);
+  sm_pencil(b, y);
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) s += double(x[k]) * double(y[k]);
+  return wave_sum(s);
+}
+// The sum of n <= 64 partials as block_sum_partials forms it (every wavefront).
+__device__ __forceinline__ double sm_total(const double* part, int n) {
+  const int lane = lane_id();
+  return wave_sum(0.0 + (lane < n ? part[lane < n ? lane : 0] : -0.0));
+}
+// KIDS: the problem's LEAF tiles are the children of its one root; else its roots.
+template <class V, bool KIDS>
+__device__ __forceinline__ void sm_solve(SmallLDS& S, const CoarsePlan& cp, int iters, int flags, V* Z, const VCycleArgs& v,
+                                         const Ctx& c) {
+  CoarseLDS& M = S.v;
+  const int tid = threadIdx.x, wave = uni(tid >> 6), q0 = uni(tid >> 8), r = tid & 255;
+  constexpr int first = KIDS ? CL_ROOTS : 0;
+  const int n = KIDS ? CL_CHILDREN : cp.n0;  // LEAF tiles
+  ProbState* ps = c.ps + cp.prob;
+  const ProbState st = state_of(state_word(ps));
+  if ((flags & F_CHECK_DONE) && st.done) return;
+  CoarseCells L0, L1;
+  {
+    CoarseRaw R0, R1;
+    if (KIDS) cl_issue<V>(c, cp, CL_ROOTS, CL_CHILDREN, R1);
+    cl_issue<V>(c, cp, 0, cp.n0, R0);
+    if (KIDS) cl_commit(cp, CL_ROOTS, CL_CHILDREN, R1, M, L1);
+    cl_commit(cp, 0, cp.n0, R0, M, L0);
+  }
+  if (tid < 4) M.z[CL_ZERO + tid] = S.p[CL_ZERO + tid] = 0.f;
+  CoarseCells& L = KIDS ? L1 : L0;
+  auto p_at = [&](uint32_t byte) -> float& { return *reinterpret_cast<float*>(reinterpret_cast<char*>(S.p) + byte); };
+  // natural cell index (in its tile) of the thread's cell of colour col
+  auto nat = [&](int col) {
+    const int i = r >> 5, j = (r >> 2) & 7;
+    return (i << 6) + (j << 3) + 2 * (r & 3) + ((col + i + j) & 1);
+  };
+  float x[2][CL_CPT];
+  auto tile_of = [&](int m) { return size_t(cp.slots[first + q0 + 4 * m].tile) * 512; };
+  auto leaf_at = [&](uint32_t at) { return (at >> 2) - first * 512; };  // index into S.r, M.t
+#pragma unroll
+  for (int col = 0; col < 2; col++)
+    cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+      const size_t g = tile_of(m) + nat(col);
+      x[col][m] = c.x[g];
+      S.r[leaf_at(at)] = c.r[g];
+      p_at(at) = c.p[g];
+    });
+  __syncthreads();
+  auto interior = [&](int col, int m) { return ((L.in >> (2 * m + col)) & 1) != 0; };
+  double gamma = st.gamma, alpha = st.alpha;
+  int it = st.iter, done = st.done;
+  if (tid == 0) S.out = st;
+  for (int k = 0; k < iters && !done; k++) {
+    if (st.pure_neumann) {  // k_mean, FIN_MEAN, k_subtract_mean
+      if (wave < n) {
+        float w[8];
+        sm_pencil(S.r + wave * 512, w);
+        const uint64_t ct = load_ct8(c.ctype + size_t(cp.slots[first + wave].tile) * 512 + lane_id() * 8);
+        double a = 0.0, q = 0.0;
+#pragma unroll
+        for (int e = 0; e < 8; e++) { a += double(w[e]); q += (ct_at(ct, e) & C_INT) ? 1.0 : 0.0; }
+        a = wave_sum(a);
+        q = wave_sum(q);
+        if (lane_id() == 0) { S.part[0][wave] = a; S.part[1][wave] = q; }
+      }
+      __syncthreads();
+      const double mean = sm_total(S.part[0], n) / sm_total(S.part[1], n);
+      if (tid == 0) S.out.mean = mean;
+#pragma unroll
+      for (int col = 0; col < 2; col++)
+        cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+          if (interior(col, m)) S.r[leaf_at(at)] = float(double(S.r[leaf_at(at)]) - mean);
+        });
+    }
+    // z = M^-1 r
+#pragma unroll
+    for (int col = 0; col < 2; col++) {
+      cl_each<false>(L0, col, [&](int, uint32_t at) { cl_at(M, at) = 0.f; });
+      if (KIDS) cl_each<true>(L1, col, [&](int, uint32_t at) { cl_at(M, at) = 0.f; });
+      cl_each<KIDS>(L, col, [&](int m, uint32_t at) { L.P[col][m].b = vround<V>(S.r[leaf_at(at)]); });
+    }
+    __syncthreads();
+    cl_vcycle<V>(M, cp, KIDS ? CL_CHILDREN : 0, L0, L1, v);
+    // gamma = r.z, beta
+    if (wave < n) {
+      const double a = sm_dot(S.r + wave * 512, M.z + (first + wave) * 512);
+      if (lane_id() == 0) S.part[2][wave] = a;
+    }
+    __syncthreads();
+    const double gamma_old = gamma;
+    gamma = sm_total(S.part[2], n);
+    const double beta = it == 0 ? 0.0 : gamma / gamma_old;
+    if (tid == 0) {
+      S.out.gamma_old = gamma_old;
+      S.out.beta = beta;
+    }
+    // the last iteration's x, p = z + beta p
+    const float fb = float(beta), fa = float(alpha);
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+        if (!interior(col, m)) return;
+        float& p = p_at(at);
+        if (it > 0) x[col][m] = __builtin_fmaf(fa, p, x[col][m]);
+        p = __builtin_fmaf(fb, p, cl_at(M, at));
+      });
+    __syncthreads();
+    // A p
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+        const CoarseCell& Q = L.P[col][m];
+        const float p = p_at(at);
+        float sum = 0.f;
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+          sum = __builtin_fmaf(L.cf, p - p_at(Q.nb[f] & 0xffffu), sum);
+          sum = __builtin_fmaf(L.cf, p - p_at(Q.nb[f] >> 16), sum);
+        }
+        M.t[leaf_at(at)] = interior(col, m) ? ((sum * L.h) * L.h) * L.h : 0.f;
+      });
+    __syncthreads();
+    if (wave < n) {
+      const double a = sm_dot(S.p + (first + wave) * 512, M.t + wave * 512);
+      if (lane_id() == 0) S.part[0][wave] = a;
+    }
+    __syncthreads();
+    const double pap = sm_total(S.part[0], n);
+    if (tid == 0) S.out.pAp = pap;
+    alpha = gamma / pap;
+    const float na = -float(alpha);
+#pragma unroll
+    for (int col = 0; col < 2; col++)
+      cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+        if (interior(col, m)) S.r[leaf_at(at)] = __builtin_fmaf(na, M.t[leaf_at(at)], S.r[leaf_at(at)]);
+      });
+    __syncthreads();
+    if (wave < n) {
+      const double a = sm_dot(S.r + wave * 512, S.r + wave * 512);
+      if (lane_id() == 0) S.part[1][wave] = a;
+    }
+    __syncthreads();
+    const double rr = sm_total(S.part[1], n);
+    it++;
+    const int cs = st.check_stride;
+    const bool converged = cs > 0 && it % cs == 0 && rr < st.thr;
+    if (converged || it >= st.max_iters) done = 1;
+    if (tid == 0) {
+      S.out.rr = rr;
+      if (converged) S.out.converged = 1;
+    }
+  }
+  // back to memory, as the launches of the last iteration would leave it
+#pragma unroll
+  for (int col = 0; col < 2; col++) {
+    cl_each<KIDS>(L, col, [&](int m, uint32_t at) {
+      const size_t g = tile_of(m) + nat(col);
+      c.x[g] = x[col][m];
+      c.p[g] = p_at(at);
+      c.r[g] = S.r[leaf_at(at)];
+      c.ap[g] = M.t[leaf_at(at)];
+      vc_rhs<V>(c)[tile_of(m) + col * 256 + r] = from_f<V>(S.r[leaf_at(at)]);
+      Z[tile_of(m) + col * 256 + r] = from_f<V>(cl_at(M, at));
+    });
+    if (KIDS)
+      cl_each<false>(L0, col, [&](int m, uint32_t at) {
+        Z[size_t(cp.slots[q0 + 4 * m].tile) * 512 + col * 256 + r] = from_f<V>(cl_at(M, at));
+      });
+  }
+  if (tid != 0) return;
+  S.out.gamma = gamma;
+  S.out.alpha = alpha;
+  S.out.iter = it;
+  S.out.done = done;
+  *ps = S.out;
+  if (c.progress) __hip_atomic_store(c.progress + cp.prob, 2 * it + done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+template <class V>
+__global__ __launch_bounds__(CL_THREADS) void k_cg_small(const CoarsePlan* __restrict__ plans, int iters, int flags, V* Z,
+                                                         VCycleArgs v, Ctx c) {
+  __shared__ SmallLDS S;
+  const CoarsePlan& cp = plans[blockIdx.x];
+  if (cp.n1) sm_solve<V, true>(S, cp, iters, flags, Z, v, c);
+  else sm_solve<V, false>(S, cp, iters, flags, Z, v, c);
+}
+
 // Pure-Neumann re-centring (MeanAsync + ReCenterLeafVoxels,
 // PoissonGrid.cu:231-325, PoissonSolver.cu:356-368): mean of r over all cells
 // of LEAF tiles divided by the INTERIOR count, subtracted on INTERIOR cells.

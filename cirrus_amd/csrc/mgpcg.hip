@@ -1083,6 +1083,32 @@ void enqueue_amg_vcycle(cg_problem& P, const VParams& v) {
   k_to_split<<<unsigned(P.leaf.n), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, X, c.z);
 }
 
+// Handles whose every problem is LDS-resident, all its LEAF tiles on one level,
+// run whole iterations in one launch (k_cg_small), as many as kSmallIters before
+// the host is asked again: 16 iterations of boxes of 9 tiles, by launches and so,
+// 1 box 617 and 255 us, 256 boxes 974 and 399, 2,048 boxes 4,969 and 3,238.
+constexpr int kSmallIters = 16;
+bool runs_small(const cg_problem& P) {
+  if (int(P.plans.size()) != P.nprob || P.ghosts.n) return false;
+  for (const DList& l : P.lvlg) if (l.n) return false;
+  for (int q = 0; q < P.nprob; q++) {
+    const CoarsePlan& cp = P.plans[q];
+    if (cp.prob != q || (cp.n1 != 0 && cp.n0 != 1) || P.leaf_count[q] != (cp.n1 ? cp.n1 : cp.n0)) return false;
+  }
+  return true;
+}
+template <class V>
+void enqueue_cg_small(cg_problem& P, const VParams& v, int iters) {
+  k_cg_small<V><<<unsigned(P.nprob), CL_THREADS, 0, P.stream>>>(
+      P.d_plans, iters, F_VCYCLE | F_CHECK_DONE, pool_z<V>(P), VCycleArgs{v.nu, v.coarsest, v.smoother, v.omega, v.ooa, v.pcoef},
+      P.ctx());
+}
+void enqueue_cg_small(cg_problem& P, const VParams& v, int iters, int storage) {
+  if (storage == CG_STORE_BF16) enqueue_cg_small<bf16>(P, v, iters);
+  else if (storage == CG_STORE_F16) enqueue_cg_small<f16>(P, v, iters);
+  else enqueue_cg_small<float>(P, v, iters);
+}
+
 // starts with the V-cycle): [re-centre r], z = M^-1 r, gamma/beta, p, A p and
 // alpha, x/r and the convergence test.
 template <class V>
@@ -1320,8 +1346,10 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   // solve by stream launches with a busy host, 2 % less than by replay with an idle
   // one, 4.0 ms by replay; 14,345 tiles (5.3 us a launch): 3.47 ms and 3.53.
   constexpr int kStreamMinTiles = 8192;
+  const bool small = !amg && runs_small(P);
+  const int chunk = small ? std::max(stride, kSmallIters) : stride;
   const bool use_graph = prm.use_graph > 0 || (prm.use_graph < 0 && (amg || P.n < kStreamMinTiles));
-  if (use_graph && P.graph_key != keybuf) {
+  if (use_graph && !small && P.graph_key != keybuf) {
     if (P.graph) HIPC(hipGraphExecDestroy(P.graph));
     P.graph = nullptr;
     hipGraph_t g;
@@ -1339,10 +1367,13 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   // Follow the device one chunk behind the enqueue front, so it never waits for
   // the host; iterations after convergence exit at their first load.
   for (int enq = 0; enq < max_iters;) {
-    for (int s = 0; s < stride; s++) one_iter();
+    if (small) enqueue_cg_small(P, v, chunk, prm.storage);
+    else
+      for (int s = 0; s < chunk; s++) one_iter();
     HIPC(hipGetLastError());
     if (enq > 0 && wait_progress(P, enq)) break;
-    enq += stride;
+    if (max_iters - enq <= chunk) break;
+    enq += chunk;
   }
   // the last iteration's x update (k_cg_update_p applies each earlier one)
   k_cg_finish_x<<<grid_for(P.leaf.n, P.swz), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, P.swz | (c.inert ? F_INERT : 0), c);
