@@ -2935,7 +2935,7 @@ __device__ __forceinline__ double tile_dot(const float* __restrict__ A, const fl
   for (int k = 0; k < 8; k++) s += double(a[k]) * double(b[k]);
   return wave_sum(s);
 }
-__global__ __launch_bounds__(64) void k_dot_tiles(Ctx c, const TileRec* __restrict__ list, int n, const float* __restrict__ A,
+__global__ __launch_bounds__(64) void k_dot_tiles(const TileRec* __restrict__ list, int n, const float* __restrict__ A,
                                                   const float* __restrict__ Bv, double* __restrict__ part) {
   const int flags = 0;
   TILE_KERNEL_PROLOGUE

@@ -128,7 +128,6 @@ struct cg_problem {
   CoarsePlan* d_plans = nullptr;
   double* d_part = nullptr;
   double* d_part2 = nullptr;
-  double* d_scalar = nullptr;
   TileRec* d_lists = nullptr;
   TileRec* d_tiles = nullptr;    // every tile's record in canonical order (the worklists are gathered from it)
   TileRec* d_tmp_list = nullptr;
@@ -136,7 +135,8 @@ struct cg_problem {
   int32_t* d_ext = nullptr;      // internal tile -> caller index (channel moves from and to device buffers)
   hipStream_t stream = nullptr;
   ProbState* h_ps = nullptr;     // pinned staging of the ProbState uploads and of the final states
-  int32_t* h_prog = nullptr;     // Ctx::progress (pinned, behind h_ps in its allocation)
+  double* h_scalar = nullptr;    // a kernel's result for the host (pinned, behind h_ps in its allocation)
+  int32_t* h_prog = nullptr;     // Ctx::progress (behind h_scalar)
   hipEvent_t ev_ps = nullptr;    // recorded after the last upload from h_ps
   bool ps_pending = false;
   hipEvent_t ev_io[2] = {nullptr, nullptr};  // orders device channel moves against the caller's stream
@@ -186,7 +186,7 @@ cg_problem::~cg_problem() {
   if (h_ps) (void)hipHostFree(h_ps);
   if (ev_ps) (void)hipEventDestroy(ev_ps);
   void* ptrs[] = {d_ctype, d_inert, d_fmask, d_diag, d_zb, d_zh, d_rhsvh, d_zbh, d_x64, d_r64, d_bsave, d_psum, d_gsum, d_ps,
-                  d_plans, d_part, d_part2, d_scalar, d_lists, d_tiles, d_tmp_list, d_amgc, d_amgct, d_ext};
+                  d_plans, d_part, d_part2, d_lists, d_tiles, d_tmp_list, d_amgc, d_amgct, d_ext};
   for (void* q : ptrs) if (q) (void)hipFree(q);
   for (auto q : d_ch) if (q) (void)hipFree(q);
   for (auto q : d_api) if (q) (void)hipFree(q);
@@ -651,7 +651,6 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
   size_t np = size_t(std::max(n, 64));
   HIPC(hipMalloc(&P.d_part, np * sizeof(double)));
   HIPC(hipMalloc(&P.d_part2, np * sizeof(double)));
-  HIPC(hipMalloc(&P.d_scalar, 8 * sizeof(double)));
   HIPC(hipMalloc(&P.d_tiles, sizeof(TileRec) * size_t(n)));
   HIPC(hipMemcpyAsync(P.d_tiles, P.tiles.data(), sizeof(TileRec) * size_t(n), hipMemcpyHostToDevice, P.stream));
   upload_schedule(P, sched_ids);
@@ -668,8 +667,9 @@ void build_pool(const cg_tree_desc* descs, int nprob, cg_problem& P) {
   k_face_mask<<<P.all.n, 64, 0, P.stream>>>(P.d_ctype, P.d_fmask, P.d_fsplit, P.L(P.all), P.all.n);
   k_diag<<<P.all.n, 64, 0, P.stream>>>(P.ctx(), P.L(P.all), P.all.n, P.d_diag);
   HIPC(hipGetLastError());
-  HIPC(hipHostMalloc(&P.h_ps, (sizeof(ProbState) + sizeof(int32_t)) * nprob, hipHostMallocCoherent));
-  P.h_prog = reinterpret_cast<int32_t*>(P.h_ps + nprob);
+  HIPC(hipHostMalloc(&P.h_ps, (sizeof(ProbState) + sizeof(int32_t)) * nprob + sizeof(double), hipHostMallocCoherent));
+  P.h_scalar = reinterpret_cast<double*>(P.h_ps + nprob);
+  P.h_prog = reinterpret_cast<int32_t*>(P.h_scalar + 1);
   HIPC(hipEventCreateWithFlags(&P.ev_ps, hipEventDisableTiming));
   HIPC(hipEventCreateWithFlags(&P.ev_io[0], hipEventDisableTiming));
   HIPC(hipEventCreateWithFlags(&P.ev_io[1], hipEventDisableTiming));
@@ -1167,18 +1167,32 @@ const TileRec* tmp_list(cg_problem& P, const std::vector<int>& tiles) {
   return P.d_tmp_list;
 }
 
-double dot_types(cg_problem& P, const float* A, const float* B, int types) {
+// The tiles of the given types in canonical order: a list of the handle where one
+// holds just these, else an uploaded one.  (A dot of the 3,424 LEAF tiles of the
+// adaptive 256^3 problem through uploaded records, its result copied back, took
+// 72 us; through the handle's list, the result written to host memory, 21.5.)
+const TileRec* list_of_types(cg_problem& P, int types, int& n) {
+  const int t = types & (LEAF | NONLEAF | GHOST);
+  const DList* own = t == LEAF ? &P.leaf : t == (LEAF | GHOST) ? &P.applyl : t == GHOST ? &P.ghosts
+                     : t == (LEAF | NONLEAF | GHOST) ? &P.all : nullptr;
+  if (own) {
+    n = own->n;
+    return P.L(*own);
+  }
   std::vector<int> l;
   for (int i = 0; i < P.n; i++) if (tr_type(P.tiles[i]) & types) l.push_back(i);
-  if (l.empty()) return 0.0;
-  const TileRec* dl = tmp_list(P, l);
-  const Ctx c = P.ctx();
-  k_dot_tiles<<<unsigned(l.size()), 64, 0, P.stream>>>(c, dl, int(l.size()), A, B, P.d_part);
-  launch_sum(P.stream, P.d_part, int(l.size()), P.d_scalar);
-  double out = 0;
-  HIPC(hipMemcpyAsync(&out, P.d_scalar, sizeof(double), hipMemcpyDeviceToHost, P.stream));
+  n = int(l.size());
+  return n ? tmp_list(P, l) : nullptr;
+}
+double dot_types(cg_problem& P, const float* A, const float* B, int types) {
+  int n = 0;
+  const TileRec* list = list_of_types(P, types, n);
+  if (n == 0) return 0.0;
+  k_dot_tiles<<<unsigned(n), 64, 0, P.stream>>>(list, n, A, B, P.d_part);
+  launch_sum(P.stream, P.d_part, n, P.h_scalar);
+  HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(P.stream));
-  return out;
+  return *P.h_scalar;
 }
 
 void full_negative_laplacian(cg_problem& P, float* X, float* AX, int diag) {

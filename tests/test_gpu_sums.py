@@ -38,3 +38,19 @@ def test_sums_of_several_problems(counts):
     for r, (o, _) in zip(res, items):
         ro = o.solve(max_iters=3, tol=1e-12, level_iters=1, coarsest_iters=2)
         assert (r["iters"], r["rr"], r["bb"]) == (ro["iters"], ro["rr"], ro["bb"])
+
+
+@pytest.mark.parametrize("kw", [dict(kind=po.SCENE_SPHERE_BAND, band_level=[4, 3, 2]), dict(kind=po.SCENE_UNIFORM, uniform_level=1)])
+def test_dot_over_every_set_of_tile_types(kw):
+    """Sets of types that are a list of the handle's, others, and empty ones (a
+    uniform tree has no GHOST tiles)."""
+    o = po.Oracle(**kw)
+    lev, crd, typ, nbr = o.topology()
+    P = ca.Problem(ca.Tree(o.params.h0, lev, crd, typ, o.celltypes()))
+    rng = np.random.default_rng(2)
+    for ch in (po.CH_P, po.CH_Z):
+        v = rng.standard_normal((P.n, 512)).astype(np.float32)
+        o.set(ch, v)
+        P.set(ch, v)
+    for types in range(1, 8):
+        assert P.dot(ca.CH_P, ca.CH_Z, types) == o.dot(po.CH_P, po.CH_Z, types), types
