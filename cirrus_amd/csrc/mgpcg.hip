@@ -88,6 +88,7 @@ struct cg_problem {
   DList leaf, gather, applyl, ghosts, all;
   std::vector<DList> act, lvl;   // per level, all problems (operator API)
   std::vector<DList> actg, lvlg; // per level, tiles the V-cycle smooths with grid-wide launches
+  std::vector<DList> gatherl;    // per level, LEAF tiles with GHOST children
   std::vector<CoarsePlan> plans; // LDS-resident coarse levels, one per problem with C >= 0
   // schedule (no effect on results): XCD-aware tile order, LDS-resident coarse
   // levels given up to grid-wide launches, tiles per wavefront of the colour sweeps
@@ -472,6 +473,9 @@ void plan_schedule(cg_problem& P, std::vector<int32_t>& ids) {
   for (int i = 0; i < n; i++)
     if (ty[i] == LEAF && !(lev[i] >= 1 && grid_level(i))) P.rz_in_vcycle = false;
   add_list(&P.gather, every, [&](int i) { return ty[i] == LEAF && tr_has_gchild(P.tiles[i]); });
+  P.gatherl.assign(L + 1, DList());
+  for (int l = 0; l <= L; l++)
+    add_list(&P.gatherl[l], bucket[l], [&](int i) { return ty[i] == LEAF && tr_has_gchild(P.tiles[i]); });
   add_list(&P.applyl, every, [&](int i) { return ty[i] == LEAF || ty[i] == GHOST; });
   add_list(&P.ghosts, every, [&](int i) { return ty[i] == GHOST; });
   add_list(&P.all, every, [&](int) { return true; });
@@ -1061,13 +1065,11 @@ void enqueue_amg_vcycle(cg_problem& P, const VParams& v) {
   };
   const int L = P.max_level;
   for (int l = L; l >= 1; l--) {
-    const DList& a = P.actg[l];
     const DList& al = P.lvlg[l];
     if (!al.n) continue;
     for (int it = 0; it < v.nu; it++) { gs(l, 0); gs(l, 1); }
-    k_amg_residual<<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, X, RHS, TMP, A, c);
-    if (a.n) k_amg_restrict<<<grid_for(a.n, fl), 64, 0, P.stream>>>(P.L(a), a.n, fl, TMP, RHS, A, v.ooa, c);
-    const DList& below = P.lvl[l - 1];  // LDS-resident ones too: their LEAF tiles may have ghost children
+    k_amg_residual<<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, X, RHS, TMP, v.ooa, A, c);
+    const DList& below = P.gatherl[l - 1];  // LDS-resident ones too
     if (below.n) k_amg_leaf_rhs<<<grid_for(below.n, fl), 64, 0, P.stream>>>(P.L(below), below.n, fl, TMP, F, RHS, c);
   }
   if (!P.plans.empty())
@@ -1080,7 +1082,7 @@ void enqueue_amg_vcycle(cg_problem& P, const VParams& v) {
     if (al.n) k_amg_prolong<<<grid_for(al.n, fl), 64, 0, P.stream>>>(P.L(al), al.n, fl, X, A, v.pcoef, c);
     for (int it = 0; it < v.nu; it++) { gs(l, 1); gs(l, 0); }
   }
-  k_to_split<<<unsigned(P.leaf.n), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, X, c.z);
+  k_amg_finish<<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, X, c.z, c);
 }
 
 // Handles whose every problem is LDS-resident, all its LEAF tiles on one level,
@@ -1135,7 +1137,7 @@ void enqueue_cg_iteration(cg_problem& P, const VParams& vp, int pure_neumann) {
   const bool rz_fused = !v.amg && v.smoother == CG_SMOOTH_RBGS && v.nu > 0 && P.rz_in_vcycle;
   if (v.amg) enqueue_amg_vcycle(P, v);
   else enqueue_vcycle<V>(P, v.smoother == CG_SMOOTH_RBGS ? pool_zb<V>(P) : Z, Z, nullptr, v, rz_fused ? F_DOT_RZ : 0);
-  if (!rz_fused) k_cg_dot_rz<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
+  if (!rz_fused && !v.amg) k_cg_dot_rz<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
   launch_finalize(P.stream, int(np), P.max_leaf, c, FIN_RZ, fl, rb, rc);
   k_cg_update_p<V><<<grid_for(P.leaf.n, fl), 64, 0, P.stream>>>(P.L(P.leaf), P.leaf.n, fl, c);
   k_apply<true><<<grid_for(P.applyl.n, fl), 64, 0, P.stream>>>(P.L(P.applyl), P.applyl.n, fl, c.p, c.ap, -1, 0, 1, c);
