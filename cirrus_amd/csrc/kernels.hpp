@@ -387,9 +387,37 @@ enum : int {
   F_INERT = 128,     // a CG iteration's launch: tiles the solve's init found inert are skipped
 };
 
-__device__ __forceinline__ bool prob_done(const Ctx& c, const TileRec& T, int flags) {
-  return (flags & F_CHECK_DONE) && c.ps[T.prob].done;
+// A problem's done flag, loaded with the tile's data (without F_CHECK_DONE the face
+// masks stand in as a readable address) and tested once that is here: tested by a
+// load of its own it cost every kernel of the iteration another memory round trip
+// (adaptive 256^3 problem: the operator 6.73 -> 6.42 us, the residual update 5.19 ->
+// 4.77, restriction from 3,232 tiles 4.40 -> 4.20; large pools within 1 %).
+__device__ __forceinline__ uint32_t done_load(const Ctx& c, const TileRec& T, int flags) {
+  return *((flags & F_CHECK_DONE) ? reinterpret_cast<const uint32_t*>(&c.ps[T.prob].done)
+                                  : reinterpret_cast<const uint32_t*>(c.fmask));
 }
+__device__ __forceinline__ bool done_test(uint32_t word, int flags) {
+  __asm__("" : "+v"(word));
+  return (flags & F_CHECK_DONE) && word;
+}
+// A problem's state as one load of the wavefront (word `lane` of it), its fields
+// taken from the lanes once they are needed: the load goes out with the partials'.
+__device__ __forceinline__ uint32_t state_word(const ProbState* ps) {
+  constexpr int kWords = int(sizeof(ProbState) / 4);
+  static_assert(kWords <= 64, "one word a lane");
+  return reinterpret_cast<const uint32_t*>(ps)[min(lane_id(), kWords - 1)];
+}
+__device__ __forceinline__ ProbState state_of(uint32_t word) {
+  union {
+    uint32_t w[sizeof(ProbState) / 4];
+    ProbState s;
+  } u;
+  __asm__("" : "+v"(word));
+#pragma unroll
+  for (int i = 0; i < int(sizeof(ProbState) / 4); i++) u.w[i] = uint32_t(__builtin_amdgcn_readlane(int(word), i));
+  return u.s;
+}
+
 
 __device__ __forceinline__ void unpack8(float4 a, float4 b, float v[8]) {
   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
@@ -515,6 +543,10 @@ __device__ __forceinline__ void hold(float4&) {}
 __device__ __forceinline__ void hold(float&) {}
 // the same for an FP32 value whose later select must not pull its wait forward
 __device__ __forceinline__ void hold_f(float& v) { __asm__("" : "+v"(v)); }
+__device__ __forceinline__ void hold8(float v[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; k++) hold_f(v[k]);
+}
 __device__ __forceinline__ void hold(uint2& q) { __asm__("" : "+v"(q.x), "+v"(q.y)); }
 __device__ __forceinline__ void hold(uint32_t& v) { __asm__("" : "+v"(v)); }
 
@@ -1213,8 +1245,9 @@ __device__ __forceinline__ void tile_jacobi(const Ctx& c, const TileRec& T, int 
                                             V* Y, const V* F, float omega, int flags, TileLDS& L) {
   Stencil S;
   float b[8];
+  const uint32_t dn = done_load(c, T, flags);
   stage_with_rhs(c, T, X, XG, F, flags, false, L, S, b);
-  if (prob_done(c, T, flags)) return;
+  if (done_test(dn, flags)) return;
   wave_sync();
   float ax[8], dg[8], out[8];
   if (S.open) {  // as gs_quad's open tiles: no masks, quotients as products with 1/D
@@ -1280,8 +1313,9 @@ __device__ __forceinline__ void tile_restrict(const Ctx& c, const TileRec& T, in
   Stencil S;
   const int lane = lane_id();
   float b[8];
+  const uint32_t dn = done_load(c, T, flags);
   stage_with_rhs<V>(c, T, X, X, F, flags, (flags & F_VCYCLE) && tr_type(T) == T_GHOST, L, S, b);
-  if (prob_done(c, T, flags)) return;
+  if (done_test(dn, flags)) return;
   wave_sync();
   float ax[8], dg[8];
   apply_pencil<true, false>(L, S, ax, dg);
@@ -1305,6 +1339,7 @@ __device__ __forceinline__ void tile_prolong(const Ctx& c, const TileRec& T, int
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t base = size_t(T.self) * 512 + lane * 8;
   const int oct = tr_octant(T), ox = oct & 1, oy = (oct >> 1) & 1, oz = (oct >> 2) & 1;
+  const uint32_t dn = done_load(c, T, flags);
   const float4 pv = load_quad_split(XC + size_t(T.parent) * 512, (ox * 4 + (i >> 1)) * 8 + (oy * 4 + (j >> 1)), oz * 4);
   const float cz[4] = {pv.x, pv.y, pv.z, pv.w};
   const uint64_t ct = load_ct8(c.ctype + base);
@@ -1312,7 +1347,8 @@ __device__ __forceinline__ void tile_prolong(const Ctx& c, const TileRec& T, int
   float fx[8];
   if (ghost || (flags & F_ZERO_X)) { for (int k = 0; k < 8; k++) fx[k] = 0.f; }
   else load8_split(XF + size_t(T.self) * 512, lane, fx);
-  if (prob_done(c, T, flags)) return;
+  hold8(fx);
+  if (done_test(dn, flags)) return;
   float out[8];
   if (ghost) {
     for (int k = 0; k < 8; k++) out[k] = (ct_at(ct, k) & C_INT) ? cz[k >> 1] : 0.f;
@@ -2282,9 +2318,12 @@ __global__ __launch_bounds__(64) void k_cg_dot_rz(const TileRec* __restrict__ li
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float rv[8], zv[8];
+  const uint32_t dn = done_load(c, T, flags);
   load8(c.r + base, rv);
   load8_split(vc_z<V>(c) + size_t(T.self) * 512, lane, zv);
-  if (prob_done(c, T, flags)) return;
+  hold8(rv);  // or the loads would move behind the test
+  hold8(zv);
+  if (done_test(dn, flags)) return;
   double a = 0.0;
   for (int k = 0; k < 8; k++) a += double(rv[k]) * double(zv[k]);
   a = wave_sum(a);
@@ -2304,12 +2343,13 @@ __global__ __launch_bounds__(64) void k_cg_update_p(const TileRec* __restrict__ 
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float pv[8], zv[8], xv[8];
+  const uint32_t word = state_word(c.ps + T.prob);
   load8(c.p + base, pv);
   load8_split(vc_z<V>(c) + size_t(T.self) * 512, lane, zv);
   load8(c.x + base, xv);
   const uint64_t ct = tile_ct8(T, c.ctype + base);
-  if (prob_done(c, T, flags)) return;
-  const ProbState& ps = c.ps[T.prob];
+  const ProbState ps = state_of(word);
+  if ((flags & F_CHECK_DONE) && ps.done) return;
   const float beta = float(ps.beta);
   const float alpha = float(ps.alpha);
   const bool upd_x = ps.iter > 0;  // an earlier iteration left its x update pending
@@ -2347,13 +2387,14 @@ __global__ __launch_bounds__(64) void k_apply(const TileRec* __restrict__ list, 
   } else {
     view_coeffs(T, sl, bcv);
   }
+  const uint32_t dn = done_load(c, T, flags);
   if (PG) {
     StagePG r = stage_issue_pg(c, T, X);
     stage_commit_pg(r, T, bcv, L, S);
   } else {
     stage_tile<false>(c, T, X, X, false, false, bcv, L, S);
   }
-  if (prob_done(c, T, flags)) return;
+  if (done_test(dn, flags)) return;
   wave_sync();
   float ax[8], dg[8];
   if (diag) apply_pencil<false, true>(L, S, dg, ax);
@@ -2382,6 +2423,7 @@ __global__ __launch_bounds__(64) void k_ghost_gather(const TileRec* __restrict__
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float av[8], pv[8];
+  const uint32_t dn = done_load(c, T, flags);
   load8(c.ap + base, av);
   load8(c.p + base, pv);
   float4 e[2];
@@ -2390,7 +2432,7 @@ __global__ __launch_bounds__(64) void k_ghost_gather(const TileRec* __restrict__
     gs[h] = c.kids[T.gslot].slot[(i >> 2) | ((j >> 2) << 1) | (h << 2)];
     if (gs[h] >= 0) e[h] = *reinterpret_cast<const float4*>(c.gsum + size_t(gs[h]) * 64 + (i & 3) * 16 + (j & 3) * 4);
   }
-  if (prob_done(c, T, flags)) return;
+  if (done_test(dn, flags)) return;
   for (int h = 0; h < 2; h++) {
     if (gs[h] < 0) continue;
     av[4 * h + 0] = av[4 * h + 0] + e[h].x;
@@ -2415,11 +2457,13 @@ __global__ __launch_bounds__(64) void k_cg_update_xr(const TileRec* __restrict__
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
   float rv[8], av[8];
+  const uint32_t word = state_word(c.ps + T.prob);
   load8(c.r + base, rv);
   load8(c.ap + base, av);
   const uint64_t ct = tile_ct8(T, c.ctype + base);
-  if (prob_done(c, T, flags)) return;
-  const float alpha = float(c.ps[T.prob].alpha);
+  const ProbState ps = state_of(word);
+  if ((flags & F_CHECK_DONE) && ps.done) return;
+  const float alpha = float(ps.alpha);
   for (int k = 0; k < 8; k++)
     if (ct_at(ct, k) & C_INT) rv[k] = __builtin_fmaf(-alpha, av[k], rv[k]);
   store8(c.r + base, rv);
@@ -2522,24 +2566,6 @@ __device__ __forceinline__ double block_sum_partials(const double* __restrict__ 
     return a;
   }
 }
-// A problem's state as one load of the wavefront (word `lane` of it), its fields
-// taken from the lanes once they are needed: the load goes out with the partials'.
-__device__ __forceinline__ uint32_t state_word(const ProbState* ps) {
-  constexpr int kWords = int(sizeof(ProbState) / 4);
-  static_assert(kWords <= 64, "one word a lane");
-  return reinterpret_cast<const uint32_t*>(ps)[min(lane_id(), kWords - 1)];
-}
-__device__ __forceinline__ ProbState state_of(uint32_t word) {
-  union {
-    uint32_t w[sizeof(ProbState) / 4];
-    ProbState s;
-  } u;
-  hold(word);
-#pragma unroll
-  for (int i = 0; i < int(sizeof(ProbState) / 4); i++) u.w[i] = uint32_t(__builtin_amdgcn_readlane(int(word), i));
-  return u.s;
-}
-
 // Per-problem finalisation of a reduction over the LEAF-tile partials.
 enum : int { FIN_BB = 0, FIN_RZ = 1, FIN_PAP = 2, FIN_RR = 3, FIN_MEAN = 4, FIN_IRBB = 5, FIN_SCALE = 6 };
 // range_count >= 0: the launch's one problem has its partials at range_begin ..
@@ -2852,14 +2878,15 @@ __global__ __launch_bounds__(CL_THREADS) void k_cg_small(const CoarsePlan* __res
 __global__ __launch_bounds__(64) void k_mean(const TileRec* __restrict__ list, int n, int flags,
                                              const float* __restrict__ X, Ctx c) {
   TILE_KERNEL_PROLOGUE_C
-  if (prob_done(c, T, flags)) return;
-  ProbState* ps = c.ps + T.prob;
-  if (!ps->pure_neumann) return;
   const int lane = lane_id();
   const size_t base = size_t(T.self) * 512 + lane * 8;
+  const uint32_t word = state_word(c.ps + T.prob);
   float v[8];
   load8(X + base, v);
   const uint64_t ct = load_ct8(c.ctype + base);
+  hold8(v);
+  const ProbState ps = state_of(word);
+  if (((flags & F_CHECK_DONE) && ps.done) || !ps.pure_neumann) return;
   double a = 0.0, q = 0.0;
   for (int k = 0; k < 8; k++) { a += double(v[k]); q += (ct_at(ct, k) & C_INT) ? 1.0 : 0.0; }
   a = wave_sum(a);
@@ -2870,14 +2897,15 @@ template <class V>
 __global__ __launch_bounds__(64) void k_subtract_mean(const TileRec* __restrict__ list, int n, int flags,
                                                       float* __restrict__ X, int write_rhsv, Ctx c) {
   TILE_KERNEL_PROLOGUE_C
-  if (prob_done(c, T, flags)) return;
-  ProbState* ps = c.ps + T.prob;
-  if (!ps->pure_neumann) return;
-  const double mean = ps->mean;
   const size_t base = size_t(T.self) * 512 + lane_id() * 8;
+  const uint32_t word = state_word(c.ps + T.prob);
   float v[8];
   load8(X + base, v);
   const uint64_t ct = load_ct8(c.ctype + base);
+  hold8(v);
+  const ProbState ps = state_of(word);
+  if (((flags & F_CHECK_DONE) && ps.done) || !ps.pure_neumann) return;
+  const double mean = ps.mean;
   for (int k = 0; k < 8; k++) if (ct_at(ct, k) & C_INT) v[k] = float(double(v[k]) - mean);
   store8(X + base, v);
   if (write_rhsv) store8_split(vc_rhs<V>(c) + size_t(T.self) * 512, lane_id(), v);
@@ -3156,10 +3184,6 @@ __global__ __launch_bounds__(64) void k_amg_init(const TileRec* __restrict__ lis
   store8(X + b, z);
 }
 
-__device__ __forceinline__ void hold8(float v[8]) {
-#pragma unroll
-  for (int k = 0; k < 8; k++) hold_f(v[k]);
-}
 // A x with the stored coefficients for the lane's 8 cells (negativeLapSameLevel,
 // AMGSolver.cu:232-250): x0 d + sum over x-, x+, y-, y+, z-, z+ of the face's
 // entry times the neighbour's x, the plus faces' entries read from the plus
@@ -3232,10 +3256,9 @@ __global__ __launch_bounds__(64) void k_amg_gs(const TileRec* __restrict__ list,
   float rhs[8], x0[8], ax[8], dg[8];
   load8(RHS + b, rhs);
   const uint64_t ct = load_ct8(A.ct + b);
-  const int32_t* dp = (flags & F_CHECK_DONE) ? &c.ps[T.prob].done : reinterpret_cast<const int32_t*>(c.fmask);
-  const int32_t done = *dp;
+  const uint32_t dn = done_load(c, T, flags);
   amg_rows(T, X, A, x0, ax, dg);
-  if ((flags & F_CHECK_DONE) && done) return;
+  if (done_test(dn, flags)) return;
   wave_sync();  // every lane has read its neighbours before any lane writes
   const bool odd = even_colour(lane) != color;  // of the pencil's cells the even or the odd ones
 #pragma unroll
@@ -3265,10 +3288,9 @@ __global__ __launch_bounds__(64) void k_amg_residual(const TileRec* __restrict__
   float x0[8], ax[8], dg[8], rhs[8];
   load8(RHS + b, rhs);
   const uint64_t ct = load_ct8(A.ct + b);
-  const int32_t* dp = (flags & F_CHECK_DONE) ? &c.ps[T.prob].done : reinterpret_cast<const int32_t*>(c.fmask);
-  const int32_t done = *dp;
+  const uint32_t dn = done_load(c, T, flags);
   amg_rows(T, X, A, x0, ax, dg);
-  if ((flags & F_CHECK_DONE) && done) return;
+  if (done_test(dn, flags)) return;
   float out[8];
 #pragma unroll
   for (int k = 0; k < 8; k++) out[k] = (ct_at(ct, k) == C_INT) ? rhs[k] - ax[k] : 0.f;
@@ -3295,7 +3317,7 @@ __global__ __launch_bounds__(64) void k_amg_leaf_rhs(const TileRec* __restrict__
                                                      const float* __restrict__ TMP, const float* __restrict__ F,
                                                      float* __restrict__ RHS, Ctx c) {
   TILE_KERNEL_PROLOGUE_C
-  if (prob_done(c, T, flags)) return;
+  const uint32_t dn = done_load(c, T, flags);
   const GhostKids& kids = c.kids[T.gslot];
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t b = size_t(T.self) * 512 + lane * 8;
@@ -3318,6 +3340,7 @@ __global__ __launch_bounds__(64) void k_amg_leaf_rhs(const TileRec* __restrict__
       out[4 * h + k] = __builtin_fmaf(sum, 1.f, out[4 * h + k]);
     }
   }
+  if (done_test(dn, flags)) return;
   store8(RHS + b, out);
 }
 
@@ -3329,9 +3352,12 @@ __global__ __launch_bounds__(64) void k_amg_finish(const TileRec* __restrict__ l
   const int lane = lane_id();
   const size_t b = size_t(T.self) * 512 + lane * 8;
   float z[8], r[8];
+  const uint32_t dn = done_load(c, T, flags);
   load8(X + b, z);
   load8(c.r + b, r);
-  if (prob_done(c, T, flags)) return;
+  hold8(z);
+  hold8(r);
+  if (done_test(dn, flags)) return;
   store8_split(Z + size_t(T.self) * 512, lane, z);
   double a = 0.0;
   for (int k = 0; k < 8; k++) a += double(r[k]) * double(z[k]);
@@ -3348,6 +3374,7 @@ __global__ __launch_bounds__(64) void k_amg_prolong(const TileRec* __restrict__ 
   const int lane = lane_id(), i = lane >> 3, j = lane & 7;
   const size_t b = size_t(T.self) * 512 + lane * 8;
   float x[8];
+  const uint32_t dn = done_load(c, T, flags);
   load8(X + b, x);
   const uint64_t ct = load_ct8(A.ct + b);
   const int o = tr_octant(T);
@@ -3355,7 +3382,9 @@ __global__ __launch_bounds__(64) void k_amg_prolong(const TileRec* __restrict__ 
                     ((o >> 2) & 1) * 4;
   float px[4];
   for (int q = 0; q < 4; q++) px[q] = X[pb + q];
-  if (prob_done(c, T, flags)) return;
+  for (int q = 0; q < 4; q++) hold_f(px[q]);
+  hold8(x);
+  if (done_test(dn, flags)) return;
   const bool ghost = tr_type(T) == T_GHOST;
   for (int k = 0; k < 8; k++) {
     const bool in = ct_at(ct, k) & C_INT;
