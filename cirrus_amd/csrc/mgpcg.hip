@@ -1485,7 +1485,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   // one, 4.0 ms by replay; 14,345 tiles (5.3 us a launch): 3.47 ms and 3.53.
   constexpr int kStreamMinTiles = 8192;
   const bool small = !amg && runs_small(P);
-  const int chunk = small ? std::max(stride, kSmallIters) : stride;
+  const int chunk = small ? kSmallIters : stride;  // (the kernel itself keeps to the stride of the checks)
   const bool use_graph = prm.use_graph > 0 || (prm.use_graph < 0 && (amg || P.n < kStreamMinTiles));
   if (use_graph && !small && P.graph_key != keybuf) {
     if (P.graph) HIPC(hipGraphExecDestroy(P.graph));
