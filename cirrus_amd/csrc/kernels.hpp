@@ -2687,11 +2687,17 @@ __global__ __launch_bounds__(NT) void k_finalize(int mode, int flags, int range_
 // sweeps a level), 19 iterations: 790 -> 360 us a solve, 10 us of it an iteration,
 // bound by the V-cycle's chain of some forty passes with a barrier each.
 // ---------------------------------------------------------------------------
+// Tile partials: a row for each of the iteration's sums.  Every wavefront reads a row
+// behind the barrier that follows its writing, and it is written again an iteration
+// later, with the barriers of the other sums between.  (A row for two sums would need
+// a barrier of its own: |r|^2 is the last sum that an iteration reads and the mean's
+// two are the first that the next one writes, with none between.)
+enum : int { SM_MEAN = 0, SM_COUNT, SM_RZ, SM_PAP, SM_RR, SM_SUMS };
 struct SmallLDS {
   float p[CL_ZERO + 4];        // in v.z's layout, so that a cell's neighbour addresses serve both
   CoarseLDS v;                 // v.t: A p outside the V-cycle
   float r[CL_CHILDREN * 512];  // from the finest level's first slot
-  double part[3][CL_CHILDREN];
+  double part[SM_SUMS][CL_CHILDREN];
   ProbState out;               // the state to leave (thread 0's)
 };
 // A tile's sum over the 64 pencils (lanes) of f(cell values of the pencil in order).
@@ -2769,10 +2775,10 @@ __device__ __forceinline__ void sm_solve(SmallLDS& S, const CoarsePlan& cp, int 
         for (int e = 0; e < 8; e++) { a += double(w[e]); q += (ct_at(ct, e) & C_INT) ? 1.0 : 0.0; }
         a = wave_sum(a);
         q = wave_sum(q);
-        if (lane_id() == 0) { S.part[0][wave] = a; S.part[1][wave] = q; }
+        if (lane_id() == 0) { S.part[SM_MEAN][wave] = a; S.part[SM_COUNT][wave] = q; }
       }
       __syncthreads();
-      const double mean = sm_total(S.part[0], n) / sm_total(S.part[1], n);
+      const double mean = sm_total(S.part[SM_MEAN], n) / sm_total(S.part[SM_COUNT], n);
       if (tid == 0) S.out.mean = mean;
 #pragma unroll
       for (int col = 0; col < 2; col++)
@@ -2792,11 +2798,11 @@ __device__ __forceinline__ void sm_solve(SmallLDS& S, const CoarsePlan& cp, int 
     // gamma = r.z, beta
     if (wave < n) {
       const double a = sm_dot(S.r + wave * 512, M.z + (first + wave) * 512);
-      if (lane_id() == 0) S.part[2][wave] = a;
+      if (lane_id() == 0) S.part[SM_RZ][wave] = a;
     }
     __syncthreads();
     const double gamma_old = gamma;
-    gamma = sm_total(S.part[2], n);
+    gamma = sm_total(S.part[SM_RZ], n);
     const double beta = it == 0 ? 0.0 : gamma / gamma_old;
     if (tid == 0) {
       S.out.gamma_old = gamma_old;
@@ -2830,10 +2836,10 @@ __device__ __forceinline__ void sm_solve(SmallLDS& S, const CoarsePlan& cp, int 
     __syncthreads();
     if (wave < n) {
       const double a = sm_dot(S.p + (first + wave) * 512, M.t + wave * 512);
-      if (lane_id() == 0) S.part[0][wave] = a;
+      if (lane_id() == 0) S.part[SM_PAP][wave] = a;
     }
     __syncthreads();
-    const double pap = sm_total(S.part[0], n);
+    const double pap = sm_total(S.part[SM_PAP], n);
     if (tid == 0) S.out.pAp = pap;
     alpha = gamma / pap;
     const float na = -float(alpha);
@@ -2845,10 +2851,10 @@ __device__ __forceinline__ void sm_solve(SmallLDS& S, const CoarsePlan& cp, int 
     __syncthreads();
     if (wave < n) {
       const double a = sm_dot(S.r + wave * 512, S.r + wave * 512);
-      if (lane_id() == 0) S.part[1][wave] = a;
+      if (lane_id() == 0) S.part[SM_RR][wave] = a;
     }
     __syncthreads();
-    const double rr = sm_total(S.part[1], n);
+    const double rr = sm_total(S.part[SM_RR], n);
     it++;
     const int cs = st.check_stride;
     const bool converged = cs > 0 && it % cs == 0 && rr < st.thr;
