@@ -71,7 +71,8 @@ __host__ __device__ __forceinline__ bool tr_all_int(const TileRec& T) { return (
 // leaves each of its values as it found them (see k_cg_init)
 __host__ __device__ __forceinline__ bool tr_inert_cand(const TileRec& T) { return ((T.meta >> 26) & 1) != 0; }
 // every cell INTERIOR and no face cut by a NEUMANN cell: each face mask byte is
-// M_OPEN_INT (the masks need not be read)
+// M_OPEN_INT (the masks need not be read); of a LEAF or NONLEAF tile also: every
+// cell's diagonal is finite and not 0
 __host__ __device__ __forceinline__ bool tr_all_open(const TileRec& T) { return ((T.meta >> 27) & 1) != 0; }
 // every face of the tile has the inside coefficient: with all_open every cell's
 // diagonal is D (rdiag)
@@ -337,11 +338,13 @@ __device__ __forceinline__ float div_by_checked(float a, double rd) {
   return q;
 }
 // The same without a test, where a branch is on the critical path: the product
-// rounded to 50 bits (9 v - (9 v - v)) is still on its side of every boundary that
-// it is not on, and is the quotient where that has 25 bits (rd within 2^-52 of 1/d).
+// rounded to 50 bits is still on its side of every boundary that it is not on, and
+// is the quotient where that has 25 bits (rd within 2^-52 of 1/d: the product is at
+// most 3 units of its last place off, and 4 go to the next multiple of 8).  Rounded
+// as an integer, which leaves an infinite product infinite and NaN NaN.
 __device__ __forceinline__ float div_by_rounded(float a, double rd) {
-  const double v = double(a) * rd, c = 9.0 * v;
-  return float(c - (c - v));
+  const uint64_t v = __builtin_bit_cast(uint64_t, double(a) * rd);
+  return float(__builtin_bit_cast(double, (v + 4) & ~uint64_t(7)));
 }
 // Four quotients with one test for all.
 __device__ __forceinline__ void div4_by(const float a[4], double r0, double r1, double r2, double r3, float q[4]) {
@@ -356,12 +359,14 @@ __device__ __forceinline__ void div4_by(const float a[4], double r0, double r1, 
     q[3] = div_again(q[3], a[3], r3);
   }
 }
-// 1/d in FP64 for finite d != 0: the FP32 reciprocal and two Newton steps (a
-// divisor beyond the range where that reciprocal is a normal number: the division).
+// 1/d in FP64 for d != 0: the FP32 reciprocal and two Newton steps (a divisor
+// beyond the range where that reciprocal is a normal number: the division).  NaN for
+// an infinite d: it comes of infinite coefficients, whose row is infinite or NaN, and
+// so is the quotient NaN, not 0.
 __device__ __forceinline__ double recip64(float d) {
   const double dd = double(d);
   const float a = __builtin_fabsf(d);
-  if (!(a >= 0x1p-100f && a <= 0x1p100f)) return 1.0 / dd;
+  if (!(a >= 0x1p-100f && a <= 0x1p100f)) return a == __builtin_inff() ? __builtin_nan("") : 1.0 / dd;
   double y = double(__builtin_amdgcn_rcpf(d));
   y = __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
   return __builtin_fma(__builtin_fma(-dd, y, 1.0), y, y);
@@ -1003,17 +1008,15 @@ __device__ __forceinline__ float open_residual(const GsCoef& G, float s, float b
   return b - (G.p2 ? s * G.h3 : ((s * G.h) * G.h) * G.h);
 }
 // 1/D of a lane's open cells: those inside the pencil (mid) and at its ends
-// k = 0 (lo) and k = 7 (hi), the sums formed as cell_row_m forms them (0: D is 0).
+// k = 0 (lo) and k = 7 (hi), the sums formed as cell_row_m forms them (an open
+// tile's are finite and not 0).
 struct OpenDiag {
   double mid, lo, hi;
 };
 __device__ __forceinline__ OpenDiag open_diag(const GsCoef& G, float bim, float bip, float bjm, float bjp) {
   if (G.uniform) return OpenDiag{G.rd, G.rd, G.rd};
   const float bi = G.bc[6], d4 = (((0.f + bim) + bip) + bjm) + bjp;
-  auto inv = [&](float d) {
-    const float g = ((d * G.h) * G.h) * G.h;
-    return g != 0.f ? recip64(g) : 0.0;
-  };
+  auto inv = [&](float d) { return recip64(((d * G.h) * G.h) * G.h); };
   return OpenDiag{inv((d4 + bi) + bi), inv((d4 + G.bc[2]) + bi), inv((d4 + bi) + G.bc[5])};
 }
 
@@ -1281,10 +1284,7 @@ __device__ __forceinline__ void tile_jacobi(const Ctx& c, const TileRec& T, int 
     div4_by(res, D.lo, D.mid, D.mid, D.mid, q);
     div4_by(res + 4, D.mid, D.mid, D.mid, D.hi, q + 4);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const double rd = k == 0 ? D.lo : (k == 7 ? D.hi : D.mid);
-      out[k] = rd != 0.0 ? S.own[k] + q[k] : 0.f;
-    }
+    for (int k = 0; k < 8; k++) out[k] = S.own[k] + q[k];
     store8_split(Y + size_t(T.self) * 512, lane_id(), out);
     return;
   }

@@ -337,16 +337,20 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
     // smoothing-view coefficients (subtree at the tile's own level)
     view_coeffs(T, l, T.bc);
     // the sweep's diagonal of a cell with six inside coefficients, summed as the
-    // kernels sum it, and its reciprocal
+    // kernels sum it, and its reciprocal.  A cell of an open tile has at least three
+    // inside coefficients and none larger, so where this diagonal is finite and not 0
+    // every cell's is.
     T.h3 = (T.h * T.h) * T.h;
+    bool regular = true;
     if (my != GHOST) {
       const float ci = T.bc[6];
       float d = 0.f;
       for (int e = 0; e < 6; e++) d = d + ci;
       d = ((d * T.h) * T.h) * T.h;
-      bool uniform = d != 0.f;
+      regular = d != 0.f && std::isfinite(d);
+      bool uniform = regular;
       for (int f = 0; f < 6; f++) uniform = uniform && T.bc[f] == ci;
-      T.rdiag = d != 0.f ? 1.0 / double(d) : 0.0;
+      T.rdiag = regular ? 1.0 / double(d) : 0.0;
       if (uniform) T.meta |= 1u << 28;
     }
     // a power of two whose third power is a normal number
@@ -369,11 +373,12 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
     if (all_int) T.meta |= 1u << 25;
     if (no_int && my == LEAF && !tr_has_gchild(T)) T.meta |= 1u << 26;
     // every face mask M_OPEN_INT (as k_face_mask forms them): all cells
-    // INTERIOR and no NEUMANN cell across a tile face (no neighbour: open).
+    // INTERIOR and no NEUMANN cell across a tile face (no neighbour: open); and
+    // regular, as the short rows divide without a test.
     // The neighbour's face layer: x faces i = 7 / 0 (words 56..63 / 0..7),
     // y faces j = 7 / 0 (word i*8 + 7 / i*8), z faces k = 7 / 0 (byte 7 / 0 of
     // every word).
-    bool open = all_int;
+    bool open = all_int && regular;
     for (int f = 0; f < 6 && open; f++) {
       if (nbl[f] < 0) continue;
       const auto nw = words(nbl[f]);
