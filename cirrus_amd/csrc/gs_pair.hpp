@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64) void k_gs_pair(const TileRec* __restrict__ list
       else if (g == 1) { XIM = ownq; XIP = rdeep; XJM = along_m; XJP = along_p; }
       else if (g == 2) { XIM = along_m; XIP = along_p; XJM = rdeep; XJP = ownq; }
       else { XIM = along_m; XIP = along_p; XJM = ownq; XJP = rdeep; }
-      const GsCoef nc{rnb.bc, h, 0.f, 0.0, false, false, false};  // the general rows: lanes differ in their neighbour
+      const GsCoef nc{rnb.bc, h, 0.0, false, false};  // the general rows: lanes differ in their neighbour
       const float4 nr = gs_quad(rc1, rc2, XIM, XIP, XJM, XJP, kv, rb, quad_mask(rm, rp), nc, ri, rj, rp);
       r1 = make_float4(vround<V>(nr.x), vround<V>(nr.y), vround<V>(nr.z), vround<V>(nr.w));
     }

@@ -44,14 +44,14 @@ struct alignas(16) TileRec {
   int32_t self;       // the tile's index
   float h;            // cell size of the tile's level
   uint32_t meta;      // level | type << 8 | octant << 16 | has_gchild << 24 | all_interior << 25 |
-                      // inert_candidate << 26 | all_open << 27 | uniform << 28 | h_pow2 << 29
+                      // inert_candidate << 26 | all_open << 27 | uniform << 28
   uint32_t ntypes;    // type of face neighbour f in bits 4f..4f+3 (0: none), std_face f in bit 24 + f
   float bc[7];        // face coefficients of the smoothing view (subtree at the
                       // tile's own level): faces x-,y-,z-,x+,y+,z+, then inside
   int32_t nbr_parent[6];  // parent tile of face neighbour f (-1: no neighbour or level 0)
-  float h3;           // (h * h) * h
+  int32_t pad0;
   double rdiag;       // 1 / D, D = the sweep's diagonal of a cell whose six faces have the inside coefficient
-  int32_t pad[2];
+  int32_t pad1[2];
 };
 static_assert(sizeof(TileRec) == 128, "TileRec is 128 bytes");
 // The ghost children of a LEAF tile by octant (-1: none): tile and ghost slot.
@@ -77,9 +77,6 @@ __host__ __device__ __forceinline__ bool tr_all_open(const TileRec& T) { return 
 // every face of the tile has the inside coefficient: with all_open every cell's
 // diagonal is D (rdiag)
 __host__ __device__ __forceinline__ bool tr_uniform(const TileRec& T) { return ((T.meta >> 28) & 1) != 0; }
-// h is a power of two (and h3 its exact cube), so that a product with h3 rounds
-// as three products with h do
-__host__ __device__ __forceinline__ bool tr_h_pow2(const TileRec& T) { return ((T.meta >> 29) & 1) != 0; }
 // every face neighbour is missing, a GHOST tile, or all_open and uniform (so the
 // diagonal of its cells is D)
 __host__ __device__ __forceinline__ bool tr_std_faces(const TileRec& T) { return ((T.ntypes >> 24) & 0x3f) == 0x3f; }
@@ -639,17 +636,15 @@ struct Stencil {
   uint64_t m;          // own face masks, one byte per cell
   float xkm, xkp;      // k-halo values (z- neighbour cell (i,j,7), z+ neighbour cell (i,j,0))
   float b_int, b_f[6]; // base coefficients: inside the tile and across face f
-  float h, h3;
+  float h;
   double rd;           // the record's rdiag, and what it says of the tile
-  bool open, uniform, p2;
+  bool open, uniform;
 };
 __device__ __forceinline__ void stencil_coeffs(const TileRec& T, const float bcv[7], Stencil& S) {
   S.h = T.h;
-  S.h3 = T.h3;
   S.rd = T.rdiag;
   S.open = tr_all_open(T);
   S.uniform = tr_uniform(T);
-  S.p2 = tr_h_pow2(T);
   S.b_int = bcv[6];
   for (int f = 0; f < 6; f++) S.b_f[f] = bcv[f];
 }
@@ -995,17 +990,12 @@ __device__ __forceinline__ void apply_pencil(const TileLDS& L, const Stencil& S,
 // and sizes, and what the record says of the tile.
 struct GsCoef {
   const float* bc;  // faces x-..z+, inside
-  float h, h3;
+  float h;
   double rd;
-  bool open, uniform, p2;
+  bool open, uniform;
 };
 __device__ __forceinline__ GsCoef gs_coef(const TileRec& T) {
-  return GsCoef{T.bc, T.h, T.h3, T.rdiag, tr_all_open(T), tr_uniform(T), tr_h_pow2(T)};
-}
-// b - A x of an open cell from its row sum: ((s h) h) h, one product when h is a
-// power of two (all three are then exact but where the last leaves FP32's range).
-__device__ __forceinline__ float open_residual(const GsCoef& G, float s, float b) {
-  return b - (G.p2 ? s * G.h3 : ((s * G.h) * G.h) * G.h);
+  return GsCoef{T.bc, T.h, T.rdiag, tr_all_open(T), tr_uniform(T)};
 }
 // 1/D of a lane's open cells: those inside the pencil (mid) and at its ends
 // k = 0 (lo) and k = 7 (hi), the sums formed as cell_row_m forms them (an open
@@ -1062,7 +1052,7 @@ __device__ __forceinline__ float4 gs_quad(float4 X0, float4 XO, float4 XIM, floa
         s = __builtin_fmaf(m == 0 ? bkm : bi, x0 - comp4(XKM, m), s);
         s = __builtin_fmaf(m == 3 ? bkp : bi, x0 - comp4(XKP, m), s);
       }
-      res[m] = ZERO ? comp4(B, m) - 0.f : open_residual(G, s, comp4(B, m));
+      res[m] = comp4(B, m) - (ZERO ? 0.f : ((s * G.h) * G.h) * G.h);
     }
     div4_by(res, dlo, D.mid, D.mid, dhi, q);
     return make_float4(X0.x + q[0], X0.y + q[1], X0.z + q[2], X0.w + q[3]);
@@ -1406,7 +1396,6 @@ __device__ __forceinline__ TileRec unpack_rec(RecWords a, RecWords b) {
   T.bc[1] = __int_as_float(a[15]);
   for (int f = 2; f < 7; f++) T.bc[f] = __int_as_float(b[f - 2]);
   for (int f = 0; f < 6; f++) T.nbr_parent[f] = b[5 + f];
-  T.h3 = __int_as_float(b[11]);
   T.rdiag = __hiloint2double(b[13], b[12]);
   return T;
 }

@@ -340,7 +340,6 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
     // kernels sum it, and its reciprocal.  A cell of an open tile has at least three
     // inside coefficients and none larger, so where this diagonal is finite and not 0
     // every cell's is.
-    T.h3 = (T.h * T.h) * T.h;
     bool regular = true;
     if (my != GHOST) {
       const float ci = T.bc[6];
@@ -353,10 +352,6 @@ void build_tree(const cg_tree_desc* d, int prob, int base, int leaf_base, int gh
       T.rdiag = regular ? 1.0 / double(d) : 0.0;
       if (uniform) T.meta |= 1u << 28;
     }
-    // a power of two whose third power is a normal number
-    uint32_t hb;
-    std::memcpy(&hb, &T.h, 4);
-    if ((hb & 0x7fffffu) == 0 && T.h > 0x1p-40f && T.h < 0x1p40f) T.meta |= 1u << 29;
     // the cell types as 64 words of 8 cells (cell index i*64 + j*8 + k)
     constexpr uint64_t kOnes = 0x0101010101010101ull;
     auto words = [&](int t) {
