@@ -778,10 +778,12 @@ class Server:
 
     def next_result(self, wait=False, with_x=True):
         """(tag, instance, result dict, pressure or None) of the oldest finished
-        request, or None if none is ready."""
+        request, or None if none is ready.  The pressure is an array of its own,
+        of the instance's size."""
         # The pressure arrives in a buffer that fits any instance: a kept one, so
         # that a call neither clears nor faults in 30 MB of fresh pages (half of what
-        # a request cost the caller), handed over where the result fills half of it.
+        # a request cost the caller), handed over where the result fills half of it,
+        # its memory cut to the result's size.
         nmax = max([*self.ntiles.values(), 1])
         x = None
         if with_x:
@@ -801,7 +803,8 @@ class Server:
             if inst.value in self._undelivered:  # submitted with download=False: no pressure was written
                 xs = np.zeros((n, 512), np.float32)
             elif 2 * n >= len(x):
-                xs, x = x[:n], None
+                x.resize((n, 512), refcheck=False)  # the buffer is this call's alone
+                xs, x = x, None
             else:
                 xs = x[:n].copy()
         if x is not None and not self._spare:
