@@ -750,6 +750,16 @@ def read_trace_mean(path, kernel, tiles):
     return None
 
 
+REPLAY_BELOW_TILES = 8192  # cg_params.use_graph = -1: handles of fewer tiles replay a graph
+
+
+def launch_form(graph, tiles):
+    """How the plain solve's iterations are launched."""
+    if graph:
+        return "hipGraph replay"
+    return f"chosen per handle ({'graph replay' if tiles < REPLAY_BELOW_TILES else 'stream launches'} at this size)"
+
+
 def read_traffic(tiles):
     """Traffic per launch from the committed counter summary, if it covers this launch."""
     try:
@@ -919,7 +929,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": desc, "tiles": P.n, "leaf_tiles": P.n_leaf, "max_level": L,
                    "leaf_cells": P.n_leaf * 512, "iterations": iters,
-                   "launch": "hipGraph replay" if args.graph else "chosen per handle (graph replay at this size)"},
+                   "launch": launch_form(args.graph, P.n)},
         "p50_ms": float(np.percentile(lat_ms, 50)),
         "p99_ms": float(np.percentile(lat_ms, 99)),
         "build_s": t_build,
