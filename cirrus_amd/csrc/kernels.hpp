@@ -637,14 +637,11 @@ struct Stencil {
   float xkm, xkp;      // k-halo values (z- neighbour cell (i,j,7), z+ neighbour cell (i,j,0))
   float b_int, b_f[6]; // base coefficients: inside the tile and across face f
   float h;
-  double rd;           // the record's rdiag, and what it says of the tile
-  bool open, uniform;
+  bool open;           // tr_all_open
 };
 __device__ __forceinline__ void stencil_coeffs(const TileRec& T, const float bcv[7], Stencil& S) {
   S.h = T.h;
-  S.rd = T.rdiag;
   S.open = tr_all_open(T);
-  S.uniform = tr_uniform(T);
   S.b_int = bcv[6];
   for (int f = 0; f < 6; f++) S.b_f[f] = bcv[f];
 }

@@ -1337,6 +1337,8 @@ std::vector<double> residual64(cg_problem& P, const float* B, int pure_neumann, 
 // their runs of records are copied (each list is problem by problem) into a second
 // array, in stream order, and the launches after that cover those only.  Without
 // memory for it the full lists stay.  The handle's lists return with this object.
+// (A replayed iteration keeps the full lists: its graph holds their addresses and
+// lengths.)
 // Solves whose problems take 8 to 30 iterations: 256 problems in bfloat16 216 ->
 // 162 ms, 24 in FP32 19.1 -> 16.3, 7 in float16 (11 to 21 iterations) 6.42 -> 5.79.
 constexpr double kLiveShare = 0.9;
@@ -1452,7 +1454,8 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   v.pcoef = prm.prolong_coeff;
   const int stride = std::max(1, prm.sync_stride);
   auto t0 = std::chrono::steady_clock::now();
-  for (int q = 0; q < P.nprob; q++) P.h_prog[q] = 0;  // the stream is idle: every entry point waits for its work
+  // no kernel in flight writes these: only a solve's do, and it ends by waiting for them
+  for (int q = 0; q < P.nprob; q++) P.h_prog[q] = 0;
   set_prob_state(P, prm.rel_tol, prm.max_iters, prm.pure_neumann, prm.sync_stride, tol_q, maxit_q, thr_abs_q);
   int max_iters = prm.max_iters;
   if (maxit_q) for (int q = 0; q < P.nprob; q++) max_iters = std::max(max_iters, maxit_q[q]);
@@ -1477,12 +1480,15 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   v.amg = amg ? 1 : 0;
   std::snprintf(keybuf, sizeof(keybuf), "%d/%d/%d/%a/%a/%a/%d/%d/%d/%d", v.nu, v.coarsest, v.smoother, double(v.omega),
                 double(v.ooa), double(v.pcoef), prm.pure_neumann, prm.storage, P.swz, v.amg);
-  // -1: replay where the host could not keep up with the device (the AMG V-cycle;
+  // -1: replay where a host may not keep up with the device (the AMG V-cycle;
   // handles of fewer than kStreamMinTiles tiles), stream launches otherwise.  A
-  // launch costs the host 3.5 to 5 us, a replayed node less, and the device 2 us
-  // more an iteration.  5,505 tiles (41 launches of 3.7 us an iteration): 4.9 ms a
-  // solve by stream launches with a busy host, 2 % less than by replay with an idle
-  // one, 4.0 ms by replay; 14,345 tiles (5.3 us a launch): 3.47 ms and 3.53.
+  // launch costs a host 3.5 to 5 us, a replayed node less, and a replay the device
+  // about 5 us more an iteration.  Where the host keeps up, stream launches and
+  // replay take, ms a solve: 585 tiles 1.80, 1.86; 2,889 tiles 3.51, 3.69; 5,505
+  // tiles 3.73, 3.85; 8,753 tiles 4.24, 4.37; 14,945 tiles 6.25, 6.39.  On a slower
+  // host the 5,505 tiles (41 launches of 3.9 us an iteration) took 4.6 to 4.9 by
+  // stream launches and 4.0 replayed.  From 8,192 tiles the device needs 4.5 us a
+  // launch and more, so what replay could save there is no more than what it costs.
   constexpr int kStreamMinTiles = 8192;
   const bool small = !amg && runs_small(P);
   const int chunk = small ? kSmallIters : stride;  // (the kernel itself keeps to the stride of the checks)
