@@ -608,9 +608,13 @@ def _pmc_per_dispatch(path, counter):
     return {k: sum(v) / len(v) for k, v in acc.items()}
 
 
+REC_BYTES = 128  # a tile's record, fetched by scalar loads, which FETCH_SIZE counts in full
+
+
 def summarize_pmc(fetch_csv, write_csv, title=None, out=None):
     """Scale FETCH_SIZE / WRITE_SIZE (KiB per dispatch) of the colour sweeps by
-    the copy kernel's reading of its known traffic; write the profile summary.
+    the copy kernel's reading of its known traffic, the tile records (counted in
+    full) apart; write the profile summary.
     Default: the adaptive 256^3 workload's summary, whose traffic line feeds
     the roofline record."""
     fetch = _pmc_per_dispatch(fetch_csv, "FETCH_SIZE")
@@ -628,7 +632,7 @@ def summarize_pmc(fetch_csv, write_csv, title=None, out=None):
     (ck, cf), (_, cw) = pick(fetch, "k_copy_tiles"), pick(write, "k_copy_tiles")
     copy_tiles = ck[1] // 64
     copy_bytes = copy_tiles * 512 * 4
-    f_scale = copy_bytes / (cf * 1024.0)
+    f_scale = copy_bytes / (cf * 1024.0 - copy_tiles * REC_BYTES)
     w_scale = copy_bytes / (cw * 1024.0)
     default = title is None
     title = title or "the adaptive 256^3 workload"
@@ -642,7 +646,8 @@ def summarize_pmc(fetch_csv, write_csv, title=None, out=None):
         "  python bench.py --summarize-pmc OUT/fetch/pmc_counter_collection.csv OUT/write/pmc_counter_collection.csv"
         + ("" if default else " --pmc-title '...' --pmc-out FILE"),
         "",
-        f"copy reference k_copy_tiles: {copy_tiles} tiles, {copy_bytes} B read and {copy_bytes} B written per dispatch",
+        f"copy reference k_copy_tiles: {copy_tiles} tiles, {copy_bytes} B read and {copy_bytes} B written per dispatch,"
+        f" and {REC_BYTES} B a tile of records read (counted in full)",
         f"  FETCH_SIZE {cf:.1f} KiB/dispatch -> read scale {f_scale:.4f}",
         f"  WRITE_SIZE {cw:.1f} KiB/dispatch -> write scale {w_scale:.4f}",
     ]
@@ -657,7 +662,8 @@ def summarize_pmc(fetch_csv, write_csv, title=None, out=None):
         # the counter run launches each sweep over the same list; its tile count
         # comes from the one-tile-per-wavefront grid
         tiles = pick(fetch, "k_gs_color<float>")[0][1] // 64
-        rd, wr = fv * 1024.0 * f_scale, wv * 1024.0 * w_scale
+        rec = tiles * REC_BYTES
+        rd, wr = (fv * 1024.0 - rec) * f_scale + rec, wv * 1024.0 * w_scale
         alg = gs_alg_bytes(tiles, s_bytes)
         lines += [f"{name}: {tiles} tiles, {per_wave} per wavefront (grid {k[1]} threads)",
                   f"  FETCH_SIZE {fv:.1f} KiB/dispatch -> {rd:.0f} B read",
