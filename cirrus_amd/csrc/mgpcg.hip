@@ -1486,7 +1486,7 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   // about 5 us more an iteration.  Where the host keeps up, stream launches and
   // replay take, ms a solve: 585 tiles 1.80, 1.86; 2,889 tiles 3.51, 3.69; 5,505
   // tiles 3.73, 3.85; 8,753 tiles 4.24, 4.37; 14,945 tiles 6.25, 6.39.  On a slower
-  // host the 5,505 tiles (41 launches of 3.9 us an iteration) took 4.6 to 4.9 by
+  // host the 5,505 tiles (40 launches of 4.1 us an iteration) took 4.6 to 4.9 by
   // stream launches and 4.0 replayed.  From 8,192 tiles the device needs 4.5 us a
   // launch and more, so what replay could save there is no more than what it costs.
   constexpr int kStreamMinTiles = 8192;
