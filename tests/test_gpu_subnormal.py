@@ -95,3 +95,28 @@ def test_solves_of_subnormal_right_hand_sides(scene, h0, solver):
         r = S.last
     assert np.array_equal([r["iters"], r["rr"], r["bb"]], [ro["iters"], ro["rr"], ro["bb"]], equal_nan=True)
     assert np.array_equal(P.get(ca.CH_X)[leaf], o.get(po.CH_X).astype(np.float32)[leaf], equal_nan=True)
+
+
+@pytest.mark.parametrize("coarsening", [2.0 ** -115, 2.0 ** -60, 2.0 ** 60, 2.0 ** 110])
+def test_reciprocals_of_extreme_diagonals(coarsening):
+    """Stored coefficients scaled per level far from 1, so that a diagonal lies beyond
+    the range of the fast reciprocal: the LDS-resident levels against the same levels by
+    grid-wide launches, which divide."""
+    o, P, typ, ctype = pair("children", 0.125)
+    leaf = typ == po.LEAF
+    f = np.random.default_rng(6).standard_normal(ctype.shape).astype(np.float32)
+    f[(ctype != ca.INTERIOR) | ~leaf[:, None]] = 0
+    S = ca.AMGSolver(one_over_alpha=coarsening)
+    S.prepareTypesAndCoeffs(P)
+    d = S.coefficients(P)[3][typ == po.NONLEAF]
+    assert (d != 0).any() and np.all((np.abs(d) < 2.0 ** -100) | (np.abs(d) > 2.0 ** 100)) == (coarsening not in (2.0 ** -60, 2.0 ** 60))
+    out = []
+    for shift in (0, 2):
+        P.set_schedule(coarse_shift=shift)
+        P.set(ca.CH_B, f)
+        S.solve(P, False, 3, 1e-6, 1, 4, 1, False)
+        r = S.last_batch[0]
+        out.append(([r["iters"], r["rr"]], P.get(ca.CH_P)[leaf], P.get(ca.CH_X)[leaf]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
+    assert np.isfinite(out[0][1]).all() and out[0][1].any()
