@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <limits>
 #include <memory>
@@ -1235,6 +1236,15 @@ std::vector<ProbState> finish_states(cg_problem& P) {
   return std::vector<ProbState>(P.h_ps, P.h_ps + P.nprob);
 }
 
+// Waits for a stream's work where an error ends the scope.
+struct WaitOnError {
+  hipStream_t stream;
+  int before = std::uncaught_exceptions();
+  ~WaitOnError() {
+    if (std::uncaught_exceptions() > before) (void)hipStreamSynchronize(stream);
+  }
+};
+
 // Waits until every problem is done or past iteration `iters`; true when all are
 // done.  The kernels write their progress to host memory (Ctx::progress), so an
 // iteration needs no copy and no event for it: those cost 8 to 12 us between two
@@ -1454,7 +1464,9 @@ void solve(cg_problem& P, const cg_params& prm, cg_result* res, const double* to
   v.pcoef = prm.prolong_coeff;
   const int stride = std::max(1, prm.sync_stride);
   auto t0 = std::chrono::steady_clock::now();
-  // no kernel in flight writes these: only a solve's do, and it ends by waiting for them
+  // no kernel in flight writes these: only a solve's do, and it ends by waiting for
+  // them, by an error too
+  const WaitOnError wait{P.stream};
   for (int q = 0; q < P.nprob; q++) P.h_prog[q] = 0;
   set_prob_state(P, prm.rel_tol, prm.max_iters, prm.pure_neumann, prm.sync_stride, tol_q, maxit_q, thr_abs_q);
   int max_iters = prm.max_iters;
